@@ -15,7 +15,10 @@ extern "C" {
 
 /* field kernels */
 enum scarf_kernel {
-    SCARF_KERNEL_AUTO = 0,        /* mfma_bf16x3 on grids, direct_f32 on point lists (float lib); direct_f64 (double lib) */
+    SCARF_KERNEL_AUTO = 0,        /* grids: a fast nonuniform transform of the library's precision where that is faster
+                                     than the direct sum (from a few hundred harmonics on), else mfma_bf16x3 or
+                                     direct_f32 (float lib), direct_f64 (double lib); point lists: direct_f32,
+                                     direct_f64 */
     SCARF_KERNEL_DIRECT_F32 = 1,  /* FP32 cos on FP64-reduced phases, FP64-promoted sums */
     SCARF_KERNEL_DIRECT_F64 = 2,  /* FP64 throughout */
     SCARF_KERNEL_MFMA_BF16X3 = 3, /* grid GEMM, 3-term bf16 split, 6 MFMA products */
@@ -29,7 +32,9 @@ int scarf_set_nharm(int nharm);
 int scarf_get_nharm(void);
 
 /* Field kernel for subsequent executes (environment SCARF_KERNEL=name also
- * works: auto, direct_f32, direct_f64, mfma_bf16x3, mfma_f16x2, mfma_bf16x2). */
+ * works: auto, direct_f32, direct_f64, mfma_bf16x3, mfma_f16x2, mfma_bf16x2).
+ * scarf_get_kernel names the direct-sum kernel of the current configuration
+ * under auto, also where the transform runs. */
 int scarf_set_kernel(int kernel);
 int scarf_get_kernel(void);
 
@@ -56,7 +61,8 @@ int scarf_srm_run(real *d_field, real stats[]);
  * live in a static device array of 64 MiB that each GPU holds for the life
  * of the process; the tables are built one chunk of harmonics at a time
  * (chunks are multiples of 128 harmonics and carry the field's running
- * sums, so the field equals scarf_srm_run's bit for bit). Takes the resident table of
+ * sums, so the field equals scarf_srm_run's with the same MFMA kernel set bit
+ * for bit; under auto it is that of the kernel scarf_get_kernel names). Takes the resident table of
  * scarf_srm_draw, and the MFMA kernels of structured grids only; uses the
  * tile chosen earlier for the grid (or the least-padding one) and tunes
  * nothing. Refuses, with an error, grids whose operand tables for 128

@@ -33,6 +33,7 @@
 #include "srm_device.hpp"
 #include "srm_host.hpp"
 #include "srm_mfma.hpp"
+#include "srm_transform.hpp"
 #include "worker_pool.hpp"
 
 #include <climits>
@@ -208,6 +209,19 @@ scarf::Geometry geometry(const SrmConfig &cfg)
     return g;
 }
 
+// The kernel that computes the field: with auto on a grid, the fast transform
+// where it is the faster one (the decision takes the configured harmonic
+// count, so that every entry point makes the same one).
+int field_kernel(const SrmConfig &cfg)
+{
+    const int k = resolve_kernel(cfg);
+    if (current_kernel() != scarf::kKernelAuto || !cfg.structured) return k;
+    const scarf::Geometry g = geometry(cfg);
+    scarf::TransformPlan plan;
+    if (!scarf::transform_plan(g, (cfg.nharm + 63) / 64 * 64, kDouble, plan)) return k;
+    return scarf::transform_ms(plan, kDouble) < scarf::direct_ms(g, cfg.nharm, k) ? scarf::kKernelTransform : k;
+}
+
 scarf::Epilogue epilogue(const SrmConfig &cfg, int ndim)
 {
     scarf::Epilogue ep;
@@ -293,10 +307,11 @@ int run(real *d_field, real stats[], const scarf::Device::SlabHook *on_slab = nu
     if (!s.table_ready) return fail("no harmonic table drawn (call scarf_srm_draw first)");
     const scarf::Geometry g = geometry(s.cfg);
     const scarf::Epilogue ep = epilogue(s.cfg, s.setup.ndim);
-    const int kernel = resolve_kernel(s.cfg);
+    const int kernel = field_kernel(s.cfg);
     double st[6] = {};
     std::string err;
-    if (!s.device->run<real>(g, kernel, s.setup.scaling, ep, d_field, st, err, on_slab)) return fail(err);
+    if (!s.device->run<real>(g, kernel, s.setup.scaling, ep, d_field, st, err, on_slab, resolve_kernel(s.cfg)))
+        return fail(err);
     report_stats(stats, st);
     s.error.clear();
     return 0;
@@ -364,7 +379,7 @@ int execute_realization(int seed, real *d_field, real stats[], const scarf::Devi
     if (!s.initialized) return fail("execute called before initialize");
     if (s.cfg.method == 0) return execute_fim(seed, d_field, stats, on_slab);
     s.cfg.nharm = s.nharm;
-    const int kernel = resolve_kernel(s.cfg);
+    const int kernel = field_kernel(s.cfg);
     const bool mfma = kernel == scarf::kKernelMfmaBf16x3 || kernel == scarf::kKernelMfmaF16x2 ||
                       kernel == scarf::kKernelMfmaBf16x2;
     if (!s.cfg.structured || !mfma || !s.stream_draw) {

@@ -21,6 +21,7 @@ enum Kernel : int {
     kKernelMfmaBf16x3 = 3,  // per-slab GEMM, 3-term bf16 split, 6 MFMA products
     kKernelMfmaF16x2 = 4,   // per-slab GEMM, scaled 2-term fp16 split, 3 products
     kKernelMfmaBf16x2 = 5,  // per-slab GEMM, 2-term bf16 split, 3 products (below 1e-5 sigma)
+    kKernelTransform = 6,   // plane-wise fast transform (srm_transform.hpp); chosen by auto, not part of the API
 };
 const char *kernel_name(int k);
 
@@ -74,10 +75,13 @@ public:
     // of the field as soon as it is final: in z order while the rest is still
     // computed (MFMA grids with no rescale or taper), else once for the whole
     // field at the end.
+    // `otherwise`: the kernel that runs instead of kKernelTransform when the
+    // device has no room for the transform's workspace.
     using SlabHook = std::function<bool(long, long, std::string &)>;
     template <class Real>
     bool run(const Geometry &g, int kernel, double scaling, const Epilogue &ep, Real *d_field,
-             double *stats_out, std::string &err, const SlabHook *on_slab = nullptr);
+             double *stats_out, std::string &err, const SlabHook *on_slab = nullptr,
+             int otherwise = kKernelDirectF32);
 
     // Source of a realization's harmonics in draw order: feed(kept, t, last)
     // appends to t the kept harmonics that bring their total to `kept`

@@ -23,6 +23,7 @@
 #include "srm_device.hpp"
 #include "srm_mfma.hpp"
 #include "srm_stats.hpp"
+#include "srm_transform.hpp"
 
 namespace scarf {
 
@@ -419,6 +420,7 @@ const char *kernel_name(int k)
     case kKernelMfmaBf16x3: return "mfma_bf16x3";
     case kKernelMfmaF16x2: return "mfma_f16x2";
     case kKernelMfmaBf16x2: return "mfma_bf16x2";
+    case kKernelTransform: return "transform";
     default: return "unknown";
     }
 }
@@ -564,7 +566,7 @@ bool Device::upload_points(const Real *x, const Real *y, const Real *z, long n, 
 
 template <class Real>
 bool Device::run(const Geometry &g, int kernel, double scaling, const Epilogue &ep, Real *d_field,
-                 double *stats_out, std::string &err, const SlabHook *on_slab)
+                 double *stats_out, std::string &err, const SlabHook *on_slab, int otherwise)
 {
     HIP_TRY(hipSetDevice(device_));
     if (!d_harm_ || nharm_ <= 0) {
@@ -577,6 +579,16 @@ bool Device::run(const Geometry &g, int kernel, double scaling, const Epilogue &
         err = "empty field";
         return false;
     }
+    TransformPlan transform;
+    if (kernel == kKernelTransform) {
+        if (!transform_plan(g, np_, sizeof(Real) == sizeof(double), transform) ||
+            !reserve(d_tab_, tab_cap_, transform.bytes, err) ||
+            !reserve(d_part_, part_cap_, size_t(3) * (transform.nparts + transform.groups) * sizeof(double), err)) {
+            (void)hipGetLastError();  // a refused allocation
+            err.clear();
+            kernel = otherwise;
+        }
+    }
     const bool mfma = g.structured && (kernel == kKernelMfmaBf16x3 || kernel == kKernelMfmaF16x2 ||
                                        kernel == kKernelMfmaBf16x2);
     TileChoice tile;
@@ -587,6 +599,7 @@ bool Device::run(const Geometry &g, int kernel, double scaling, const Epilogue &
     HIP_TRY(hipEventRecord(ev_[0], stream_));
 
     int nparts = 0;
+    double *part = nullptr;  // the statistics partials, where they are not d_part_
     // field parts (first point, points, event) handed to on_slab while the
     // rest is computed: z slabs of whole k-tile rows, MFMA grids only, and
     // only when no rescale or taper changes the field afterwards
@@ -623,6 +636,11 @@ bool Device::run(const Geometry &g, int kernel, double scaling, const Epilogue &
             } else if (!mfma_field(plan, g, d_tab_, scaling, d_field, d_part_, stream_, err)) {
                 return false;
             }
+        } else if (kernel == kKernelTransform) {
+            if (!transform_field<Real>(transform, g, d_harm_, d_tab_, scaling, d_field, d_part_, stream_, ev_[1], err))
+                return false;
+            nparts = transform.groups;
+            part = d_part_ + 3 * size_t(transform.nparts);
         } else {
             const bool f64 = kernel == kKernelDirectF64;
             const size_t elt = f64 ? sizeof(double) : sizeof(float);
@@ -678,7 +696,7 @@ bool Device::run(const Geometry &g, int kernel, double scaling, const Epilogue &
                                                                     d_harm_, np_, scaling, d_field, d_part_);
         HIP_TRY(hipGetLastError());
     }
-    return finish<Real>(g, ep, d_field, nparts, stats_out, slab_first, slab_points, err, on_slab);
+    return finish<Real>(g, ep, d_field, nparts, stats_out, slab_first, slab_points, err, on_slab, part);
 }
 
 template <class Real>
@@ -955,9 +973,9 @@ bool Device::run_streamed(const Geometry &g, int kernel, int nharm, double scali
 template bool Device::upload_points<float>(const float *, const float *, const float *, long, std::string &);
 template bool Device::upload_points<double>(const double *, const double *, const double *, long, std::string &);
 template bool Device::run<float>(const Geometry &, int, double, const Epilogue &, float *, double *, std::string &,
-                                 const SlabHook *);
+                                 const SlabHook *, int);
 template bool Device::run<double>(const Geometry &, int, double, const Epilogue &, double *, double *,
-                                  std::string &, const SlabHook *);
+                                  std::string &, const SlabHook *, int);
 template bool Device::run_noalloc<float>(const Geometry &, int, double, const Epilogue &, float *, double *,
                                          std::string &);
 template bool Device::run_noalloc<double>(const Geometry &, int, double, const Epilogue &, double *, double *,
