@@ -31,6 +31,7 @@
 #include "../../include/scarf3d_srm.h"
 #include "fim.hpp"
 #include "srm_device.hpp"
+#include "srm_draw.hpp"
 #include "srm_host.hpp"
 #include "srm_mfma.hpp"
 #include "srm_transform.hpp"
@@ -57,6 +58,7 @@ struct State {
     std::string error;
     std::unique_ptr<scarf::Device> device;
     std::unique_ptr<scarf::FimDevice> fim;
+    std::unique_ptr<scarf::TrialDevice> trials;
     std::unique_ptr<scarf::Ensemble> ensemble;
     // resident realization (scarf_srm_draw -> scarf_srm_run)
     bool table_ready = false;
@@ -248,8 +250,21 @@ bool ensure_device()
         fail(err);
         return false;
     }
-    s.device->set_external_reserved(s.fim ? s.fim->reserved_bytes() : 0);
+    if (!s.trials) s.trials = std::make_unique<scarf::TrialDevice>();
+    const size_t fim = s.fim ? s.fim->reserved_bytes() : 0;
+    s.trials->set_elsewhere(s.device->reserved_bytes() + fim);
+    s.device->set_external_reserved(s.trials->reserved_bytes() + fim);
     return true;
+}
+
+// The draw of one seed as device records, its trials screened on the GPU.
+std::unique_ptr<scarf::HarmonicSampler> sampler(const SrmConfig &cfg, const scarf::SrmSetup &setup, int seed)
+{
+    State &s = state();
+    return kDouble ? scarf::HarmonicSampler::create_rows<double>(cfg, setup, seed, s.trials.get(), s.draw_threads,
+                                                                 s.draw_block)
+                   : scarf::HarmonicSampler::create_rows<float>(cfg, setup, seed, s.trials.get(), s.draw_threads,
+                                                                s.draw_block);
 }
 
 void clear_stats(real stats[])
@@ -271,17 +286,16 @@ int prepare(int seed)
     const int rc = kDouble ? scarf::srm_setup<double>(s.cfg, s.setup, err) : scarf::srm_setup<float>(s.cfg, s.setup, err);
     if (rc != 0) return fail(err);
     if (!ensure_device()) return -1;
-    const scarf::HarmonicDraw d = kDouble ? scarf::srm_draw<double>(s.cfg, s.setup, seed, s.draw_threads, s.draw_block)
-                                          : scarf::srm_draw<float>(s.cfg, s.setup, seed, s.draw_threads, s.draw_block);
-    const scarf::HarmonicTable t = scarf::build_table(s.setup, d);
+    const std::unique_ptr<scarf::HarmonicSampler> draw = sampler(s.cfg, s.setup, seed);
+    const int kept = draw->draw_until(INT_MAX);
     s.host_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-    if (!s.device->upload_table(t, err)) return fail(err);
+    if (!s.device->upload_table(draw->rows(0, kept), err)) return fail(err);
     if (!s.cfg.structured) {
         if (!s.device->upload_points<real>(s.x, s.y, s.z, s.cfg.npts, err)) return fail(err);
     }
     s.table_ready = true;
     s.error.clear();
-    return d.n_used;
+    return kept;
 }
 
 // stats(1:8) of a finished realization (src/scarflib.f90:363,377)
@@ -393,15 +407,14 @@ int execute_realization(int seed, real *d_field, real stats[], const scarf::Devi
     if (rc != 0) return fail(err);
     double host = std::chrono::duration<double>(clock::now() - t0).count();
     if (!ensure_device()) return -1;
-    std::unique_ptr<scarf::HarmonicSampler> sampler =
-        kDouble ? scarf::HarmonicSampler::create<double>(s.cfg, s.setup, seed, s.draw_threads, s.draw_block)
-                : scarf::HarmonicSampler::create<float>(s.cfg, s.setup, seed, s.draw_threads, s.draw_block);
-    const scarf::Device::HarmonicFeed feed = [&](int kept, scarf::HarmonicTable &t, bool &last, std::string &) {
+    const std::unique_ptr<scarf::HarmonicSampler> draw = sampler(s.cfg, s.setup, seed);
+    int drawn = 0;  // kept harmonics handed over
+    const scarf::Device::HarmonicFeed feed = [&](int kept, scarf::HarmonicRows &t, bool &last, std::string &) {
         const auto a = clock::now();
-        const int l0 = sampler->position();
-        sampler->draw_until(kept);
-        scarf::append_table(s.setup, sampler->draw(), l0, sampler->position(), t);
-        last = sampler->finished();
+        const int now = draw->draw_until(kept);
+        t = draw->rows(drawn, now);
+        drawn = now;
+        last = draw->finished();
         host += std::chrono::duration<double>(clock::now() - a).count();
         return true;
     };
@@ -415,10 +428,9 @@ int execute_realization(int seed, real *d_field, real stats[], const scarf::Devi
         // an amplitude the scaled-fp16 table cannot hold unscaled: the rest of
         // the draw, then the whole table with its power-of-two scale
         const auto a = clock::now();
-        sampler->draw_until(INT_MAX);
-        const scarf::HarmonicTable t = scarf::build_table(s.setup, sampler->draw());
+        const int kept = draw->draw_until(INT_MAX);
         s.host_seconds = host + std::chrono::duration<double>(clock::now() - a).count();
-        if (!s.device->upload_table(t, err)) return fail(err);
+        if (!s.device->upload_table(draw->rows(0, kept), err)) return fail(err);
         s.table_ready = true;
         return run(d_field, stats, on_slab);
     }

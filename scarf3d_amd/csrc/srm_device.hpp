@@ -64,7 +64,7 @@ public:
 
     // Uploads the harmonic table (FP64 SoA) and, for point lists, the
     // coordinates (widened to FP64).
-    bool upload_table(const HarmonicTable &t, std::string &err);
+    bool upload_table(const HarmonicRows &t, std::string &err);
     template <class Real>
     bool upload_points(const Real *x, const Real *y, const Real *z, long n, std::string &err);
 
@@ -84,10 +84,10 @@ public:
              int otherwise = kKernelDirectF32);
 
     // Source of a realization's harmonics in draw order: feed(kept, t, last)
-    // appends to t the kept harmonics that bring their total to `kept`
+    // gives in t the kept harmonics that bring their total to `kept`
     // (fewer only when the draw has ended; last = true once every harmonic
     // has been drawn).
-    using HarmonicFeed = std::function<bool(int kept, HarmonicTable &t, bool &last, std::string &err)>;
+    using HarmonicFeed = std::function<bool(int kept, HarmonicRows &t, bool &last, std::string &err)>;
     // The same realization as run() on an MFMA kernel of a structured grid,
     // with the harmonics taken from `feed` in chunks while the device works:
     // each chunk's record upload, operand tables and field pass are queued as
@@ -187,7 +187,8 @@ private:
     // harmonic record: wx, wy, wz (rad/m), phase (rad), amp; plus revolution copies
     double *d_harm_ = nullptr;
     size_t harm_cap_ = 0;
-    double *h_rec_ = nullptr;  // pinned staging of a streamed record
+    bool stage_record(size_t bytes, std::string &err);
+    double *h_rec_ = nullptr;  // pinned staging of the record
     size_t h_rec_cap_ = 0;
     // per-axis tables (FP32 or FP64 revolutions, operand tables of the GEMM)
     void *d_tab_ = nullptr;

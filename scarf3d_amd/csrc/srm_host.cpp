@@ -134,7 +134,7 @@ int srm_setup(const SrmConfig &cfg, SrmSetup &out, std::string &err)
     // usable acceptance somewhere in [kmin, kmax]; upstream it spins forever
     // otherwise (e.g. a Gaussian spectrum on a box much smaller than cl).
     double peak = 0.0;
-    for (int q = 0; q <= 4096; ++q) {
+    for (int q = 0; q <= 4096 && !(peak > 1.0e-7); ++q) {
         const Real u = kmin + (kmax - kmin) * static_cast<Real>(q) / Real(4096);
         peak = std::max(peak, spec(static_cast<double>(u)) * static_cast<double>(cnst));
     }
@@ -189,7 +189,7 @@ struct DrawContext {
     static Real uniform(int64_t raw) { return static_cast<Real>(Yarn2::to_uniform01(raw)); }
 
     // Squeeze: bound[b] is at least the acceptance of every r0 in
-    // [b/kBins, (b+1)/kBins], so a trial with r1 >= bound[b] is rejected
+    // [b/bins, (b+1)/bins], so a trial with r1 >= bound[b] is rejected
     // without evaluating the spectrum; the others take the exact test. The
     // decisions are the exact test's. srm_fn * const = u^d psd(u) has one
     // maximum, at u^2 = d / (2 nu - d) (von Karman) or 2d (Gaussian), with
@@ -198,7 +198,7 @@ struct DrawContext {
     // acceptance (a few roundings of `real` and one libm pow or exp, well
     // under 1e-5 relative) stays below that end's value times 1 + 1e-4.
     // Bins near the maximum have no bound.
-    static constexpr int kBins = 4096;
+    int bins = 4096;
     std::vector<Real> bound;
     void make_bounds(int ndim)
     {
@@ -206,10 +206,10 @@ struct DrawContext {
         const double nu = static_cast<double>(spec.nu);
         const double up2 = spec.acf == 0 ? (2.0 * nu > d ? d / (2.0 * nu - d) : -1.0) : 2.0 * d;
         const double up = up2 > 0.0 ? std::sqrt(up2) : 0.0;
-        bound.assign(kBins, std::numeric_limits<Real>::infinity());
-        for (int b = 0; b < kBins; ++b) {
-            const Real ulo = radial(static_cast<Real>(b) / static_cast<Real>(kBins));
-            const Real uhi = radial(static_cast<Real>(b + 1) / static_cast<Real>(kBins));
+        bound.assign(bins, std::numeric_limits<Real>::infinity());
+        for (int b = 0; b < bins; ++b) {
+            const Real ulo = radial(static_cast<Real>(b) / static_cast<Real>(bins));
+            const Real uhi = radial(static_cast<Real>(b + 1) / static_cast<Real>(bins));
             Real end;
             if (static_cast<double>(ulo) >= up * (1.0 + 1e-3)) end = acceptance(ulo);       // decreasing
             else if (static_cast<double>(uhi) <= up * (1.0 - 1e-3)) end = acceptance(uhi);  // increasing
@@ -220,7 +220,7 @@ struct DrawContext {
     }
     bool accepts_fast(Real r0, Real r1) const
     {
-        const int b = std::min(static_cast<int>(r0 * static_cast<Real>(kBins)), kBins - 1);
+        const int b = std::min(static_cast<int>(r0 * static_cast<Real>(bins)), bins - 1);
         if (!(r1 < bound[b])) return false;
         return accepts(r0, r1);
     }
@@ -269,6 +269,19 @@ SharedPool &shared_pool()
     return *p;
 }
 
+// {wx, wy, wz, phase, amp} of a harmonic (srm_host.hpp, HarmonicTable):
+// w = M^T v, as theta = sum_r v_r ((M p)_r + bar_r) = (M^T v) . p + v . bar
+void record(const SrmSetup &s, double v1, double v2, double v3, double a, double b, double (&row)[5])
+{
+    const double *m = s.matrix;
+    row[0] = v1 * m[0] + v2 * m[1] + v3 * m[2];
+    row[1] = v1 * m[3] + v2 * m[4] + v3 * m[5];
+    row[2] = v1 * m[6] + v2 * m[7] + v3 * m[8];
+    const double vbar = v1 * s.bar[0] + v2 * s.bar[1] + v3 * s.bar[2];
+    row[3] = vbar - std::atan2(a, b);
+    row[4] = std::hypot(a, b);
+}
+
 // Harmonic draw (src/scarflib_srm.f90:731-778): rejection sampling of the
 // radial wavenumber against srm_fn*const, a uniform direction, and a, b from
 // the cosine branch of Box-Muller with one srng call each.
@@ -280,18 +293,28 @@ SharedPool &shared_pool()
 // workers that each jump to their sub-range (Yarn2::discard); the walk then
 // only looks up the next accepted pair. The pairs consumed, and so every
 // harmonic, are those of the one-pair-at-a-time loop.
+//
+// With a TrialScreen the stream is generated and screened elsewhere and only
+// the pairs that may pass arrive (TrialBlock); the workers give them the exact
+// test, the walk picks the trials, and the workers compute the harmonics. A
+// screen that fails leaves the rest of the draw to the blocks above.
 template <class Real>
 class Sampler final : public HarmonicSampler {
 public:
-    Sampler(const SrmConfig &cfg, const SrmSetup &s, int seed, int threads, long block_pairs)
-        : n_(cfg.nharm), ndim_(s.ndim)
+    Sampler(const SrmConfig &cfg, const SrmSetup &s, int seed, int threads, long block_pairs, bool rows = false,
+            TrialScreen *screen = nullptr)
+        : n_(cfg.nharm), ndim_(s.ndim), seed_(seed), rows_only_(rows), setup_(s), screen_(screen)
     {
-        d_.v1.assign(n_, 0.0);
-        d_.v2.assign(n_, 0.0);
-        d_.v3.assign(n_, 0.0);
-        d_.a.assign(n_, 0.0);
-        d_.b.assign(n_, 0.0);
-        d_.used.assign(n_, 0);
+        if (rows) {
+            rows_.reset(new double[size_t(5) * n_]);
+        } else {
+            d_.v1.assign(n_, 0.0);
+            d_.v2.assign(n_, 0.0);
+            d_.v3.assign(n_, 0.0);
+            d_.a.assign(n_, 0.0);
+            d_.b.assign(n_, 0.0);
+            d_.used.assign(n_, 0);
+        }
         ctx_.spec.acf = cfg.acf;
         ctx_.spec.ndim = s.ndim;
         ctx_.spec.nu = static_cast<Real>(s.nu);
@@ -300,11 +323,28 @@ public:
         ctx_.kc = static_cast<Real>(s.kc);
         ctx_.cnst = static_cast<Real>(s.cnst);
         ctx_.seed = static_cast<unsigned long>(seed);  // set_seed: unsigned long myseed = seed
+        // expected trials per harmonic: 1 / (mean acceptance over the band)
+        const double p = s.kmax > s.kmin ? s.cnst * s.band / (s.kmax - s.kmin) : 1.0;
+        trials_ = 1.0 / std::min(1.0, std::max(p, 1e-9));
+        const double pairs = n_ * (trials_ + 3.0);
+        if (screen_ && pairs < kScreenPairs) screen_ = nullptr;
+        // a finer table rejects a little more and costs one spectrum value per bin
+        while (screen_ && ctx_.bins > 64 && 64.0 * ctx_.bins > pairs) ctx_.bins /= 2;
+        if (screen_) ctx_.bins = std::min(ctx_.bins, 1024);
         ctx_.make_bounds(s.ndim);
+        if (screen_) {
+            limit_.resize(ctx_.bins);
+            for (int b = 0; b < ctx_.bins; ++b) {
+                // above every output whose uniform, rounded to Real, is below the bound
+                const double v = static_cast<double>(ctx_.bound[b]) * (1.0 + 1e-6) * Yarn2::kModulus + 2.0;
+                limit_[b] = v < 2147483648.0 ? static_cast<uint32_t>(v) : 2147483648u;
+            }
+        }
         cl_[0] = static_cast<Real>(cfg.cl[0]);
         cl_[1] = static_cast<Real>(cfg.cl[1]);
         cl_[2] = static_cast<Real>(cfg.cl[2]);
         if (threads <= 0) threads = default_draw_threads();
+        capped_ = block_pairs > 0;
         max_block_ = block_pairs > 0 ? block_pairs : (1L << 18);
         next_size_ = std::min(max_block_, std::max(64L, 16L * n_));  // first block: a few trials per harmonic
         if (threads > 1) {
@@ -323,12 +363,21 @@ public:
     bool finished() const override { return l_ >= n_; }
     const HarmonicDraw &draw() const override { return d_; }
     int position() const override { return l_; }
+    HarmonicRows rows(int k0, int k1) const override
+    {
+        HarmonicRows r;
+        r.n = k1 - k0;
+        for (int f = 0; f < 5; ++f) r.field[f] = rows_.get() + size_t(f) * n_ + k0;
+        return r;
+    }
 
     int draw_until(int kept) override
     {
-        const Real pi = kPi<Real>;
-        Real r[2];
         while (l_ < n_ && d_.n_used < kept) {
+            if (screen_) {
+                draw_screened(kept);
+                continue;  // done, or the screen failed
+            }
             const int l = l_++;
             long q = -1;
             while (q < 0) {
@@ -342,39 +391,12 @@ public:
                 if (q < 0) pos_ = blk_.end;
             }
             if (q + 3 >= blk_.end) fill(q);  // the trial and the (up to) three pairs after it
-            pair(q, r);
-            const Real u = ctx_.radial(r[0]);
-            pair(q + 1, r);
-            if (u > ctx_.kc) {  // dropped, still counted by the scaling
-                pos_ = q + 2;
-                d_.uniforms = 2 * pos_;
-                continue;
+            const int64_t *raw = blk_.raw.data() + 2 * static_cast<size_t>(q - blk_.start);
+            if (take_trial(q, raw[0])) {
+                uint32_t v[8];
+                for (int k = 0; k < 8; ++k) v[k] = static_cast<uint32_t>(raw[k]);
+                harmonic(l, d_.n_used - 1, v);
             }
-            const Real phi = r[0] * Real(2) * pi;
-            Real v1, v2, v3;
-            if (ndim_ == 3) {
-                const Real theta = std::acos(Real(1) - Real(2) * r[1]);
-                v1 = u * std::sin(phi) * std::sin(theta) / cl_[0];
-                v2 = u * std::cos(phi) * std::sin(theta) / cl_[1];
-                v3 = u * std::cos(theta) / cl_[2];
-            } else {
-                v1 = u * std::cos(phi) / cl_[0];
-                v2 = u * std::sin(phi) / cl_[1];
-                v3 = 0;
-            }
-            pair(q + 2, r);
-            const Real a = std::sqrt(-(Real(2) * std::log(r[0]))) * std::cos(Real(2) * pi * r[1]);
-            pair(q + 3, r);
-            const Real b = std::sqrt(-(Real(2) * std::log(r[0]))) * std::cos(Real(2) * pi * r[1]);
-            pos_ = q + 4;
-            d_.v1[l] = v1;
-            d_.v2[l] = v2;
-            d_.v3[l] = v3;
-            d_.a[l] = a;
-            d_.b[l] = b;
-            d_.used[l] = 1;
-            ++d_.n_used;
-            d_.uniforms = 2 * pos_;
         }
         return d_.n_used;
     }
@@ -382,6 +404,123 @@ public:
     HarmonicDraw take() { return std::move(d_); }
 
 private:
+    // fewer pairs cost less here (17 ns each) than the round trip to the GPU (about 50 us)
+    static constexpr double kScreenPairs = 2000.0;
+
+    // the accepted pair q: false when its harmonic is dropped (above kc, still
+    // counted by the scaling)
+    bool take_trial(long q, int64_t first)
+    {
+        const bool keep = !(ctx_.radial(DrawContext<Real>::uniform(first)) > ctx_.kc);
+        pos_ = q + (keep ? 4 : 2);
+        d_.n_used += keep;
+        d_.uniforms = 2 * pos_;
+        return keep;
+    }
+
+    // harmonic l, the kept-th kept one, from the outputs of its trial and the
+    // three pairs after it
+    void harmonic(int l, int kept, const uint32_t *raw)
+    {
+        const Real pi = kPi<Real>;
+        Real r[8];
+        for (int k = 0; k < 8; ++k) r[k] = DrawContext<Real>::uniform(raw[k]);
+        const Real u = ctx_.radial(r[0]);
+        const Real phi = r[2] * Real(2) * pi;
+        Real v1, v2, v3;
+        if (ndim_ == 3) {
+            const Real theta = std::acos(Real(1) - Real(2) * r[3]);
+            v1 = u * std::sin(phi) * std::sin(theta) / cl_[0];
+            v2 = u * std::cos(phi) * std::sin(theta) / cl_[1];
+            v3 = u * std::cos(theta) / cl_[2];
+        } else {
+            v1 = u * std::cos(phi) / cl_[0];
+            v2 = u * std::sin(phi) / cl_[1];
+            v3 = 0;
+        }
+        const Real a = std::sqrt(-(Real(2) * std::log(r[4]))) * std::cos(Real(2) * pi * r[5]);
+        const Real b = std::sqrt(-(Real(2) * std::log(r[6]))) * std::cos(Real(2) * pi * r[7]);
+        if (rows_only_) {
+            double row[5];
+            record(setup_, v1, v2, v3, a, b, row);
+            for (int f = 0; f < 5; ++f) rows_[size_t(f) * n_ + kept] = row[f];
+            return;
+        }
+        d_.v1[l] = v1;
+        d_.v2[l] = v2;
+        d_.v3[l] = v3;
+        d_.a[l] = a;
+        d_.b[l] = b;
+        d_.used[l] = 1;
+    }
+
+    // f(first, last) over [0, count) on the workers, in equal parts
+    template <class F>
+    void share(size_t count, F &&f)
+    {
+        if (!pool_ || count < 64) {
+            f(size_t(0), count);
+            return;
+        }
+        const size_t nt = pool_->size(), part = (count + nt - 1) / nt;
+        const std::function<void(int)> job = [&](int t) {
+            const size_t lo = std::min(count, t * part), hi = std::min(count, lo + part);
+            if (lo < hi) f(lo, hi);
+        };
+        pool_->run(job);
+    }
+
+    // as many pairs from `first` on as the rest of the draw is expected to need
+    void screen_block(long first)
+    {
+        const double left = n_ - l_;
+        const double want = left * (trials_ + 3.0) * 1.01 + 8.0 * std::sqrt(left) * trials_ + 256.0;
+        long count = static_cast<long>(std::min(want, double(1L << 25)));
+        if (capped_) count = std::min(count, max_block_);
+        if (!screen_->screen(seed_, first, std::max(count, 4L), limit_.data(), ctx_.bins, tb_)) {
+            screen_ = nullptr;
+            return;
+        }
+        cand_.resize(tb_.total);
+        size_t at = 0;
+        for (size_t c = 0; c < tb_.chunks; ++c)
+            for (uint32_t k = 0; k < tb_.spans[2 * c + 1]; ++k) cand_[at++] = tb_.spans[2 * c] + k;
+        passed_.resize(tb_.total);
+        share(tb_.total, [&](size_t lo, size_t hi) {
+            for (size_t i = lo; i < hi; ++i) {
+                const uint32_t *r = tb_.records + size_t(TrialBlock::kWords) * cand_[i];
+                passed_[i] = ctx_.accepts(DrawContext<Real>::uniform(r[1]), DrawContext<Real>::uniform(r[2])) ? 1 : 0;
+            }
+        });
+        next_ = 0;
+    }
+
+    void draw_screened(int kept)
+    {
+        if (pos_ < tb_.start || pos_ >= tb_.end) {
+            screen_block(pos_);
+            if (!screen_) return;
+        }
+        picked_.clear();
+        const int before = d_.n_used;
+        while (l_ < n_ && d_.n_used < kept) {
+            while (next_ < cand_.size() && (!passed_[next_] || pair_of(next_) < pos_)) ++next_;
+            if (next_ == cand_.size()) {
+                pos_ = std::max(pos_, tb_.end);
+                break;
+            }
+            const uint32_t *r = tb_.records + size_t(TrialBlock::kWords) * cand_[next_];
+            if (take_trial(pair_of(next_), r[1])) picked_.push_back(Picked{l_, cand_[next_]});
+            ++l_;
+        }
+        share(picked_.size(), [&](size_t lo, size_t hi) {
+            for (size_t i = lo; i < hi; ++i)
+                harmonic(picked_[i].l, before + static_cast<int>(i),
+                         tb_.records + size_t(TrialBlock::kWords) * picked_[i].record + 1);
+        });
+    }
+    long pair_of(size_t i) const { return tb_.start + tb_.records[size_t(TrialBlock::kWords) * cand_[i]]; }
+
     // make pairs [first, first + >= 4) resident
     void fill(long first)
     {
@@ -403,21 +542,31 @@ private:
         };
         pool_->run(job);
     }
-    void pair(long p, Real r[2]) const
-    {
-        const size_t i = static_cast<size_t>(p - blk_.start);
-        r[0] = DrawContext<Real>::uniform(blk_.raw[2 * i]);
-        r[1] = DrawContext<Real>::uniform(blk_.raw[2 * i + 1]);
-    }
 
-    const int n_, ndim_;
+    struct Picked {
+        int l;
+        uint32_t record;
+    };
+    const int n_, ndim_, seed_;
+    const bool rows_only_;
+    const SrmSetup setup_;
     Real cl_[3];
     DrawContext<Real> ctx_;
     HarmonicDraw d_;
+    std::unique_ptr<double[]> rows_;
     PairBlock<Real> blk_;
     long max_block_ = 0, next_size_ = 0;
+    bool capped_ = false;
     long pos_ = 0;  // next pair the loop would read
     int l_ = 0;     // next harmonic index
+    TrialScreen *screen_;
+    double trials_ = 1;
+    std::vector<uint32_t> limit_;
+    TrialBlock tb_;
+    std::vector<uint32_t> cand_;   // records in stream order
+    std::vector<uint8_t> passed_;  // their exact tests
+    std::vector<Picked> picked_;
+    size_t next_ = 0;              // first of cand_ not yet passed by the walk
     std::unique_lock<std::mutex> lock_;
     std::unique_ptr<WorkerPool> own_;
     WorkerPool *pool_ = nullptr;
@@ -433,27 +582,18 @@ std::unique_ptr<HarmonicSampler> HarmonicSampler::create(const SrmConfig &cfg, c
 }
 
 template <class Real>
+std::unique_ptr<HarmonicSampler> HarmonicSampler::create_rows(const SrmConfig &cfg, const SrmSetup &setup, int seed,
+                                                              TrialScreen *screen, int threads, long block_pairs)
+{
+    return std::unique_ptr<HarmonicSampler>(new Sampler<Real>(cfg, setup, seed, threads, block_pairs, true, screen));
+}
+
+template <class Real>
 HarmonicDraw srm_draw(const SrmConfig &cfg, const SrmSetup &s, int seed, int threads, long block_pairs)
 {
     Sampler<Real> w(cfg, s, seed, threads, block_pairs);
     w.draw_until(cfg.nharm);
     return w.take();
-}
-
-void append_table(const SrmSetup &s, const HarmonicDraw &d, int l0, int l1, HarmonicTable &t)
-{
-    const double *m = s.matrix;
-    for (int l = l0; l < l1; ++l) {
-        if (!d.used[l]) continue;
-        const double v[3] = {d.v1[l], d.v2[l], d.v3[l]};
-        // w = M^T v: theta = sum_r v_r ((M p)_r + bar_r) = (M^T v) . p + v . bar
-        t.wx.push_back(v[0] * m[0] + v[1] * m[1] + v[2] * m[2]);
-        t.wy.push_back(v[0] * m[3] + v[1] * m[4] + v[2] * m[5]);
-        t.wz.push_back(v[0] * m[6] + v[1] * m[7] + v[2] * m[8]);
-        const double vbar = v[0] * s.bar[0] + v[1] * s.bar[1] + v[2] * s.bar[2];
-        t.phase.push_back(vbar - std::atan2(d.a[l], d.b[l]));
-        t.amp.push_back(std::hypot(d.a[l], d.b[l]));
-    }
 }
 
 HarmonicTable build_table(const SrmSetup &s, const HarmonicDraw &d)
@@ -465,7 +605,16 @@ HarmonicTable build_table(const SrmSetup &s, const HarmonicDraw &d)
     t.wz.reserve(n);
     t.phase.reserve(n);
     t.amp.reserve(n);
-    append_table(s, d, 0, static_cast<int>(d.used.size()), t);
+    for (size_t l = 0; l < d.used.size(); ++l) {
+        if (!d.used[l]) continue;
+        double row[5];
+        record(s, d.v1[l], d.v2[l], d.v3[l], d.a[l], d.b[l], row);
+        t.wx.push_back(row[0]);
+        t.wy.push_back(row[1]);
+        t.wz.push_back(row[2]);
+        t.phase.push_back(row[3]);
+        t.amp.push_back(row[4]);
+    }
     return t;
 }
 
@@ -477,5 +626,9 @@ template std::unique_ptr<HarmonicSampler> HarmonicSampler::create<float>(const S
                                                                          int, long);
 template std::unique_ptr<HarmonicSampler> HarmonicSampler::create<double>(const SrmConfig &, const SrmSetup &, int,
                                                                           int, long);
+template std::unique_ptr<HarmonicSampler> HarmonicSampler::create_rows<float>(const SrmConfig &, const SrmSetup &, int,
+                                                                              TrialScreen *, int, long);
+template std::unique_ptr<HarmonicSampler> HarmonicSampler::create_rows<double>(const SrmConfig &, const SrmSetup &,
+                                                                               int, TrialScreen *, int, long);
 
 }  // namespace scarf

@@ -65,8 +65,36 @@ struct HarmonicTable {
     int count() const { return static_cast<int>(amp.size()); }
 };
 
+// The same record as five arrays held elsewhere.
+struct HarmonicRows {
+    const double *field[5] = {};  // wx, wy, wz, phase, amp
+    int n = 0;
+};
+
 template <class Real>
 int srm_setup(const SrmConfig &cfg, SrmSetup &out, std::string &err);
+
+// Pairs of a seed's stream screened for the rejection test: every pair in
+// [start, end) that may pass it, in records of kWords words {pair - start,
+// the 8 generator outputs of the pair and the three after it}. Chunk c of the
+// block holds spans[2 c + 1] records from spans[2 c] on; chunks and their
+// records are in stream order.
+struct TrialBlock {
+    static constexpr int kWords = 9;
+    long start = 0, end = 0;
+    const uint32_t *spans = nullptr, *records = nullptr;
+    size_t chunks = 0, total = 0;
+};
+
+// Where the stream is generated and screened, other than by the draw's own
+// threads. A pair is kept when its second output is below limit[b], b the
+// first output's bin of 2^31 / bins values. The block stays valid until the
+// next call. False: not possible now (the draw then screens for itself).
+class TrialScreen {
+public:
+    virtual ~TrialScreen() = default;
+    virtual bool screen(int seed, long first, long count, const uint32_t *limit, int bins, TrialBlock &out) = 0;
+};
 
 // The harmonic draw of one seed as a resumable walk: draw_until(m) runs the
 // reference's draw loop until m harmonics have been kept (or every harmonic
@@ -81,6 +109,11 @@ public:
     template <class Real>
     static std::unique_ptr<HarmonicSampler> create(const SrmConfig &cfg, const SrmSetup &setup, int seed,
                                                    int threads = 0, long block_pairs = 0);
+    // The same draw with its kept harmonics as device records only (rows();
+    // draw() stays empty), its trials screened by `screen` where that pays.
+    template <class Real>
+    static std::unique_ptr<HarmonicSampler> create_rows(const SrmConfig &cfg, const SrmSetup &setup, int seed,
+                                                        TrialScreen *screen, int threads = 0, long block_pairs = 0);
     virtual ~HarmonicSampler() = default;
     // returns the number of kept harmonics so far
     virtual int draw_until(int kept) = 0;
@@ -89,6 +122,8 @@ public:
     // harmonics drawn so far: v/a/b/used for indices [0, position())
     virtual const HarmonicDraw &draw() const = 0;
     virtual int position() const = 0;
+    // records of the kept harmonics [k0, k1) in draw order
+    virtual HarmonicRows rows(int k0, int k1) const = 0;
 };
 
 template <class Real>
@@ -98,7 +133,5 @@ HarmonicDraw srm_draw(const SrmConfig &cfg, const SrmSetup &setup, int seed, int
 int default_draw_threads();
 
 HarmonicTable build_table(const SrmSetup &setup, const HarmonicDraw &draw);
-// the kept harmonics among indices [l0, l1) appended to t
-void append_table(const SrmSetup &setup, const HarmonicDraw &draw, int l0, int l1, HarmonicTable &t);
 
 }  // namespace scarf

@@ -527,24 +527,37 @@ void *Device::field_buffer(size_t bytes, std::string &err)
     return d_field_;
 }
 
-bool Device::upload_table(const HarmonicTable &t, std::string &err)
+// Pinned room for a record, free to be written: the copies queued from it
+// have run.
+bool Device::stage_record(size_t bytes, std::string &err)
 {
-    const int n = t.count();
-    const int np_ = static_cast<int>(round_up(std::max(n, 1), kHarmPad));
-    std::vector<double> rec(size_t(5) * np_, 0.0);
-    for (int l = 0; l < n; ++l) {
-        rec[l] = t.wx[l];
-        rec[np_ + l] = t.wy[l];
-        rec[2 * size_t(np_) + l] = t.wz[l];
-        rec[3 * size_t(np_) + l] = t.phase[l];
-        rec[4 * size_t(np_) + l] = t.amp[l];
-    }
-    if (!reserve(d_harm_, harm_cap_, rec.size() * sizeof(double), err)) return false;
-    HIP_TRY(hipMemcpyAsync(d_harm_, rec.data(), rec.size() * sizeof(double), hipMemcpyHostToDevice, stream_));
     HIP_TRY(hipStreamSynchronize(stream_));
-    nharm_ = np_;
+    if (h_rec_cap_ >= bytes) return true;
+    if (h_rec_) HIP_TRY(hipHostFree(h_rec_));
+    h_rec_ = nullptr;
+    h_rec_cap_ = 0;
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&h_rec_), bytes, hipHostMallocDefault));
+    h_rec_cap_ = bytes;
+    return true;
+}
+
+bool Device::upload_table(const HarmonicRows &t, std::string &err)
+{
+    const int n = t.n;
+    const int np_ = static_cast<int>(round_up(std::max(n, 1), kHarmPad));
+    const size_t bytes = size_t(5) * np_ * sizeof(double);
+    nharm_ = 0;
+    if (!stage_record(bytes, err)) return false;
     amp_max_ = 0;
-    for (int l = 0; l < n; ++l) amp_max_ = std::max(amp_max_, t.amp[l]);
+    for (int f = 0; f < 5; ++f) {
+        double *dst = h_rec_ + size_t(f) * np_;
+        std::copy(t.field[f], t.field[f] + n, dst);
+        std::fill(dst + n, dst + np_, 0.0);
+    }
+    for (int l = 0; l < n; ++l) amp_max_ = std::max(amp_max_, t.field[4][l]);
+    if (!reserve(d_harm_, harm_cap_, bytes, err)) return false;
+    HIP_TRY(hipMemcpyAsync(d_harm_, h_rec_, bytes, hipMemcpyHostToDevice, stream_));
+    nharm_ = np_;
     return true;
 }
 
@@ -890,33 +903,25 @@ bool Device::run_streamed(const Geometry &g, int kernel, int nharm, double scali
     const size_t rec_bytes = size_t(5) * cap * sizeof(double);
     if (!reserve(d_harm_, harm_cap_, rec_bytes, err)) return false;
     nharm_ = 0;  // the streamed record is not a resident table for run()
-    if (h_rec_cap_ < rec_bytes) {
-        HIP_TRY(hipStreamSynchronize(stream_));
-        if (h_rec_) HIP_TRY(hipHostFree(h_rec_));
-        h_rec_ = nullptr;
-        h_rec_cap_ = 0;
-        HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&h_rec_), rec_bytes, hipHostMallocDefault));
-        h_rec_cap_ = rec_bytes;
-    }
+    if (!stage_record(rec_bytes, err)) return false;
     if (!reserve(d_tab_, tab_cap_, plan.table_bytes, err)) return false;
     const int nparts = plan.nparts;
     if (!reserve(d_part_, part_cap_, size_t(3) * nparts * sizeof(double), err)) return false;
 
     timings_ = Timings{};
     HIP_TRY(hipEventRecord(ev_[0], stream_));
-    HIP_TRY(hipStreamSynchronize(stream_));  // the staging buffer is free
     const std::vector<int> targets = chunk_targets(nharm, chunk);
     std::vector<long> slab_first, slab_points;
-    HarmonicTable t;
+    HarmonicRows t;
     int kept = 0;  // harmonics queued so far (padding included in the last chunk)
     bool last = false;
     for (size_t c = 0; !last; ++c) {
-        t = HarmonicTable{};
+        t = HarmonicRows{};
         // the host draws this chunk while the device runs the chunks before it
         if (!feed(c < targets.size() ? targets[c] : nharm, t, last, err)) return false;
-        const int n = t.count();
+        const int n = t.n;
         double amp_max = 0;
-        for (int l = 0; l < n; ++l) amp_max = std::max(amp_max, t.amp[l]);
+        for (int l = 0; l < n; ++l) amp_max = std::max(amp_max, t.field[4][l]);
         if (mfma_zscale(kernel, amp_max) != 1.0) {
             HIP_TRY(hipStreamSynchronize(stream_));
             if (restart) *restart = true;
@@ -932,10 +937,9 @@ bool Device::run_streamed(const Geometry &g, int kernel, int nharm, double scali
         // the chunk's part of each record field, zero-padded, staged in
         // pinned memory (each chunk has its own range: nothing is rewritten
         // while its copy may still run)
-        const double *src[5] = {t.wx.data(), t.wy.data(), t.wz.data(), t.phase.data(), t.amp.data()};
         for (int f = 0; f < 5; ++f) {
             double *dst = h_rec_ + size_t(f) * cap + kept;
-            std::copy(src[f], src[f] + n, dst);
+            std::copy(t.field[f], t.field[f] + n, dst);
             std::fill(dst + n, dst + nh, 0.0);
             HIP_TRY(hipMemcpyAsync(d_harm_ + size_t(f) * cap + kept, dst, size_t(nh) * sizeof(double),
                                    hipMemcpyHostToDevice, stream_));
