@@ -808,11 +808,47 @@ static int scarf_srm_run_body(real *d_field, real stats[])
     return run(d_field, stats);
 }
 
+// One grouped-GEMM launch over the drawn members (records of nps[m] harmonics).
+static int ensemble_grouped(const std::vector<SrmConfig> &cfgs, const std::vector<scarf::SrmSetup> &setups,
+                            const std::vector<std::vector<double>> &records, const std::vector<int> &nps,
+                            real *const *d_fields, int kernel, std::vector<double> &st, double &ms)
+{
+    State &s = state();
+    const int n = static_cast<int>(cfgs.size());
+    if (!s.ensemble) s.ensemble = std::make_unique<scarf::Ensemble>();
+    std::vector<scarf::EnsembleMember> em(n);
+    for (int m = 0; m < n; ++m) {
+        em[m].g = geometry(cfgs[m]);
+        em[m].np_ = nps[m];
+        em[m].record = records[m].data();
+        for (int l = 0; l < nps[m]; ++l) em[m].amp_max = std::max(em[m].amp_max, records[m][4 * size_t(nps[m]) + l]);
+        em[m].scaling = setups[m].scaling;
+        em[m].rescale = cfgs[m].rescale;
+        em[m].sigma = cfgs[m].sigma;
+        em[m].d_field = d_fields[m];
+    }
+    // tiles per member: in one full launch a member's tile is worth its
+    // padded work over the tile's saturated throughput (timed once)
+    if (scarf::TileTuner::enabled()) {
+        std::string terr;
+        for (int m = 0; m < n; ++m) {
+            scarf::TileChoice tc;
+            if (!s.device->tuner().choose_saturated<real>(em[m].g, kernel, s.device->stream(), tc, terr))
+                return fail("tile tuner: " + terr);
+            em[m].tk = tc.tk;
+        }
+    }
+    std::string err;
+    if (!s.ensemble->run<real>(s.device->stream(), kernel, em, st, ms, err)) return fail(err);
+    return 0;
+}
+
 static int scarf_ensemble_execute_body(int n, const struct scarf_member *members, real *const *d_fields, real *stats,
                            int kernel)
 {
     State &s = state();
     if (n < 1 || !members || !d_fields) return fail("scarf_ensemble_execute: empty ensemble or NULL arguments");
+    const bool choose = kernel == scarf::kKernelAuto;
     if (kernel == scarf::kKernelAuto) kernel = scarf::kKernelMfmaBf16x3;
     if (kernel != scarf::kKernelMfmaBf16x3 && kernel != scarf::kKernelMfmaF16x2 && kernel != scarf::kKernelMfmaBf16x2)
         return fail("scarf_ensemble_execute: ensembles run on the MFMA kernels");
@@ -844,16 +880,11 @@ static int scarf_ensemble_execute_body(int n, const struct scarf_member *members
         c.rescale = a.rescale;
         c.nharm = a.nharm > 0 ? a.nharm : s.nharm;
     }
-    // Host draws. Every member's setup first (one per thread), then its
-    // expected draw cost, nharm over the rejection test's acceptance
-    // (cnst * intg(kmin, kmax) / (kmax - kmin)). The members that would hold
-    // up the rest (cost above a share of the total) are drawn one after the
-    // other with every thread of the sampler, the others one per thread,
-    // costliest first. The draws are the exact streams either way.
+    // Every member's setup first, one per thread of a pool.
     std::vector<scarf::SrmSetup> setups(n);
     std::vector<std::vector<double>> records(n);
     std::vector<int> nps(n, 0);
-    std::vector<double> host_s(n, 0.0), cost(n, 0.0);
+    std::vector<double> host_s(n, 0.0);
     std::vector<std::string> errs(n);
     auto guard = [&](int m, auto &&f) {
         try {
@@ -864,91 +895,76 @@ static int scarf_ensemble_execute_body(int n, const struct scarf_member *members
             errs[m] = "internal error";
         }
     };
-    auto on_members = [&](const std::vector<int> &list, auto &&f) {
-        std::atomic<int> next{0};
-        const std::function<void(int)> worker = [&](int) {
-            for (int q = next++; q < static_cast<int>(list.size()); q = next++) guard(list[q], [&] { f(list[q]); });
-        };
-        member_pool().run(worker);
+    std::atomic<int> next{0};
+    const std::function<void(int)> worker = [&](int) {
+        for (int m = next++; m < n; m = next++)
+            guard(m, [&] {
+                const auto t0 = std::chrono::steady_clock::now();
+                std::string e;
+                const int rc = kDouble ? scarf::srm_setup<double>(cfgs[m], setups[m], e)
+                                       : scarf::srm_setup<float>(cfgs[m], setups[m], e);
+                if (rc != 0) errs[m] = e;
+                host_s[m] = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+            });
     };
-    std::vector<int> all(n);
-    for (int m = 0; m < n; ++m) all[m] = m;
-    on_members(all, [&](int m) {
-        const auto t0 = std::chrono::steady_clock::now();
-        std::string e;
-        const int rc = kDouble ? scarf::srm_setup<double>(cfgs[m], setups[m], e)
-                               : scarf::srm_setup<float>(cfgs[m], setups[m], e);
-        if (rc != 0) errs[m] = e;
-        const scarf::SrmSetup &su = setups[m];
-        const double p = su.kmax > su.kmin ? su.cnst * su.band / (su.kmax - su.kmin) : 1.0;
-        cost[m] = cfgs[m].nharm / std::min(1.0, std::max(p, 1e-6));
-        host_s[m] = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-    });
-    for (int m = 0; m < n; ++m)
-        if (!errs[m].empty()) return fail("member " + std::to_string(m) + ": " + errs[m]);
-    auto draw_member = [&](int m, int threads) {
-        const auto t0 = std::chrono::steady_clock::now();
-        const scarf::HarmonicDraw d =
-            kDouble ? scarf::srm_draw<double>(cfgs[m], setups[m], members[m].seed, threads)
-                    : scarf::srm_draw<float>(cfgs[m], setups[m], members[m].seed, threads);
-        const scarf::HarmonicTable t = scarf::build_table(setups[m], d);
-        const int np_ = std::max(64, (t.count() + 63) / 64 * 64);
-        std::vector<double> &r = records[m];
-        r.assign(size_t(5) * np_, 0.0);
-        for (int l = 0; l < t.count(); ++l) {
-            r[l] = t.wx[l];
-            r[np_ + l] = t.wy[l];
-            r[2 * size_t(np_) + l] = t.wz[l];
-            r[3 * size_t(np_) + l] = t.phase[l];
-            r[4 * size_t(np_) + l] = t.amp[l];
-        }
-        nps[m] = np_;
-        host_s[m] += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-    };
-    std::vector<int> order = all;
-    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cost[a] > cost[b]; });
-    const int threads = member_pool().size();
-    double total = 0.0;
-    for (int m = 0; m < n; ++m) total += cost[m];
-    std::vector<int> light;
-    for (int m : order) {
-        if (threads > 1 && cost[m] > total / (2.0 * threads)) {
-            guard(m, [&] { draw_member(m, threads); });  // the sampler's own workers
-        } else {
-            light.push_back(m);
-        }
-    }
-    on_members(light, [&](int m) { draw_member(m, 1); });
+    member_pool().run(worker);
     for (int m = 0; m < n; ++m)
         if (!errs[m].empty()) return fail("member " + std::to_string(m) + ": " + errs[m]);
     if (!ensure_device()) return -1;
-    if (!s.ensemble) s.ensemble = std::make_unique<scarf::Ensemble>();
-    std::vector<scarf::EnsembleMember> em(n);
-    for (int m = 0; m < n; ++m) {
-        em[m].g = geometry(cfgs[m]);
-        em[m].np_ = nps[m];
-        em[m].record = records[m].data();
-        for (int l = 0; l < nps[m]; ++l) em[m].amp_max = std::max(em[m].amp_max, records[m][4 * size_t(nps[m]) + l]);
-        em[m].scaling = setups[m].scaling;
-        em[m].rescale = cfgs[m].rescale;
-        em[m].sigma = cfgs[m].sigma;
-        em[m].d_field = d_fields[m];
-    }
-    // tiles per member: in one full launch a member's tile is worth its
-    // padded work over the tile's saturated throughput (timed once)
-    if (scarf::TileTuner::enabled()) {
-        std::string terr;
-        for (int m = 0; m < n; ++m) {
-            scarf::TileChoice tc;
-            if (!s.device->tuner().choose_saturated<real>(em[m].g, kernel, s.device->stream(), tc, terr))
-                return fail("tile tuner: " + terr);
-            em[m].tk = tc.tk;
-        }
-    }
+    // A member's draw: trials screened on the GPU, exact tests and harmonics
+    // on every worker, so members follow one another.
+    auto draw_member = [&](int m) {
+        const auto t0 = std::chrono::steady_clock::now();
+        std::unique_ptr<scarf::HarmonicSampler> w = sampler(cfgs[m], setups[m], members[m].seed);
+        w->draw_until(INT_MAX);
+        host_s[m] += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+        return w;
+    };
     std::vector<double> st;
     double ms = 0;
     std::string err;
-    if (!s.ensemble->run<real>(s.device->stream(), kernel, em, st, ms, err)) return fail(err);
+    // Under auto the members run one after the other by the fast transform,
+    // each drawn while the device computes the one before, where that is
+    // faster than all draws followed by the grouped launch (5e10 points and
+    // harmonics per ms, at least 8e-5 ms per harmonic of the longest member).
+    // Draws: measured 0.15 ms and 2.5e-5 ms per harmonic.
+    bool transform = choose;
+    double by_transform = 0, draws = 0, work = 0, longest = 0;
+    std::vector<scarf::Device::Member> tm(transform ? n : 0);
+    for (int m = 0; transform && m < n; ++m) {
+        tm[m].g = geometry(cfgs[m]);
+        tm[m].nharm = cfgs[m].nharm;
+        tm[m].scaling = setups[m].scaling;
+        tm[m].sigma = cfgs[m].sigma;
+        tm[m].rescale = cfgs[m].rescale;
+        tm[m].d_field = d_fields[m];
+        scarf::TransformPlan plan;
+        transform = scarf::transform_plan(tm[m].g, (cfgs[m].nharm + 63) / 64 * 64, kDouble, plan);
+        by_transform += scarf::transform_ms(plan, kDouble);
+        draws += 0.15 + 2.5e-5 * cfgs[m].nharm;
+        work += double(tm[m].g.points()) * cfgs[m].nharm;
+        longest = std::max(longest, double(cfgs[m].nharm));
+    }
+    const double grouped = draws + 0.1 + std::max(work / 5e10, 8e-5 * longest);
+    if (transform && std::max(by_transform, draws) < grouped && s.device->reserve_members<real>(tm)) {
+        std::unique_ptr<scarf::HarmonicSampler> w;
+        const scarf::Device::MemberDraw draw = [&](int m, scarf::HarmonicRows &rows, std::string &) {
+            w.reset();  // its lease of the workers ends before the next draw
+            w = draw_member(m);
+            rows = w->rows(0, w->draw_until(INT_MAX));
+            return true;
+        };
+        if (!s.device->run_members<real>(tm, draw, st, ms, err)) return fail(err);
+    } else {
+        for (int m = 0; m < n; ++m) {
+            const std::unique_ptr<scarf::HarmonicSampler> w = draw_member(m);
+            const scarf::HarmonicRows t = w->rows(0, w->draw_until(INT_MAX));
+            nps[m] = std::max(64, (t.n + 63) / 64 * 64);
+            records[m].assign(size_t(5) * nps[m], 0.0);
+            for (int f = 0; f < 5; ++f) std::copy(t.field[f], t.field[f] + t.n, records[m].begin() + size_t(f) * nps[m]);
+        }
+        if (ensemble_grouped(cfgs, setups, records, nps, d_fields, kernel, st, ms) != 0) return -1;
+    }
     s.ensemble_ms = ms;
     if (stats) {
         for (int m = 0; m < n; ++m) {

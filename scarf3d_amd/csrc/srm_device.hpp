@@ -122,6 +122,25 @@ public:
     bool run_noalloc(const Geometry &g, int kernel, double scaling, const Epilogue &ep, Real *d_field,
                      double *stats_out, std::string &err);
 
+    // Realizations of structured grids by the transform, one after the other
+    // on the stream: draw(m, rows) gives member m's harmonics, and the host
+    // draws member m + 1 while the device computes member m. stats: six values
+    // per member as run()'s. reserve_members makes the room they need (false,
+    // with no error left behind: the device has not got it).
+    struct Member {
+        Geometry g;
+        int nharm = 0;  // at most this many are kept
+        double scaling = 0, sigma = 0;
+        int rescale = 0;
+        void *d_field = nullptr;
+    };
+    using MemberDraw = std::function<bool(int m, HarmonicRows &rows, std::string &err)>;
+    template <class Real>
+    bool reserve_members(const std::vector<Member> &members);
+    template <class Real>
+    bool run_members(const std::vector<Member> &members, const MemberDraw &draw, std::vector<double> &stats,
+                     double &device_ms, std::string &err);
+
     hipStream_t stream() const { return stream_; }
     const Timings &timings() const { return timings_; }
 
@@ -188,6 +207,11 @@ private:
     double *d_harm_ = nullptr;
     size_t harm_cap_ = 0;
     bool stage_record(size_t bytes, std::string &err);
+    // rows, zero-padded to np_ per field, to a device record by way of their
+    // place in the staging memory
+    bool queue_record(const HarmonicRows &t, int np_, double *staged, double *record, std::string &err);
+    double *d_member_ = nullptr;  // record of run_members (the resident one stays)
+    size_t member_cap_ = 0;
     double *h_rec_ = nullptr;  // pinned staging of the record
     size_t h_rec_cap_ = 0;
     // per-axis tables (FP32 or FP64 revolutions, operand tables of the GEMM)

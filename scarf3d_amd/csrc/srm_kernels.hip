@@ -460,7 +460,7 @@ Device::~Device()
     if (device_ < 0) return;
     hipSetDevice(device_);
     if (stream_) hipStreamSynchronize(stream_);
-    void *bufs[] = {d_harm_, d_tab_, d_pts_, d_part_, d_stat_, d_field_, d_poi_};
+    void *bufs[] = {d_harm_, d_member_, d_tab_, d_pts_, d_part_, d_stat_, d_field_, d_poi_};
     for (void *b : bufs)
         if (b) hipFree(b);
     if (h_stat_) hipHostFree(h_stat_);
@@ -541,23 +541,93 @@ bool Device::stage_record(size_t bytes, std::string &err)
     return true;
 }
 
+bool Device::queue_record(const HarmonicRows &t, int np_, double *staged, double *record, std::string &err)
+{
+    for (int f = 0; f < 5; ++f) {
+        double *dst = staged + size_t(f) * np_;
+        std::copy(t.field[f], t.field[f] + t.n, dst);
+        std::fill(dst + t.n, dst + np_, 0.0);
+    }
+    HIP_TRY(hipMemcpyAsync(record, staged, size_t(5) * np_ * sizeof(double), hipMemcpyHostToDevice, stream_));
+    return true;
+}
+
 bool Device::upload_table(const HarmonicRows &t, std::string &err)
 {
-    const int n = t.n;
-    const int np_ = static_cast<int>(round_up(std::max(n, 1), kHarmPad));
+    const int np_ = static_cast<int>(round_up(std::max(t.n, 1), kHarmPad));
     const size_t bytes = size_t(5) * np_ * sizeof(double);
     nharm_ = 0;
-    if (!stage_record(bytes, err)) return false;
-    amp_max_ = 0;
-    for (int f = 0; f < 5; ++f) {
-        double *dst = h_rec_ + size_t(f) * np_;
-        std::copy(t.field[f], t.field[f] + n, dst);
-        std::fill(dst + n, dst + np_, 0.0);
-    }
-    for (int l = 0; l < n; ++l) amp_max_ = std::max(amp_max_, t.field[4][l]);
-    if (!reserve(d_harm_, harm_cap_, bytes, err)) return false;
-    HIP_TRY(hipMemcpyAsync(d_harm_, h_rec_, bytes, hipMemcpyHostToDevice, stream_));
+    if (!stage_record(bytes, err) || !reserve(d_harm_, harm_cap_, bytes, err) || !queue_record(t, np_, h_rec_, d_harm_, err))
+        return false;
     nharm_ = np_;
+    amp_max_ = 0;
+    for (int l = 0; l < t.n; ++l) amp_max_ = std::max(amp_max_, t.field[4][l]);
+    return true;
+}
+
+template <class Real>
+bool Device::reserve_members(const std::vector<Member> &members)
+{
+    size_t rec = 0, staged = 0, work = 0, parts = 0;
+    std::string err;
+    bool ok = hipSetDevice(device_) == hipSuccess;
+    for (const Member &m : members) {
+        TransformPlan plan;
+        const int np_ = static_cast<int>(round_up(std::max(m.nharm, 1), kHarmPad));
+        if (!ok || !transform_plan(m.g, np_, sizeof(Real) == sizeof(double), plan)) return false;
+        rec = std::max(rec, size_t(5) * np_ * sizeof(double));
+        staged += size_t(5) * np_ * sizeof(double);
+        work = std::max(work, plan.bytes);
+        parts = std::max(parts, size_t(3) * (plan.nparts + plan.groups));
+    }
+    ok = stage_record(staged, err) && reserve(d_member_, member_cap_, rec, err) && reserve(d_tab_, tab_cap_, work, err) &&
+         reserve(d_part_, part_cap_, (parts + 6 * members.size()) * sizeof(double), err);
+    if (!ok) (void)hipGetLastError();
+    return ok;
+}
+
+template <class Real>
+bool Device::run_members(const std::vector<Member> &members, const MemberDraw &draw, std::vector<double> &stats,
+                         double &device_ms, std::string &err)
+{
+    const size_t n = members.size();
+    double *staged = h_rec_, *stat = d_part_ + part_cap_ / sizeof(double) - 6 * n;
+    HIP_TRY(hipSetDevice(device_));
+    HIP_TRY(hipEventRecord(ev_[0], stream_));
+    for (size_t q = 0; q < n; ++q) {
+        const Member &m = members[q];
+        HarmonicRows t;
+        if (!draw(static_cast<int>(q), t, err)) {
+            (void)hipStreamSynchronize(stream_);
+            return false;
+        }
+        const int np_ = static_cast<int>(round_up(std::max(t.n, 1), kHarmPad));
+        TransformPlan plan;
+        if (t.n > m.nharm || !transform_plan(m.g, np_, sizeof(Real) == sizeof(double), plan)) {
+            err = "ensemble member outside its plan";
+            return false;
+        }
+        Real *field = static_cast<Real *>(m.d_field);
+        if (!queue_record(t, np_, staged, d_member_, err) ||
+            !transform_field<Real>(plan, m.g, d_member_, d_tab_, m.scaling, field, d_part_, stream_, ev_[1], err))
+            return false;
+        staged += size_t(5) * np_;
+        stats_finalize<Real><<<1, 256, 0, stream_>>>(d_part_ + 3 * size_t(plan.nparts), plan.groups, m.sigma, stat + 6 * q);
+        HIP_TRY(hipGetLastError());
+        if (m.rescale == 1) {
+            const int blocks = int(std::min<long>((m.g.points() + 255) / 256, 16384));
+            epilogue_grid<Real><<<blocks, 256, 0, stream_>>>(field, m.g.nx, m.g.ny, m.g.nz, m.g.ox, m.g.oy, m.g.oz,
+                                                             m.g.ds, stat + 6 * q, 1, nullptr, 0, -999.0, -999.0);
+            HIP_TRY(hipGetLastError());
+        }
+    }
+    HIP_TRY(hipEventRecord(ev_[4], stream_));
+    stats.assign(6 * n, 0.0);
+    HIP_TRY(hipMemcpyAsync(stats.data(), stat, 6 * n * sizeof(double), hipMemcpyDeviceToHost, stream_));
+    HIP_TRY(hipStreamSynchronize(stream_));
+    float ms = 0.f;
+    HIP_TRY(hipEventElapsedTime(&ms, ev_[0], ev_[4]));
+    device_ms = ms;
     return true;
 }
 
@@ -980,6 +1050,12 @@ template bool Device::run<float>(const Geometry &, int, double, const Epilogue &
                                  const SlabHook *, int);
 template bool Device::run<double>(const Geometry &, int, double, const Epilogue &, double *, double *,
                                   std::string &, const SlabHook *, int);
+template bool Device::reserve_members<float>(const std::vector<Member> &);
+template bool Device::reserve_members<double>(const std::vector<Member> &);
+template bool Device::run_members<float>(const std::vector<Member> &, const MemberDraw &, std::vector<double> &, double &,
+                                         std::string &);
+template bool Device::run_members<double>(const std::vector<Member> &, const MemberDraw &, std::vector<double> &,
+                                          double &, std::string &);
 template bool Device::run_noalloc<float>(const Geometry &, int, double, const Epilogue &, float *, double *,
                                          std::string &);
 template bool Device::run_noalloc<double>(const Geometry &, int, double, const Epilogue &, double *, double *,

@@ -168,3 +168,56 @@ print("ok")
     r = subprocess.run([sys.executable, "-c", code.replace("DIRECT", repr(direct))], cwd=ROOT, capture_output=True,
                        text=True, timeout=100, env={**os.environ, "SCARF_TUNE": "0"})
     assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stdout + r.stderr
+
+
+def _members(nharm, n=6):
+    out = []
+    for q in range(n):
+        out.append(dict(fe=(60 + 17 * q, 50 + 9 * q, 24 + 5 * q), ds=25.0, acf=q % 2, cl=(300.0, 250.0, 180.0), sigma=0.05,
+                        hurst=0.1 + 0.1 * q, nharm=nharm + 64 * q, seed=q + 1, rescale=int(q == 2),
+                        alpha=10.0 * (q == 3)))
+    out[4].update(nd=2, fe=(210, 150, 1), cl=(400.0, 300.0, 0.0))
+    return out
+
+
+@pytest.mark.parametrize("flavour", ["f", "d"])
+def test_ensemble_members_equal_single_runs(request, flavour):
+    """Under auto an ensemble of many harmonics runs its members by the
+    transform: each is its single run bit for bit, and a table drawn before
+    stays resident."""
+    lib = request.getfixturevalue("lib_" + flavour)
+    hip = Hip()
+    members = _members(3000)
+    bufs = [hip.empty(int(np.prod(m["fe"])), lib.dtype) for m in members]
+    cfg = structured_cfg(n=(40, 30, 20), ds=25.0, cl=(300.0, 250.0, 180.0), nharm=2000, real=lib.dtype)
+    init_library(lib, cfg)
+    lib.set_kernel("auto")
+    lib.srm_draw(5)
+    d = hip.empty(40 * 30 * 20, lib.dtype)
+    lib.srm_run(d.ptr)
+    before = d.numpy().copy()
+    for _ in range(2):
+        stats = lib.ensemble_execute(members, [b.ptr for b in bufs])
+    lib.srm_run(d.ptr)
+    assert np.array_equal(d.numpy(), before)
+    lib.finalize()
+    for m, b, st in zip(members, bufs, stats):
+        print("[case]", flavour, m["fe"], m["nharm"], flush=True)
+        c = structured_cfg(n=m["fe"], ds=m["ds"], acf=m["acf"], cl=m["cl"], sigma=m["sigma"], hurst=m["hurst"],
+                           nharm=m["nharm"], alpha=m["alpha"], rescale=m["rescale"], real=lib.dtype)
+        init_library(lib, c)
+        single, one = lib.execute(m["seed"])
+        lib.finalize()
+        assert np.array_equal(b.numpy(), single.reshape(-1, order="F"))
+        assert np.array_equal(st[:4], one[:4])
+
+
+def test_ensemble_of_few_harmonics_is_grouped(lib_f):
+    hip = Hip()
+    members = [dict(m, nd=3, fe=(600, 500, 40), cl=(600.0, 500.0, 200.0)) for m in _members(64)]
+    bufs = [hip.empty(int(np.prod(m["fe"])), np.float32) for m in members]
+    a = lib_f.ensemble_execute(members, [b.ptr for b in bufs])
+    fields = [b.numpy().copy() for b in bufs]
+    b_ = lib_f.ensemble_execute(members, [b.ptr for b in bufs], "mfma_bf16x3")
+    assert np.array_equal(a[:, :4], b_[:, :4])
+    assert all(np.array_equal(f, b.numpy()) for f, b in zip(fields, bufs))
