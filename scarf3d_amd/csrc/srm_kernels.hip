@@ -359,6 +359,14 @@ __global__ __launch_bounds__(256) void direct_points(const double *__restrict__ 
 // Epilogue: rescale (field*s - mean, src/scarflib_srm.f90:897-912) and the
 // mute/taper of every point of interest in order (taper_factor), at `real`
 // precision without contraction, as the reference computes them on the host.
+//
+// One wave per x-line. Lane q tests point of interest q against the line: one
+// farther than mute + taper (or mute) in y and z alone, by more than any
+// rounding, changes no value of it, and only the others are evaluated, in
+// their order. A line that nothing changes is not read. HBM-bound then: 16
+// points of interest on 1024 x 1024 x 512 with a rescale take 0.80 ms, where
+// every point of interest at every value, with the value's indices by 64-bit
+// division, took 5.9 ms.
 template <class Real>
 __global__ __launch_bounds__(256) void epilogue_grid(Real *__restrict__ field, int nx, int ny, int nz, int ox,
                                                      int oy, int oz, double ds_, const double *__restrict__ stat,
@@ -366,22 +374,50 @@ __global__ __launch_bounds__(256) void epilogue_grid(Real *__restrict__ field, i
                                                      double mute_, double taper_)
 {
 #pragma clang fp contract(off)
-    const long n = long(nx) * ny * nz;
+    constexpr int U = 4;  // values per lane in flight
+    const long rows = long(ny) * nz, waves = long(gridDim.x) * (blockDim.x >> 6);
+    const int lane = threadIdx.x & 63;
     const Real ds = static_cast<Real>(ds_), mute = static_cast<Real>(mute_), taper = static_cast<Real>(taper_);
     const Real sc = static_cast<Real>(stat[5]), mu = static_cast<Real>(stat[4]);
-    for (long e = blockIdx.x * long(blockDim.x) + threadIdx.x; e < n; e += long(gridDim.x) * blockDim.x) {
-        Real v = field[e];
-        if (rescale) v = v * sc - mu;
-        if (npoi > 0) {
-            const int i = int(e % nx), j = int((e / nx) % ny), k = int(e / (long(nx) * ny));
-            for (int q = 0; q < npoi; ++q) {
-                Real dx = static_cast<Real>(i + ox) * ds - static_cast<Real>(poi[3 * q]);
-                Real dy = static_cast<Real>(j + oy) * ds - static_cast<Real>(poi[3 * q + 1]);
-                Real dz = static_cast<Real>(k + oz) * ds - static_cast<Real>(poi[3 * q + 2]);
-                v = taper_factor(v, dx * dx, dy * dy, dz * dz, mute, taper);
+    const double reach = max(static_cast<double>(mute), static_cast<double>(mute) + static_cast<double>(taper));
+    const double far2 = reach >= 0.0 ? reach * reach * (1.0 + 1e-4) : -1.0;
+    for (long row = blockIdx.x * long(blockDim.x >> 6) + (threadIdx.x >> 6); row < rows; row += waves) {
+        const int j = int(row % ny), k = int(row / ny);
+        const Real py = static_cast<Real>(j + oy) * ds, pz = static_cast<Real>(k + oz) * ds;
+        auto near = [&](int q) {  // whether point of interest q can change the line
+            if (q >= npoi) return false;
+            const Real dy = py - static_cast<Real>(poi[3 * q + 1]), dz = pz - static_cast<Real>(poi[3 * q + 2]);
+            return static_cast<double>(dy) * dy + static_cast<double>(dz) * dz <= far2;
+        };
+        uint64_t first = __ballot(near(lane)), any = first;
+        for (int q0 = 64; q0 < npoi; q0 += 64) any |= __ballot(near(q0 + lane));
+        if (!rescale && !any) continue;
+        Real *line = field + row * nx;
+        for (int i0 = lane; i0 - lane < nx; i0 += 64 * U) {
+            Real v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[u] = i0 + 64 * u < nx ? line[i0 + 64 * u] : Real(0);
+            if (rescale) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) v[u] = v[u] * sc - mu;
             }
+            for (int q0 = 0; any && q0 < npoi; q0 += 64) {
+                for (uint64_t m = q0 == 0 ? first : __ballot(near(q0 + lane)); m; m &= m - 1) {
+                    const int q = q0 + __ffsll(static_cast<unsigned long long>(m)) - 1;
+                    const Real px = static_cast<Real>(poi[3 * q]);
+                    const Real dy = py - static_cast<Real>(poi[3 * q + 1]);
+                    const Real dz = pz - static_cast<Real>(poi[3 * q + 2]);
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const Real dx = static_cast<Real>(i0 + 64 * u + ox) * ds - px;
+                        v[u] = taper_factor(v[u], dx * dx, dy * dy, dz * dz, mute, taper);
+                    }
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (i0 + 64 * u < nx) line[i0 + 64 * u] = v[u];
         }
-        field[e] = v;
     }
 }
 
@@ -615,7 +651,7 @@ bool Device::run_members(const std::vector<Member> &members, const MemberDraw &d
         stats_finalize<Real><<<1, 256, 0, stream_>>>(d_part_ + 3 * size_t(plan.nparts), plan.groups, m.sigma, stat + 6 * q);
         HIP_TRY(hipGetLastError());
         if (m.rescale == 1) {
-            const int blocks = int(std::min<long>((m.g.points() + 255) / 256, 16384));
+            const int blocks = int(std::min<long>((long(m.g.ny) * m.g.nz + 3) / 4, 16384));
             epilogue_grid<Real><<<blocks, 256, 0, stream_>>>(field, m.g.nx, m.g.ny, m.g.nz, m.g.ox, m.g.oy, m.g.oz,
                                                              m.g.ds, stat + 6 * q, 1, nullptr, 0, -999.0, -999.0);
             HIP_TRY(hipGetLastError());
@@ -806,8 +842,9 @@ bool Device::finish(const Geometry &g, const Epilogue &ep, Real *d_field, int np
                                    stream_));
         }
         const int blocks = int(std::min<long>((npts + 255) / 256, 16384));
+        const int row_blocks = int(std::min<long>((long(g.ny) * g.nz + 3) / 4, 16384));
         if (g.structured)
-            epilogue_grid<Real><<<blocks, 256, 0, stream_>>>(d_field, g.nx, g.ny, g.nz, g.ox, g.oy, g.oz, g.ds,
+            epilogue_grid<Real><<<row_blocks, 256, 0, stream_>>>(d_field, g.nx, g.ny, g.nz, g.ox, g.oy, g.oz, g.ds,
                                                              stat, ep.rescale == 1, poi, npoi, ep.mute, ep.taper);
         else
             epilogue_points<Real><<<blocks, 256, 0, stream_>>>(d_field, npts, d_pts_, d_pts_ + npts,
