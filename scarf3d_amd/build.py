@@ -37,6 +37,7 @@ UNITS = [
     ("srm_kernels.hip", DEVICE, "srm_kernels.o"),
     ("srm_mfma.hip", DEVICE, "srm_mfma.o"),
     ("srm_transform.hip", DEVICE, "srm_transform.o"),
+    ("srm_points.hip", DEVICE, "srm_points.o"),
     ("srm_draw.hip", DEVICE, "srm_draw.o"),
     ("srm_host.cpp", DEVICE + HOST_EXACT, "srm_host.o"),
     ("quadpack.cpp", DEVICE + HOST_EXACT, "quadpack.o"),
@@ -159,7 +160,7 @@ def build(jobs: int = 4, verbose: bool = False) -> list[Path]:
         futs = [ex.submit(_compile, s, f, o, verbose) for s, f, o in UNITS]
         for fut in futs:
             fut.result()
-    shared = ["srm_kernels.o", "srm_mfma.o", "srm_transform.o", "srm_draw.o", "srm_host.o", "quadpack.o", "fim.o", "fim_host.o"]
+    shared = ["srm_kernels.o", "srm_mfma.o", "srm_transform.o", "srm_points.o", "srm_draw.o", "srm_host.o", "quadpack.o", "fim.o", "fim_host.o"]
     outs = []
     for obj, name in (("scarf_capi_f.o", "libscarf3df.so"), ("scarf_capi_d.o", "libscarf3d.so")):
         out = LIB / name

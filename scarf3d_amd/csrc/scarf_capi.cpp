@@ -29,6 +29,7 @@
 
 #include "../../include/scarf3d.h"
 #include "../../include/scarf3d_srm.h"
+#include "extent.hpp"
 #include "fim.hpp"
 #include "srm_device.hpp"
 #include "srm_draw.hpp"
@@ -207,17 +208,20 @@ scarf::Geometry geometry(const SrmConfig &cfg)
         g.ds = static_cast<real>(cfg.ds);
     } else {
         g.npts = cfg.npts;
+        g.flat = cfg.nd != 3;
     }
     return g;
 }
 
 // The kernel that computes the field: with auto on a grid, the fast transform
 // where it is the faster one (the decision takes the configured harmonic
-// count, so that every entry point makes the same one).
+// count, so that every entry point makes the same one); on a point list the
+// device decides, which knows the points' extent.
 int field_kernel(const SrmConfig &cfg)
 {
     const int k = resolve_kernel(cfg);
-    if (current_kernel() != scarf::kKernelAuto || !cfg.structured) return k;
+    if (current_kernel() != scarf::kKernelAuto) return k;
+    if (!cfg.structured) return scarf::kKernelTransform;
     const scarf::Geometry g = geometry(cfg);
     scarf::TransformPlan plan;
     if (!scarf::transform_plan(g, (cfg.nharm + 63) / 64 * 64, kDouble, plan)) return k;
@@ -291,7 +295,7 @@ int prepare(int seed)
     s.host_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     if (!s.device->upload_table(draw->rows(0, kept), err)) return fail(err);
     if (!s.cfg.structured) {
-        if (!s.device->upload_points<real>(s.x, s.y, s.z, s.cfg.npts, err)) return fail(err);
+        if (!s.device->upload_points<real>(s.x, s.y, s.z, s.cfg.npts, drain_pool(), err)) return fail(err);
     }
     s.table_ready = true;
     s.error.clear();
@@ -352,7 +356,7 @@ int execute_fim(int seed, real *d_field, real stats[], const scarf::Device::Slab
     if (!s.fim) s.fim = std::make_unique<scarf::FimDevice>();
     const double *pts = nullptr;
     if (!s.cfg.structured) {
-        if (!s.device->upload_points<real>(s.x, s.y, s.z, s.cfg.npts, err)) return fail(err);
+        if (!s.device->upload_points<real>(s.x, s.y, s.z, s.cfg.npts, drain_pool(), err)) return fail(err);
         pts = s.device->points();
     }
     int fsi[3], fei[3];
@@ -590,9 +594,14 @@ static void scarf_nocart_initialize_body(const int nd, const int npts, const rea
             continue;
         }
         real lo = axes[a][0], hi = axes[a][0];
-        for (int i = 1; i < npts; ++i) {
-            lo = std::min(lo, axes[a][i]);
-            hi = std::max(hi, axes[a][i]);
+        if (npts < 65536) {
+            scarf::add_extent(axes[a], npts, lo, hi);
+        } else {
+            scarf::WorkerPool &pool = drain_pool();
+            std::vector<real> l(pool.size(), lo), h(pool.size(), hi);
+            scarf::in_parts(pool, npts, [&](int t, size_t p, size_t q) { scarf::add_extent(axes[a] + p, q - p, l[t], h[t]); });
+            lo = *std::min_element(l.begin(), l.end());
+            hi = *std::max_element(h.begin(), h.end());
         }
         c.nc[a] = lo;
         c.fc[a] = hi;

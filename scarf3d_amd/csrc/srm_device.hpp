@@ -21,7 +21,7 @@ enum Kernel : int {
     kKernelMfmaBf16x3 = 3,  // per-slab GEMM, 3-term bf16 split, 6 MFMA products
     kKernelMfmaF16x2 = 4,   // per-slab GEMM, scaled 2-term fp16 split, 3 products
     kKernelMfmaBf16x2 = 5,  // per-slab GEMM, 2-term bf16 split, 3 products (below 1e-5 sigma)
-    kKernelTransform = 6,   // plane-wise fast transform (srm_transform.hpp); chosen by auto, not part of the API
+    kKernelTransform = 6,   // fast transform (srm_transform.hpp, srm_points.hpp); chosen by auto, not part of the API
 };
 const char *kernel_name(int k);
 
@@ -32,6 +32,7 @@ struct Geometry {
     int ox = 0, oy = 0, oz = 0;       // global 0-based offset of the block (fs - 1)
     double ds = 0;                    // grid step
     long npts = 0;                    // unstructured point count
+    bool flat = false;                // of points in a plane (2D)
     long points() const { return structured ? long(nx) * ny * nz : npts; }
 };
 
@@ -51,6 +52,7 @@ struct Timings {
 };
 
 class TileTuner;
+class WorkerPool;
 
 class Device {
 public:
@@ -63,10 +65,10 @@ public:
     bool ensure(std::string &err);
 
     // Uploads the harmonic table (FP64 SoA) and, for point lists, the
-    // coordinates (widened to FP64).
+    // coordinates (widened to FP64 there; `pool` fills the staging memory).
     bool upload_table(const HarmonicRows &t, std::string &err);
     template <class Real>
-    bool upload_points(const Real *x, const Real *y, const Real *z, long n, std::string &err);
+    bool upload_points(const Real *x, const Real *y, const Real *z, long n, WorkerPool &pool, std::string &err);
 
     // Runs tables + field + statistics (+ epilogue) into d_field (device,
     // `Real` elements). stats_out[0..3] = {count, mean, variance, sigma_d}
@@ -76,7 +78,8 @@ public:
     // computed (MFMA grids with no rescale or taper), else once for the whole
     // field at the end.
     // `otherwise`: the kernel that runs instead of kKernelTransform when the
-    // device has no room for the transform's workspace.
+    // device has no room for the transform's workspace, or for a point list
+    // that it serves better.
     using SlabHook = std::function<bool(long, long, std::string &)>;
     template <class Real>
     bool run(const Geometry &g, int kernel, double scaling, const Epilogue &ep, Real *d_field,
@@ -201,6 +204,7 @@ private:
     void *scratch_ = nullptr;  // this device's copy of the no-alloc scratch array
     int nharm_ = 0;
     double amp_max_ = 0;  // largest amplitude of the resident table
+    double wmax_[3] = {}; // and its largest |wx|, |wy|, |wz|
     std::unique_ptr<TileTuner> tuner_;
     int last_nbx_ = 0, last_tk_ = 0;
     // harmonic record: wx, wy, wz (rad/m), phase (rad), amp; plus revolution copies
@@ -221,6 +225,11 @@ private:
     double *d_pts_ = nullptr;
     size_t pts_cap_ = 0;
     long npts_ = 0;
+    double pts_lo_[3] = {}, pts_hi_[3] = {};  // their extent
+    char *h_pts_ = nullptr;                   // pinned staging, kPointStages buffers of kPointStage bytes
+    static constexpr size_t kPointStage = size_t(2) << 20;
+    static constexpr int kPointStages = 4;
+    hipEvent_t pts_ev_[kPointStages] = {};
     // statistics partials and results
     double *d_part_ = nullptr;
     size_t part_cap_ = 0;

@@ -18,6 +18,7 @@
 #include <type_traits>
 
 #include "fft_lds.hpp"
+#include "kaiser_bessel.hpp"
 #include "srm_stats.hpp"
 
 namespace scarf {
@@ -64,26 +65,10 @@ constexpr int kClass = 8 * kTiles<Real>;
 template <class Real>
 constexpr int kFirstX = sizeof(Real) == 4 ? 8 : 4;
 
-// e^-beta I0(beta sqrt(1 - (2 x / w)^2)) by its power series, all terms
-// positive: K terms reach 1e-17 of the sum for every beta of w = 9 (16) taps
-template <int K>
-__device__ inline double kaiser_bessel(double x, int w, double beta, double e_beta)
-{
-    const double u = 2.0 * x / w;
-    const double t = 0.25 * beta * beta * (1.0 - u * u);
-    if (!(t >= 0.0)) return 0.0;
-    double s = 1.0;
-#pragma unroll
-    for (int k = K; k >= 1; --k) s = fma(s, t * (1.0 / (double(k) * k)), 1.0);
-    return s * e_beta;
-}
-
-// 1 / phi^ at j / n: e^beta a / (w sinh a), a = sqrt(beta^2 - (pi w j / n)^2)
+// 1 / phi^ of output j of a transform of n frequencies
 __device__ inline double deconvolution(int j, int n, int w, double beta)
 {
-    const double r = kPiD * w * j / n;
-    const double a = sqrt(beta * beta - r * r);
-    return 2.0 * a * exp(beta - a) / (w * (1.0 - exp(-2.0 * a)));
+    return kaiser_bessel_inverse(2.0 * kPiD * j / n, w, beta);
 }
 
 // One harmonic on the oversampled frequency grid: positions gx in [0, m], gy,
