@@ -4,10 +4,6 @@
 #pragma once
 #include <algorithm>
 #include <cstddef>
-#include <functional>
-#include <vector>
-
-#include "worker_pool.hpp"
 
 namespace scarf {
 
@@ -33,18 +29,6 @@ void add_extent(const Real *src, size_t n, Real &lo, Real &hi)
         lo = std::min(lo, l[q]);
         hi = std::max(hi, h[q]);
     }
-}
-
-// body(part, first, last) over [0, n) in equal parts on the pool's threads
-template <class F>
-void in_parts(WorkerPool &pool, size_t n, F &&body)
-{
-    const size_t threads = pool.size(), part = (n + threads - 1) / threads;
-    const std::function<void(int)> job = [&](int t) {
-        const size_t a = std::min(n, t * part), b = std::min(n, a + part);
-        if (a < b) body(t, a, b);
-    };
-    pool.run(job);
 }
 
 }  // namespace scarf

@@ -295,7 +295,7 @@ int prepare(int seed)
     s.host_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     if (!s.device->upload_table(draw->rows(0, kept), err)) return fail(err);
     if (!s.cfg.structured) {
-        if (!s.device->upload_points<real>(s.x, s.y, s.z, s.cfg.npts, drain_pool(), err)) return fail(err);
+        if (!s.device->upload_points<real>(s.x, s.y, s.z, s.cfg.npts, err)) return fail(err);
     }
     s.table_ready = true;
     s.error.clear();
@@ -356,7 +356,7 @@ int execute_fim(int seed, real *d_field, real stats[], const scarf::Device::Slab
     if (!s.fim) s.fim = std::make_unique<scarf::FimDevice>();
     const double *pts = nullptr;
     if (!s.cfg.structured) {
-        if (!s.device->upload_points<real>(s.x, s.y, s.z, s.cfg.npts, drain_pool(), err)) return fail(err);
+        if (!s.device->upload_points<real>(s.x, s.y, s.z, s.cfg.npts, err)) return fail(err);
         pts = s.device->points();
     }
     int fsi[3], fei[3];
@@ -594,15 +594,7 @@ static void scarf_nocart_initialize_body(const int nd, const int npts, const rea
             continue;
         }
         real lo = axes[a][0], hi = axes[a][0];
-        if (npts < 65536) {
-            scarf::add_extent(axes[a], npts, lo, hi);
-        } else {
-            scarf::WorkerPool &pool = drain_pool();
-            std::vector<real> l(pool.size(), lo), h(pool.size(), hi);
-            scarf::in_parts(pool, npts, [&](int t, size_t p, size_t q) { scarf::add_extent(axes[a] + p, q - p, l[t], h[t]); });
-            lo = *std::min_element(l.begin(), l.end());
-            hi = *std::max_element(h.begin(), h.end());
-        }
+        scarf::add_extent(axes[a], npts, lo, hi);
         c.nc[a] = lo;
         c.fc[a] = hi;
     }

@@ -52,7 +52,6 @@ struct Timings {
 };
 
 class TileTuner;
-class WorkerPool;
 
 class Device {
 public:
@@ -65,10 +64,10 @@ public:
     bool ensure(std::string &err);
 
     // Uploads the harmonic table (FP64 SoA) and, for point lists, the
-    // coordinates (widened to FP64 there; `pool` fills the staging memory).
+    // coordinates (widened to FP64 there).
     bool upload_table(const HarmonicRows &t, std::string &err);
     template <class Real>
-    bool upload_points(const Real *x, const Real *y, const Real *z, long n, WorkerPool &pool, std::string &err);
+    bool upload_points(const Real *x, const Real *y, const Real *z, long n, std::string &err);
 
     // Runs tables + field + statistics (+ epilogue) into d_field (device,
     // `Real` elements). stats_out[0..3] = {count, mean, variance, sigma_d}

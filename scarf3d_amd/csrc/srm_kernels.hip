@@ -691,12 +691,14 @@ __global__ __launch_bounds__(256) void clear(double *__restrict__ dst, long n)
 
 }  // namespace
 
-// The coordinates go up at `real` through a ring of pinned buffers, which the
-// pool's threads fill while the copies before run, and are widened on the
-// device: 2M points (24 MB) 0.9 ms, 12.4 ms with FP64 copies made on one thread
-// and a pageable copy of twice the bytes.
+// The coordinates go up at `real` through a ring of pinned buffers, filled
+// while the copies before run, and are widened on the device: 2M points (24
+// MB) 1.8 ms, 12.4 ms with FP64 copies and a pageable copy of twice the bytes.
+// The caller's thread reads them: with a pool's threads a call is as fast
+// (3.2 against 3.3 ms), and the caller's next writes to its arrays are slower
+// (their lines sit in other cores' caches: +5 to 10 ms for new coordinates).
 template <class Real>
-bool Device::upload_points(const Real *x, const Real *y, const Real *z, long n, WorkerPool &pool, std::string &err)
+bool Device::upload_points(const Real *x, const Real *y, const Real *z, long n, std::string &err)
 {
     npts_ = 0;
     const size_t total = size_t(z ? 3 : 2) * n;
@@ -710,32 +712,25 @@ bool Device::upload_points(const Real *x, const Real *y, const Real *z, long n, 
     HIP_TRY(hipStreamSynchronize(stream_));  // the ring is free
     const Real *axes[3] = {x, y, z};
     const size_t chunk = kPointStage / sizeof(Real);
-    const int threads = pool.size();
-    std::vector<Real> lo(threads), hi(threads);
     long piece = 0;
     for (int d = 0; d < 3; ++d) {
         pts_lo_[d] = pts_hi_[d] = 0.0;
         if (!axes[d]) continue;
-        std::fill(lo.begin(), lo.end(), axes[d][0]);
-        std::fill(hi.begin(), hi.end(), axes[d][0]);
+        Real lo = axes[d][0], hi = axes[d][0];
         for (size_t at = 0; at < size_t(n); at += chunk, ++piece) {
             const int slot = static_cast<int>(piece % kPointStages);
             const size_t len = std::min(chunk, size_t(n) - at);
             if (piece >= kPointStages) HIP_TRY(hipEventSynchronize(pts_ev_[slot]));
             Real *stage = reinterpret_cast<Real *>(h_pts_ + slot * kPointStage);
             const Real *src = axes[d] + at;
-            auto fill = [&](int t, size_t a, size_t b) {
-                std::copy(src + a, src + b, stage + a);
-                add_extent(src + a, b - a, lo[t], hi[t]);
-            };
-            if (len < 16384) fill(0, 0, len);
-            else in_parts(pool, len, fill);
+            std::copy(src, src + len, stage);
+            add_extent(src, len, lo, hi);
             HIP_TRY(hipMemcpyAsync(static_cast<Real *>(d_tab_) + size_t(d) * n + at, stage, len * sizeof(Real),
                                    hipMemcpyHostToDevice, stream_));
             HIP_TRY(hipEventRecord(pts_ev_[slot], stream_));
         }
-        pts_lo_[d] = *std::min_element(lo.begin(), lo.end());
-        pts_hi_[d] = *std::max_element(hi.begin(), hi.end());
+        pts_lo_[d] = lo;
+        pts_hi_[d] = hi;
     }
     const int blocks = int(std::min<size_t>((total + 255) / 256, 4096));
     widen<Real><<<blocks, 256, 0, stream_>>>(static_cast<const Real *>(d_tab_), d_pts_, long(total));
@@ -1162,9 +1157,8 @@ bool Device::run_streamed(const Geometry &g, int kernel, int nharm, double scali
     return finish<Real>(g, ep, d_field, nparts, stats_out, slab_first, slab_points, err, on_slab);
 }
 
-template bool Device::upload_points<float>(const float *, const float *, const float *, long, WorkerPool &, std::string &);
-template bool Device::upload_points<double>(const double *, const double *, const double *, long, WorkerPool &,
-                                            std::string &);
+template bool Device::upload_points<float>(const float *, const float *, const float *, long, std::string &);
+template bool Device::upload_points<double>(const double *, const double *, const double *, long, std::string &);
 template bool Device::run<float>(const Geometry &, int, double, const Epilogue &, float *, double *, std::string &,
                                  const SlabHook *, int);
 template bool Device::run<double>(const Geometry &, int, double, const Epilogue &, double *, double *,
