@@ -39,6 +39,19 @@ __device__ __forceinline__ Cplx<Real> mul_i(Cplx<Real> a)  // i a
     return {-a.y, a.x};
 }
 
+// element `offset` of an array at a uniform address, counted in 32 bits: the
+// form that loads and stores take without address arithmetic
+template <class T>
+__device__ __forceinline__ const T &element(const T *p, unsigned offset)
+{
+    return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(p) + offset * unsigned(sizeof(T)));
+}
+template <class T>
+__device__ __forceinline__ T &element(T *p, unsigned offset)
+{
+    return *reinterpret_cast<T *>(reinterpret_cast<char *>(p) + offset * unsigned(sizeof(T)));
+}
+
 // a pass: radix | log2 of the span << 8
 __host__ __device__ constexpr int kind_of(int radix, int shift) { return radix | shift << 8; }
 
@@ -171,39 +184,63 @@ __device__ __forceinline__ void dft(Cplx<Real> (&x)[R])
     }
 }
 
+// A length's passes, for the device.
+struct Passes {
+    int n = 0, count = 0;
+    int kind[6] = {};
+    uint32_t magic[6] = {};  // 2^32 / (n / radix), rounded up: exact quotients for the counts of a block
+};
+
+// A barrier for LDS alone: loads from global memory stay in flight across it.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // One pass of radix R and span 2^S (S < 0: 2^shift, at least 16) over `lines`
-// lines of n elements. With the span known the positions of a butterfly are
-// one address and constant offsets. The twiddles come from a table of n
-// entries (one rounding each), not from products. store(line, index, value)
+// lines of n elements, behind a barrier. With the span known the positions of
+// a butterfly are one address and constant offsets, and a span up to 64
+// divides the block: every butterfly of a thread has the same twiddles, loaded
+// before the barrier. They come from a table (one rounding each), not from
+// products, in the order of the lanes: read at multiples of the butterfly's
+// number they cost a cache line per lane, which bound the pass (512^3 float,
+// y pass of 64 planes, 201 us; in order, 179 us). store(line, index, value)
 // receives the outputs of a last pass; otherwise they go back to their places.
 struct InPlace {};
 template <int R, int S, class Real, class Store>
-__device__ __forceinline__ void pass(Cplx<Real> *lds, const Cplx<Real> *__restrict__ tw, int n, int line_pitch,
-                                     int lines, int shift, int tid, int threads, const Store &store)
+__device__ __forceinline__ void pass(Cplx<Real> *lds, const Cplx<Real> *__restrict__ tw, int n, uint32_t magic,
+                                     int line_pitch, int lines, int shift, int tid, int threads, const Store &store)
 {
     using C = Cplx<Real>;
     if constexpr (S >= 0) shift = S;
     const int per = n / R;
-    const int tw_step = per >> shift;
     const int span = 1 << shift;
-    const uint32_t magic = static_cast<uint32_t>((0x100000000ull + per - 1) / per);  // exact for the counts here
-    for (int q = tid; q < lines * per; q += threads) {
+    const int total = lines * per;
+    auto off = [&](int r) {  // of element base + r * span
+        if constexpr (S >= 0 && S < 4) return (r << S) + ((r << S) >> 4);
+        else return r * (span + (span >> 4));
+    };
+    C t[R];
+    auto twiddles = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 1; r < R; ++r) t[r] = element(tw + (r << shift), unsigned(j));
+    };
+    if constexpr (S > 0) twiddles(tid & (span - 1));
+    lds_barrier();
+    for (int q = tid; q < total; q += threads) {
         const int line = per == 1 ? q : static_cast<int>(__umulhi(static_cast<uint32_t>(q), magic));
         const int b = q - line * per;
-        const int j = b & (span - 1);
-        const int base = ((b >> shift) * R << shift) + j;
+        const int base = ((b >> shift) * R << shift) + (b & (span - 1));
         C *p = lds + line * line_pitch + pad(base);
-        auto off = [&](int r) {  // of element base + r * span
-            if constexpr (S >= 0 && S < 4) return (r << S) + ((r << S) >> 4);
-            else return r * (span + (span >> 4));
-        };
         C x[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) x[r] = p[off(r)];
-        if (S != 0) {
-            const int step = j * tw_step;
+        if constexpr (S < 0) twiddles(base & (span - 1));
+        if constexpr (S != 0) {
 #pragma unroll
-            for (int r = 1; r < R; ++r) x[r] = mul(x[r], tw[r * step]);
+            for (int r = 1; r < R; ++r) x[r] = mul(x[r], t[r]);
         }
         dft<R>(x);
         if constexpr (std::is_same_v<Store, InPlace>) {
@@ -211,7 +248,10 @@ __device__ __forceinline__ void pass(Cplx<Real> *lds, const Cplx<Real> *__restri
             for (int r = 0; r < R; ++r) p[off(r)] = x[r];
         } else {
 #pragma unroll
-            for (int r = 0; r < R; ++r) store(line, base + (r << shift), x[r]);
+            for (int r = 0; r < R; ++r) {
+                if (r > 0 && r % 4 == 0) __builtin_amdgcn_sched_barrier(0);  // store's operands of 4 outputs at a time
+                store(line, base + (r << shift), x[r]);
+            }
         }
     }
 }
@@ -219,71 +259,97 @@ __device__ __forceinline__ void pass(Cplx<Real> *lds, const Cplx<Real> *__restri
 // The passes from `first` on; the last one's outputs go to store. A barrier
 // precedes every pass.
 template <class Real, class Store>
-__device__ __forceinline__ void transform(Cplx<Real> *lds, const Cplx<Real> *__restrict__ tw, int n, int first,
-                                          int passes, const int (&kind)[6], int line_pitch, int lines, int tid,
-                                          int threads, const Store &store)
+__device__ __forceinline__ void transform(Cplx<Real> *lds, const Cplx<Real> *__restrict__ tw, int first,
+                                          const Passes &plan, int line_pitch, int lines, int tid, int threads,
+                                          const Store &store)
 {
-    for (int p = first; p < passes; ++p) {
-        __syncthreads();
-        const int radix = kind[p] & 255, shift = kind[p] >> 8;
+    for (int p = first; p < plan.count; ++p) {
+        const int radix = plan.kind[p] & 255, shift = plan.kind[p] >> 8, n = plan.n;
+        const uint32_t magic = plan.magic[p];
+        asm volatile("" : "+v"(tid));  // keeps the addresses of all kinds of pass from being held over the loop
         auto go = [&](const auto &out) __attribute__((always_inline)) {
-            switch (kind[p]) {
-            case kind_of(4, 0): pass<4, 0>(lds, tw, n, line_pitch, lines, shift, tid, threads, out); break;
-            case kind_of(4, 2): pass<4, 2>(lds, tw, n, line_pitch, lines, shift, tid, threads, out); break;
-            case kind_of(8, 2): pass<8, 2>(lds, tw, n, line_pitch, lines, shift, tid, threads, out); break;
-            case kind_of(16, 2): pass<16, 2>(lds, tw, n, line_pitch, lines, shift, tid, threads, out); break;
-            case kind_of(8, 0): pass<8, 0>(lds, tw, n, line_pitch, lines, shift, tid, threads, out); break;
-            case kind_of(2, 3): pass<2, 3>(lds, tw, n, line_pitch, lines, shift, tid, threads, out); break;
-            case kind_of(4, 3): pass<4, 3>(lds, tw, n, line_pitch, lines, shift, tid, threads, out); break;
-            case kind_of(8, 3): pass<8, 3>(lds, tw, n, line_pitch, lines, shift, tid, threads, out); break;
-            case kind_of(16, 3): pass<16, 3>(lds, tw, n, line_pitch, lines, shift, tid, threads, out); break;
-            case kind_of(8, 6): pass<8, 6>(lds, tw, n, line_pitch, lines, shift, tid, threads, out); break;
-            case kind_of(16, 6): pass<16, 6>(lds, tw, n, line_pitch, lines, shift, tid, threads, out); break;
+            if constexpr (sizeof(Real) == 4) {
+                switch (plan.kind[p]) {
+                case kind_of(16, 2): pass<16, 2>(lds, tw, n, magic, line_pitch, lines, shift, tid, threads, out); return;
+                case kind_of(16, 3): pass<16, 3>(lds, tw, n, magic, line_pitch, lines, shift, tid, threads, out); return;
+                case kind_of(16, 6): pass<16, 6>(lds, tw, n, magic, line_pitch, lines, shift, tid, threads, out); return;
+                default: break;
+                }
+                if (radix == 16) {
+                    pass<16, -1>(lds, tw, n, magic, line_pitch, lines, shift, tid, threads, out);
+                    return;
+                }
+            }
+            switch (plan.kind[p]) {
+            case kind_of(4, 0): pass<4, 0>(lds, tw, n, magic, line_pitch, lines, shift, tid, threads, out); break;
+            case kind_of(4, 2): pass<4, 2>(lds, tw, n, magic, line_pitch, lines, shift, tid, threads, out); break;
+            case kind_of(8, 2): pass<8, 2>(lds, tw, n, magic, line_pitch, lines, shift, tid, threads, out); break;
+            case kind_of(8, 0): pass<8, 0>(lds, tw, n, magic, line_pitch, lines, shift, tid, threads, out); break;
+            case kind_of(2, 3): pass<2, 3>(lds, tw, n, magic, line_pitch, lines, shift, tid, threads, out); break;
+            case kind_of(4, 3): pass<4, 3>(lds, tw, n, magic, line_pitch, lines, shift, tid, threads, out); break;
+            case kind_of(8, 3): pass<8, 3>(lds, tw, n, magic, line_pitch, lines, shift, tid, threads, out); break;
+            case kind_of(8, 6): pass<8, 6>(lds, tw, n, magic, line_pitch, lines, shift, tid, threads, out); break;
             default:
                 switch (radix) {
-                case 3: pass<3, -1>(lds, tw, n, line_pitch, lines, shift, tid, threads, out); break;
-                case 4: pass<4, -1>(lds, tw, n, line_pitch, lines, shift, tid, threads, out); break;
-                case 5: pass<5, -1>(lds, tw, n, line_pitch, lines, shift, tid, threads, out); break;
-                case 7: pass<7, -1>(lds, tw, n, line_pitch, lines, shift, tid, threads, out); break;
-                case 8: pass<8, -1>(lds, tw, n, line_pitch, lines, shift, tid, threads, out); break;
-                case 9: pass<9, -1>(lds, tw, n, line_pitch, lines, shift, tid, threads, out); break;
-                default: pass<16, -1>(lds, tw, n, line_pitch, lines, shift, tid, threads, out); break;
+                case 3: pass<3, -1>(lds, tw, n, magic, line_pitch, lines, shift, tid, threads, out); break;
+                case 4: pass<4, -1>(lds, tw, n, magic, line_pitch, lines, shift, tid, threads, out); break;
+                case 5: pass<5, -1>(lds, tw, n, magic, line_pitch, lines, shift, tid, threads, out); break;
+                case 7: pass<7, -1>(lds, tw, n, magic, line_pitch, lines, shift, tid, threads, out); break;
+                case 8: pass<8, -1>(lds, tw, n, magic, line_pitch, lines, shift, tid, threads, out); break;
+                default: pass<9, -1>(lds, tw, n, magic, line_pitch, lines, shift, tid, threads, out); break;
                 }
             }
         };
-        if (p + 1 < passes) go(InPlace{});
+        if (p + 1 < plan.count) go(InPlace{});
         else go(store);
     }
 }
 
-// Radices of a length m * 2^a, `first` (4 or 8) first.
-__host__ inline int plan(int n, int first, int (&kind)[6])
+// Radices of a length m * 2^a, `first` (4 or 8) first. wide: none above 8 and
+// 9, since 16 FP64 values do not fit the registers.
+__host__ inline Passes plan(int length, int first, bool wide)
 {
-    int a = 0, passes = 0, shift = 0;
+    Passes p;
+    p.n = length;
+    int a = 0, shift = 0, n = length;
     while (n % 2 == 0) {
         n /= 2;
         ++a;
     }
-    auto add = [&](int log2_radix) {
-        kind[passes++] = kind_of(1 << log2_radix, shift);
+    auto add = [&](int radix, int log2_radix) {
+        const uint64_t per = length / radix;
+        p.magic[p.count] = static_cast<uint32_t>((0x100000000ull + per - 1) / per);
+        p.kind[p.count++] = kind_of(radix, shift);
         shift += log2_radix;
     };
-    add(first == 4 ? 2 : 3);
+    add(first, first == 4 ? 2 : 3);
     // the rest in 8s and 16s, and one 2 or 4 where it has to be
-    static const int logs[12][3] = {{}, {1}, {2}, {3}, {4}, {3, 2}, {3, 3}, {3, 4}, {4, 4}, {3, 3, 3}, {3, 3, 4},
-                                    {3, 4, 4}};
-    const int *rest = logs[a - shift];
-    for (int q = 0; q < 3 && rest[q] > 0; ++q) add(rest[q]);
-    if (n > 1) kind[passes++] = kind_of(n, shift);
-    return passes;
+    static const int narrow_logs[12][4] = {{}, {1}, {2}, {3}, {4}, {3, 2}, {3, 3}, {3, 4}, {4, 4}, {3, 3, 3}, {3, 3, 4},
+                                           {3, 4, 4}};
+    static const int wide_logs[12][4] = {{}, {1}, {2}, {3}, {2, 2}, {3, 2}, {3, 3}, {3, 2, 2}, {3, 3, 2}, {3, 3, 3},
+                                         {3, 3, 2, 2}, {3, 3, 3, 2}};
+    const int *rest = (wide ? wide_logs : narrow_logs)[a - shift];
+    for (int q = 0; q < 4 && rest[q] > 0; ++q) add(1 << rest[q], rest[q]);
+    if (n > 1) add(n, 0);
+    return p;
+}
+
+// Entry e of a plan's table of n twiddles: r j / (radix span) turns for
+// e = r span + j, j < span, 0 < r < radix: the passes' ranges follow each other.
+__device__ inline double turns(int e, const Passes &plan)
+{
+    int p = 0;
+    while (p + 1 < plan.count && (1 << (plan.kind[p + 1] >> 8)) <= e) ++p;
+    const int shift = plan.kind[p] >> 8, r = e >> shift, j = e & ((1 << shift) - 1);
+    return double(r * j) / double((plan.kind[p] & 255) << shift);
 }
 
 // position of natural index k before the first pass
-__host__ __device__ inline int digit_reverse(int k, int n, int passes, const int (&kind)[6])
+__host__ __device__ inline int digit_reverse(int k, const Passes &plan)
 {
-    int pos = 0;
-    for (int p = passes - 1; p >= 0; --p) {
-        const int radix = kind[p] & 255, q = k % radix;
+    int pos = 0, n = plan.n;
+    for (int p = plan.count - 1; p >= 0; --p) {
+        const int radix = plan.kind[p] & 255, q = k % radix;
         k /= radix;
         n /= radix;
         pos += q * n;

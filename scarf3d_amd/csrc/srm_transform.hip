@@ -17,7 +17,6 @@
 #include <cstdint>
 #include <type_traits>
 
-#include "fft_lds.hpp"
 #include "kaiser_bessel.hpp"
 #include "srm_stats.hpp"
 
@@ -30,6 +29,7 @@ constexpr double kInvTwoPi = 0.15915494309189533577;
 constexpr double kPiD = 3.14159265358979323846;
 constexpr int kThreads = 512;
 constexpr size_t kLineBytes = 64 << 10;  // lines of a block (unpadded): two blocks per CU
+constexpr size_t kMaxLds = 160 << 10;    // of a block alone
 constexpr double kMinOversampling = 1.9;
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
@@ -40,17 +40,18 @@ struct Args {
     int w, nx, ny, nz, m, l, columns, np_;
     int ox, oy, oz;
     double ds, beta_x, beta_y, scaling;
-    int px, rx[6], py, ry[6];
+    fft::Passes px, py;
     int zb, yb, nzb, slab, z0, zn;  // zn: planes of this round
     unsigned *key;           // class of the first ky << 14 | first column; ~0: amplitude 0
-    int *order, *start, *count;
-    int *first;              // first column, from here on in sorted order
-    double *tapx, *tapy;     // [np][w], [np][2 class widths] from the class' first ky on
+    int *order, *start;
+    int *last;               // last column that a harmonic touches
+    // in sorted order: [16][np], column c at c mod 16; [np][2 class widths] from the class' first ky on
+    double *tapx, *tapy;
     Cplx<Real> *twy, *twx, *twr;
     unsigned short *revy, *revx;
-    Real *decy;
-    double *decx;
-    Cplx<Real> *wave, *t;
+    double *decx, *decy;
+    bool pairs;              // the field takes aligned pairs
+    Cplx<Real> *wave, *t;    // wave: [slab / zb][np][zb]
 };
 
 // Classes of the first ky: a class' harmonics reach two class widths of ky
@@ -97,7 +98,7 @@ template <class Real>
 __global__ __launch_bounds__(256) void transform_keys(Args<Real> a, const double *__restrict__ harm)
 {
     const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n < a.columns) a.count[n] = 0;
+    if (n == 0) *a.last = 0;
     if (n >= a.np_) return;
     const Placed p = place(a, harm, n);
     const int col = min(max(p.kx + a.w / 2, 0), a.m), ky = p.ky < 0 ? p.ky + a.l : p.ky;
@@ -142,6 +143,7 @@ __global__ __launch_bounds__(1024) void transform_order(Args<Real> a)
     int running = 0;
     for (int q = 0; q < waves; ++q) running += wave_sum[q];
     int *start = a.start + long(cls) * (a.m + 2);
+    int top = 0;
     for (int b0 = 0; b0 < bins; b0 += threads) {
         const int bin = b0 + tid;
         int tot = 0;
@@ -168,10 +170,10 @@ __global__ __launch_bounds__(1024) void transform_order(Args<Real> a)
                 hist[q * bins + bin] = at;
                 at += h;
             }
-            if (tot > 0)
-                for (int c = bin; c < bin + a.w; ++c) a.count[c] = 1;  // every writer stores 1
+            if (tot > 0) top = bin + a.w - 1;
         }
     }
+    if (top > 0) atomicMax(a.last, top);
     if (tid == 0) start[bins] = running;
     __syncthreads();
     volatile int *place = mine;  // this wave's own row
@@ -196,12 +198,15 @@ __global__ __launch_bounds__(1024) void transform_order(Args<Real> a)
     }
 }
 
-// c_n(z) of plane z of a round, harmonics in sorted order: wave[p][z]. Phases
-// in FP64, about the centre of the block along x and y.
+// c_n(z) of the planes of a round, harmonics in sorted order: item e is plane
+// e % zb of group e / (zb present). Phases in FP64, about the centre of the
+// block along x and y.
 template <class Real>
-__device__ inline void wave_item(const Args<Real> &a, const double *__restrict__ harm, long e)
+__device__ inline void wave_item(const Args<Real> &a, const double *__restrict__ harm, long e, int present)
 {
-    const int p = int(e / a.slab), z = int(e - long(p) * a.slab), n = a.order[p];
+    const long pairs = e / a.zb;
+    const int group = int(pairs / present), p = int(pairs - long(group) * present), zz = int(e - pairs * a.zb);
+    const int z = group * a.zb + zz, n = a.order[p];
     const double wx = harm[n], wy = harm[a.np_ + n], wz = harm[2 * long(a.np_) + n];
     const double xc = double(a.ox + a.nx / 2) * a.ds, yc = double(a.oy + a.ny / 2) * a.ds;
     double t = (wz * (double(a.z0 + z + a.oz) * a.ds)) * kInvTwoPi +
@@ -212,7 +217,7 @@ __device__ inline void wave_item(const Args<Real> &a, const double *__restrict__
     double s, c;
     sincospi(tx < 0.0 ? -2.0 * t : 2.0 * t, &s, &c);
     const double amp = harm[4 * long(a.np_) + n];
-    a.wave[e] = Cplx<Real>{static_cast<Real>(amp * c), static_cast<Real>(amp * s)};
+    a.wave[(long(group) * a.np_ + p) * a.zb + zz] = Cplx<Real>{static_cast<Real>(amp * c), static_cast<Real>(amp * s)};
 }
 
 template <class Real>
@@ -221,55 +226,51 @@ __global__ __launch_bounds__(256) void transform_waves(Args<Real> a, const doubl
     const long present = a.start[long(a.l / kClass<Real> - 1) * (a.m + 2) + a.m + 1];
     const long total = present * a.slab;
     for (long e = blockIdx.x * long(blockDim.x) + threadIdx.x; e < total; e += long(gridDim.x) * blockDim.x)
-        wave_item(a, harm, e);
+        wave_item(a, harm, e, int(present));
 }
 
 // Tables of one realization in sorted order, and the waves of the first
-// round. Work items: waves; taps along y (the zeros around them included) and
-// x, one each; first columns; twiddles, digit-reversed positions and
-// deconvolution factors.
+// round. Work items: waves; taps along y and x, one each, the zeros around them
+// included; twiddles, digit-reversed positions and deconvolution factors.
 template <class Real>
 __global__ __launch_bounds__(256) void transform_tables(Args<Real> a, const double *__restrict__ harm)
 {
     constexpr int W = sizeof(Real) == 4 ? 9 : 16, K = sizeof(Real) == 4 ? 45 : 66, R = 2 * kClass<Real>;
     const long present = a.start[long(a.l / kClass<Real> - 1) * (a.m + 2) + a.m + 1];
-    const long i0 = present * a.slab, i1 = i0 + present * R, i2 = i1 + present * W, i3 = i2 + present;
-    const long total = i3 + a.l + 2 * long(a.m) + a.ny + a.nx;
+    const long i0 = present * a.slab, i1 = i0 + present * R, i2 = i1 + present * 16;
+    const long total = i2 + a.l + 2 * long(a.m) + a.ny + a.nx;
     for (long e = blockIdx.x * long(blockDim.x) + threadIdx.x; e < total; e += long(gridDim.x) * blockDim.x) {
         if (e < i0) {
-            wave_item(a, harm, e);
+            wave_item(a, harm, e, int(present));
             continue;
         }
         if (e < i2) {
             const bool along_y = e < i1;
-            const int p = int(along_y ? (e - i0) / R : (e - i1) / W);
+            const int p = int(along_y ? (e - i0) / R : (e - i1) % present);
             const Placed h = place(a, harm, a.order[p]);
             if (along_y) {
                 const int ky = h.ky < 0 ? h.ky + a.l : h.ky;
                 const int d = int((e - i0) % R) - ky % kClass<Real>;  // tap at the class' row
                 a.tapy[e - i0] = d >= 0 && d < W ? kaiser_bessel<K>(h.ky + d - h.gy, W, a.beta_y, exp(-a.beta_y)) : 0.0;
             } else {
-                a.tapx[e - i1] = kaiser_bessel<K>(h.kx + int((e - i1) % W) - h.gx, W, a.beta_x, exp(-a.beta_x));
+                const int slot = int((e - i1) / present), d = (slot - h.kx - a.w / 2) & 15;  // columns are kx + w/2
+                a.tapx[long(slot) * a.np_ + p] = d < W ? kaiser_bessel<K>(h.kx + d - h.gx, W, a.beta_x, exp(-a.beta_x)) : 0.0;
             }
             continue;
         }
-        if (e < i3) {
-            a.first[e - i2] = int(a.key[a.order[e - i2]] & 0x3fffu);
-            continue;
-        }
-        int r = int(e - i3);
+        int r = int(e - i2);
         double s, c;
         if (r < a.l) {
-            sincospi(2.0 * double(r) / a.l, &s, &c);
+            sincospi(2.0 * fft::turns(r, a.py), &s, &c);
             a.twy[r] = Cplx<Real>{Real(c), Real(s)};
-            a.revy[r] = static_cast<unsigned short>(fft::pad(fft::digit_reverse(r, a.l, a.py, a.ry)));
+            a.revy[r] = static_cast<unsigned short>(fft::pad(fft::digit_reverse(r, a.py)));
             continue;
         }
         r -= a.l;
         if (r < a.m) {
-            sincospi(2.0 * double(r) / a.m, &s, &c);
+            sincospi(2.0 * fft::turns(r, a.px), &s, &c);
             a.twx[r] = Cplx<Real>{Real(c), Real(s)};
-            a.revx[r] = static_cast<unsigned short>(fft::pad(fft::digit_reverse(r, a.m, a.px, a.rx)));
+            a.revx[r] = static_cast<unsigned short>(fft::pad(fft::digit_reverse(r, a.px)));
             continue;
         }
         r -= a.m;
@@ -279,20 +280,31 @@ __global__ __launch_bounds__(256) void transform_tables(Args<Real> a, const doub
             continue;
         }
         r -= a.m;
-        if (r < a.ny) a.decy[r] = static_cast<Real>(deconvolution(r - a.ny / 2, a.l, W, a.beta_y));
+        if (r < a.ny) a.decy[r] = deconvolution(r - a.ny / 2, a.l, W, a.beta_y);
         else if (r < a.ny + a.nx) a.decx[r - a.ny] = a.scaling * deconvolution(r - a.ny - a.nx / 2, 2 * a.m, W, a.beta_x);
     }
 }
 
-// LDS of the y pass behind the lines: partial sums of half the waves, the
+// LDS of the y pass behind the lines: partial sums of four waves, the
 // classes' ranges for the block's column and the digit-reversed positions.
-constexpr int kYWaves = kThreads / 64;
 template <class Real>
 size_t lds_y_bytes(int zb, int l)
 {
     const size_t classes = size_t(l) / kClass<Real>;
-    return size_t(zb) * fft::pitch(l) * sizeof(Cplx<Real>) + 16 + size_t(kYWaves / 2) * 256 * sizeof(double) +
-           classes * (sizeof(int2) + sizeof(unsigned short)) + size_t(l) * sizeof(unsigned short) + 16;
+    return size_t(zb) * fft::pitch(l) * sizeof(Cplx<Real>) + 16 + size_t(4) * 256 * sizeof(double) +
+           classes * sizeof(int2) + size_t(l) * sizeof(unsigned short) + 16;
+}
+
+// inclusive sum over the lanes up to each one
+__device__ inline int wave_scan(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // lane 15 of a row to the next one
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // lane 31 to the upper half
+    return v;
 }
 
 // Spread and y pass: one block per (kx column, zb planes). The spread is a
@@ -301,151 +313,248 @@ size_t lds_y_bytes(int zb, int l)
 // instruction,
 //   A[ky][p] = phi_y, B[p][z] = phi_x c_p(z),
 // so the sums are FP64 in a fixed order for either field type. A class reaches
-// the rows of the next one too: even classes, whose rows are disjoint, store
-// their tiles over the cleared lines, then the odd ones add theirs. One wave takes a class, and all
-// of them together one of kShared harmonics or more (most harmonics can sit in
-// a few columns and classes: at a small correlation length per box nearly all
-// do). Then the lines are transformed in LDS. Blocks of one z group follow
-// each other nzb apart: with nzb = 8 each XCD's L2 holds one group's waves.
-constexpr int kShared = 128;
-template <class Real>
-__global__ __launch_bounds__(kThreads, 4) void transform_y(Args<Real> a)
+// the rows of the next one too, and those are the upper half of its tiles:
+// after a class' last step the lower half is stored and the upper one becomes
+// the lower half of the next class' sums, with no exchange between lanes. A
+// wave takes a run of classes with its share of the column's steps, kAhead of
+// them in flight: most classes hold a few harmonics, and one class after the
+// other is a chain of waits (512^3 float x 20k, 64 planes: 203 us; classes in
+// flight but added to LDS by atomics, 298 us; so, 187 us, and 138 us with
+// 32-bit offsets, a scan without LDS and the deconvolution left to the x
+// pass). All waves together take a class of kShared steps and a sixteenth of
+// the column's or more (at a small correlation length per box nearly all
+// harmonics are in a few columns and classes); these columns are bound by the
+// matrix cores. Then the lines are transformed in LDS. Blocks of
+// one z group follow each other nzb apart: with nzb = 8 each XCD's L2 holds
+// one group's waves.
+constexpr int kShared = 32;
+constexpr int kAhead = 4;
+template <class Real, int Threads>
+__global__ __launch_bounds__(Threads, 4) void transform_y(Args<Real> a)
 {
-    constexpr int G = kTiles<Real>, CW = kClass<Real>, W = sizeof(Real) == 4 ? 9 : 16;
+    constexpr int G = kTiles<Real>, CW = kClass<Real>, W = sizeof(Real) == 4 ? 9 : 16, D = kAhead, kYWaves = Threads / 64;
     extern __shared__ __align__(16) unsigned char smem[];
     const int zblk = blockIdx.x % a.nzb, col = blockIdx.x / a.nzb;
-    if (!a.count[col]) return;  // the x pass takes this column as zero
+    const int zoff = zblk * a.zb, planes = min(a.zb, a.zn - zoff);
+    Cplx<Real> *out = a.t + (size_t(zoff) * a.columns + col) * a.ny;
+    const unsigned plane = unsigned(a.columns) * a.ny;
+    const Cplx<Real> zero{Real(0), Real(0)};
     const int line = fft::pitch(a.l), classes = a.l / CW;
     Cplx<Real> *lds = reinterpret_cast<Cplx<Real> *>(smem);
     Real *flat = reinterpret_cast<Real *>(smem);
     double *slots = reinterpret_cast<double *>(smem + (size_t(a.zb) * line * sizeof(Cplx<Real>) + 15) / 16 * 16);
-    int2 *range = reinterpret_cast<int2 *>(slots + (kYWaves / 2) * 256);
-    unsigned short *shared_cls = reinterpret_cast<unsigned short *>(range + classes);
-    unsigned short *rev = shared_cls + classes;
-    __shared__ int nshared;
+    int2 *range = reinterpret_cast<int2 *>(slots + 4 * 256);
+    unsigned short *rev = reinterpret_cast<unsigned short *>(range + classes);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int jj = lane & 15, slot = lane >> 4;
     const int lo = max(0, col - W + 1), hi = min(col, a.m);
-    const int zoff = zblk * a.zb;
     const bool mine = jj < 2 * a.zb;
-    const Real *wv = reinterpret_cast<const Real *>(a.wave) + 2 * zoff + (mine ? jj : 0);
-    if (tid == 0) nshared = 0;
-    __syncthreads();
-    for (int q = tid; q < classes; q += kThreads) {
+    for (int q = tid; q < classes; q += Threads) {
         const int *st = a.start + long(q) * (a.m + 2);
-        const int s0 = st[lo], n = st[hi + 1] - s0;
-        range[q] = make_int2(s0, n);
-        if (n >= kShared) shared_cls[atomicAdd(&nshared, 1)] = static_cast<unsigned short>(q);
+        const int s0 = st[lo];
+        range[q] = make_int2(s0, st[hi + 1] - s0);
     }
-    for (int q = tid; q < a.l; q += kThreads) rev[q] = a.revy[q];
-    const Cplx<Real> zero{Real(0), Real(0)};
-    for (int q = tid; q < a.zb * line; q += kThreads) lds[q] = zero;
+    for (int q = tid; q < a.l; q += Threads) rev[q] = a.revy[q];
+    for (int q = tid; q < a.zb * line; q += Threads) lds[q] = zero;
     __syncthreads();
-    // A and B of this lane's harmonic i of a range (beyond it: a zero)
-    auto load = [&](int s0, int n, int i, double &x, double &w, double (&y)[G]) __attribute__((always_inline)) {
-        const long p = s0 + min(i, n - 1);
-        x = a.tapx[p * W + (col - a.first[p])];
-        w = static_cast<double>(wv[2 * p * a.slab]);
-        x = i < n ? x : 0.0;
+    // A and B of this lane's harmonic of step i of a range, or of its last one:
+    // uniform bases and 32-bit offsets, which the loads take as they are
+    const double *tapx = a.tapx + long(col & 15) * a.np_;
+    const Cplx<Real> *waves = a.wave + long(zblk) * a.np_ * a.zb;
+    const unsigned wave_step = unsigned(a.zb * sizeof(Cplx<Real>));
+    const unsigned ylane = jj * sizeof(double), wlane = (mine ? jj : 0) * sizeof(Real);
+    auto load = [&](int s0, int n, int i, double &x, Real &w, double (&y)[G]) __attribute__((always_inline)) {
+        const unsigned k = static_cast<unsigned>(min(i + slot, n - 1));
+        const char *yv = reinterpret_cast<const char *>(a.tapy + long(s0) * (16 * G));
+        const char *wv = reinterpret_cast<const char *>(waves + long(s0) * a.zb);
+        x = fft::element(tapx + s0, k);
+        w = *reinterpret_cast<const Real *>(wv + (k * wave_step + wlane));
 #pragma unroll
-        for (int g = 0; g < G; ++g) y[g] = a.tapy[p * (16 * G) + 16 * g + jj];
+        for (int g = 0; g < G; ++g) y[g] = *reinterpret_cast<const double *>(yv + (k * (128u * G) + ylane) + 128 * g);
     };
-    // steps step, step + stride, ... of four harmonics each, added to acc; the
-    // loads of U steps are issued together
-    auto sum = [&](int s0, int n, int step, int stride, f64x4 (&acc)[G]) __attribute__((always_inline)) {
-        auto steps = [&](int i0, auto count) __attribute__((always_inline)) {
-            constexpr int U = decltype(count)::value;
-            double x[U], w[U], y[U][G];
+    // rem: harmonics from the step on; those beyond count as zeros
+    auto product = [&](int rem, double x, Real w, const double (&y)[G], f64x4 (&acc)[G]) __attribute__((always_inline)) {
+        const double b = slot < rem ? static_cast<double>(w) * x : 0.0;
 #pragma unroll
-            for (int u = 0; u < U; ++u) load(s0, n, i0 + 4 * u * stride + slot, x[u], w[u], y[u]);
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int g = 0; g < G; ++g)
-                    acc[g] = __builtin_amdgcn_mfma_f64_16x16x4f64(y[u][g], w[u] * x[u], acc[g], 0, 0, 0);
-        };
-        constexpr int U = 4;
-        int i0 = 4 * step;
-        for (; i0 + 4 * (U - 1) * stride < n; i0 += 4 * U * stride) steps(i0, std::integral_constant<int, U>{});
-        for (; i0 < n; i0 += 4 * stride) steps(i0, std::integral_constant<int, 1>{});
+        for (int g = 0; g < G; ++g) acc[g] = __builtin_amdgcn_mfma_f64_16x16x4f64(y[g], b, acc[g], 0, 0, 0);
     };
-    auto put = [&](int q, bool add, const f64x4 (&acc)[G]) __attribute__((always_inline)) {
+    auto clear = [](f64x4 (&acc)[G]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) acc[g] = f64x4{0.0, 0.0, 0.0, 0.0};
+    };
+    // rows 4 r + slot of class q, from the lane's sums v[r], stored or added
+    auto put = [&](int q, bool add, const double (&v)[CW / 4]) __attribute__((always_inline)) {
+        int at[CW / 4];
+#pragma unroll
+        for (int r = 0; r < CW / 4; ++r) {
+            const int ky = q * CW + 4 * r + slot;
+            at[r] = 2 * ((jj >> 1) * line + rev[ky >= a.l ? ky - a.l : ky]) + (jj & 1);
+        }
         if (!mine) return;
 #pragma unroll
-        for (int g = 0; g < G; ++g)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                int ky = q * CW + 16 * g + 4 * r + slot;
-                if (ky >= a.l) ky -= a.l;
-                Real &v = flat[2 * ((jj >> 1) * line + rev[ky]) + (jj & 1)];
-                v = static_cast<Real>(add ? static_cast<double>(v) + acc[g][r] : acc[g][r]);
-            }
+        for (int r = 0; r < CW / 4; ++r)
+            flat[at[r]] = static_cast<Real>(add ? static_cast<double>(flat[at[r]]) + v[r] : v[r]);
     };
-    const int heavy = nshared;
-    constexpr int B = 4 / G;
-    for (int odd = 0; odd < 2; ++odd) {
-        for (int q0 = 2 * wave + odd; q0 < classes; q0 += 2 * kYWaves * B) {
-            // B classes at a time: most hold a few harmonics, and their loads overlap
-            f64x4 acc[B][G];
-            int s0[B], n[B];
-            double x[B], w[B], y[B][G];
-#pragma unroll
-            for (int c = 0; c < B; ++c) {
-                const int q = q0 + 2 * kYWaves * c;
-                const int2 r = q < classes ? range[q] : make_int2(0, 0);
-                s0[c] = __builtin_amdgcn_readfirstlane(r.x);
-                n[c] = __builtin_amdgcn_readfirstlane(r.y);
-                if (n[c] >= kShared) n[c] = -1;
-                if (n[c] > 0) load(s0[c], n[c], slot, x[c], w[c], y[c]);
-            }
-#pragma unroll
-            for (int c = 0; c < B; ++c) {
-                const int q = q0 + 2 * kYWaves * c;
-                if (n[c] <= 0) continue;
-#pragma unroll
-                for (int g = 0; g < G; ++g)
-                    acc[c][g] = __builtin_amdgcn_mfma_f64_16x16x4f64(y[c][g], w[c] * x[c], f64x4{0.0, 0.0, 0.0, 0.0},
-                                                                     0, 0, 0);
-                sum(s0[c], n[c], 1, 1, acc[c]);
-                put(q, odd, acc[c]);
-            }
+    // the halves of a class' tiles
+    auto put_lower = [&](int q, bool add, const f64x4 (&acc)[G]) __attribute__((always_inline)) {
+        if constexpr (G == 1) put(q, add, {acc[0][0], acc[0][1]});
+        else put(q, add, {acc[0][0], acc[0][1], acc[0][2], acc[0][3]});
+    };
+    auto move_down = [&](f64x4 (&acc)[G]) __attribute__((always_inline)) {
+        if constexpr (G == 1) acc[0] = f64x4{acc[0][2], acc[0][3], 0.0, 0.0};
+        else {
+            acc[0] = acc[G - 1];
+            acc[G - 1] = f64x4{0.0, 0.0, 0.0, 0.0};
         }
-        for (int h = 0; h < heavy; ++h) {
-            const int q = __builtin_amdgcn_readfirstlane(shared_cls[h]);
-            if ((q & 1) != odd) continue;
-            const int s0 = __builtin_amdgcn_readfirstlane(range[q].x), n = __builtin_amdgcn_readfirstlane(range[q].y);
-            f64x4 acc[G];
-#pragma unroll
-            for (int g = 0; g < G; ++g) acc[g] = f64x4{0.0, 0.0, 0.0, 0.0};
-            sum(s0, n, wave, kYWaves, acc);
-            for (int half = kYWaves / 2; half >= 1; half /= 2)
-#pragma unroll
-                for (int g = 0; g < G; ++g) {
-                    __syncthreads();
-                    if (wave >= half && wave < 2 * half) {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) slots[(wave - half) * 256 + 64 * r + lane] = acc[g][r];
-                    }
-                    __syncthreads();
-                    if (wave < half) {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) acc[g][r] += slots[wave * 256 + 64 * r + lane];
-                    }
-                }
-            if (wave == 0) put(q, odd, acc);
-        }
-        __syncthreads();
+    };
+    // steps of classes base .. base + 63, one per lane
+    auto steps = [&](int base, int2 &r) __attribute__((always_inline)) {
+        r = base + lane < classes ? range[base + lane] : make_int2(0, 0);
+        return (r.y + 3) >> 2;
+    };
+    int total = 0, light = 0, before = 0;
+    for (int base = 0; base < classes; base += 64) {
+        int2 r;
+        total += __builtin_amdgcn_readlane(wave_scan(steps(base, r)), 63);
     }
-    // the last pass' outputs leave the block: the ny kept ones, divided by phi^
-    const int planes = min(a.zb, a.zn - zoff);
-    Cplx<Real> *out = a.t + (size_t(zoff) * a.columns + col) * a.ny;
-    const size_t plane = size_t(a.columns) * a.ny;
-    fft::transform(lds, a.twy, a.l, 0, a.py, a.ry, line, a.zb, tid, kThreads,
+    if (total == 0) {  // no harmonic touches the column: zeros, of which the x pass reads those of the next one too
+        if (col <= *a.last + 1)
+            for (int z = 0; z < planes; ++z)
+                for (int y = tid; y < a.ny; y += Threads) fft::element(out, unsigned(z) * plane + y) = zero;
+        return;
+    }
+    const int limit = max(kShared, total / 16);
+    for (int base = 0; base < classes; base += 64) {
+        int2 r;
+        const int own = steps(base, r);
+        light += __builtin_amdgcn_readlane(wave_scan(own <= limit ? own : 0), 63);
+    }
+    const int first = light * wave / kYWaves, last = light * (wave + 1) / kYWaves;
+    f64x4 acc[G];
+    clear(acc);
+    int cur = -1;  // the class whose rows the lower half of acc belongs to
+    for (int base = 0; base < classes; base += 64) {
+        int2 r;
+        int own = steps(base, r);
+        own = own <= limit ? own : 0;
+        const int upto = wave_scan(own), at = before + upto - own;
+        uint64_t left = __ballot(own > 0 && at >= first && at < last);
+        before += __builtin_amdgcn_readlane(upto, 63);
+        if (left == 0) continue;
+        int s0 = 0, n = 0, i = 0, q = 0;  // the next step: harmonics i .. i + 3 of class q
+        double x[D], y[D][G];
+        Real w[D];
+        int rem[D], cls[D];
+        auto issue = [&](int u) __attribute__((always_inline)) {
+            if (i >= n && left) {
+                const int k = __ffsll(static_cast<unsigned long long>(left)) - 1;
+                left &= left - 1;
+                s0 = __builtin_amdgcn_readlane(r.x, k);
+                n = __builtin_amdgcn_readlane(r.y, k);
+                q = base + k;
+                i = 0;
+            }
+            rem[u] = n - i;  // none left: 0 or less
+            cls[u] = q;
+            load(s0, n, i, x[u], w[u], y[u]);
+            i += 4;
+        };
+#pragma unroll
+        for (int u = 0; u < D; ++u) issue(u);
+        while (rem[0] > 0) {
+#pragma unroll
+            for (int u = 0; u < D; ++u) {
+                const int rest = rem[u], c = cls[u];
+                if (rest <= 0) break;
+                if (c != cur) {  // not the class after the last one
+                    if (cur >= 0) put_lower(cur, false, acc);
+                    clear(acc);
+                    cur = c;
+                }
+                product(rest, x[u], w[u], y[u], acc);
+                issue(u);
+                if (rest <= 4) {
+                    put_lower(c, false, acc);
+                    move_down(acc);
+                    cur = c + 1;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    if (cur >= 0) put_lower(cur, true, acc);  // another wave's class, or an empty one
+    if (light < total) {
+        int base = -64, s0 = 0, n = 0, q = 0;
+        uint64_t left = 0;
+        auto next = [&]() __attribute__((always_inline)) {
+            while (left == 0) {
+                base += 64;
+                if (base >= classes) return false;
+                int2 r;
+                left = __ballot(steps(base, r) > limit);
+            }
+            q = base + __ffsll(static_cast<unsigned long long>(left)) - 1;
+            left &= left - 1;
+            s0 = __builtin_amdgcn_readfirstlane(range[q].x);
+            n = __builtin_amdgcn_readfirstlane(range[q].y);
+            return true;
+        };
+        constexpr int U = kAhead;
+        double x[U], y[U][G];
+        Real w[U];
+        auto issue = [&](int i0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) load(s0, n, i0 + 4 * u * kYWaves, x[u], w[u], y[u]);
+        };
+        bool more = next();
+        issue(4 * wave);
+        while (more) {
+            clear(acc);
+            for (int i0 = 4 * wave; i0 < n;) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) product(n - i0 - 4 * u * kYWaves, x[u], w[u], y[u], acc);
+                i0 += 4 * U * kYWaves;
+                if (i0 < n) issue(i0);
+            }
+            const int c = q;
+            more = next();
+            if (more) issue(4 * wave);  // in flight over the reduction
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                double *mine_of = slots + (wave & 3) * 256 + lane;
+                for (int four = 4; four < kYWaves; four += 4) {
+                    fft::lds_barrier();
+                    if (wave >= four && wave < four + 4)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) mine_of[64 * r] = acc[g][r];
+                    fft::lds_barrier();
+                    if (wave < 4)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) acc[g][r] += mine_of[64 * r];
+                }
+                fft::lds_barrier();
+                if (wave >= 1 && wave < 4)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) mine_of[64 * r] = acc[g][r];
+                fft::lds_barrier();
+                if (wave == 0)
+#pragma unroll
+                    for (int v = 1; v < 4; ++v)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) acc[g][r] += slots[256 * v + 64 * r + lane];
+            }
+            if (wave == 0) {
+                put_lower(c, true, acc);
+                move_down(acc);
+                put_lower(c + 1, true, acc);
+            }
+        }
+    }
+    // the ny kept outputs of the last pass leave the block
+    fft::transform(lds, a.twy, 0, a.py, line, a.zb, tid, Threads,
                    [&](int z, int q, Cplx<Real> v) __attribute__((always_inline)) {
-                       const int y = (2 * q < a.l ? q : q - a.l) + a.ny / 2;
-                       if (z >= planes || y < 0 || y >= a.ny) return;
-                       const Real d = a.decy[y];
-                       out[z * plane + y] = Cplx<Real>{v.x * d, v.y * d};
+                       const unsigned y = (2 * q < a.l ? q : q - a.l) + a.ny / 2;
+                       if (z < planes && y < unsigned(a.ny)) fft::element(out, unsigned(z) * plane + y) = v;
                    });
 }
 
@@ -456,8 +565,10 @@ __global__ __launch_bounds__(kThreads, 4) void transform_y(Args<Real> a)
 // An item is the first butterflies, of radix R = kFirstX, of inputs b + r m/R
 // and m/R - b + r m/R, which hold each other's partners (butterflies 0 and
 // m/2R hold their own): T comes straight into registers, and the last pass
-// stores the field from registers, scaled and rounded, with the statistics
-// partials.
+// stores the field from registers, divided by phi^ of both axes, scaled and
+// rounded, with the statistics partials. 512^3 float, 64 planes: 90 us (147
+// with T through LDS; 110 with a check of every column, single stores and
+// twiddles out of the lanes' order), of which the 200 MB moved take 43.
 template <class Real>
 __global__ __launch_bounds__(kThreads, 4) void transform_x(Args<Real> a, Real *__restrict__ field,
                                                                              double *__restrict__ part)
@@ -471,13 +582,14 @@ __global__ __launch_bounds__(kThreads, 4) void transform_x(Args<Real> a, Real *_
     const int lines = min(a.yb, a.ny - y0);
     const C *t = a.t + size_t(z) * a.columns * a.ny + y0;
     const int off = a.w / 2, above = a.w - 1 - a.w / 2;  // columns below 0 and above m
+    const int zeros = *a.last + 1;  // the first column of zeros only
     constexpr int R = kFirstX<Real>;
     const int step = a.m / R;
     for (int e = tid; e < (step / 2) * a.yb; e += kThreads) {
         const int yy = e & (a.yb - 1), b = e / a.yb;
         if (yy >= lines) continue;
         auto at = [&](int kx) __attribute__((always_inline)) {
-            return a.count[kx + off] ? t[size_t(kx + off) * a.ny + yy] : C{Real(0), Real(0)};
+            return fft::element(t, unsigned(min(kx + off, zeros)) * unsigned(a.ny) + yy);
         };
         C p[R], q[R], pm{};
         const int bp = b, bq = b == 0 ? step / 2 : step - b;
@@ -487,21 +599,23 @@ __global__ __launch_bounds__(kThreads, 4) void transform_x(Args<Real> a, Real *_
             q[r] = at(bq + r * step);
         }
         if (b == 0) pm = at(a.m);
-        // columns outside 0 .. m fold onto their conjugates
-        auto fold = [&](C &v, int kx) __attribute__((always_inline)) {
-            if (kx > 0 && kx <= off) {
-                const C u = at(-kx);
-                v = C{v.x + u.x, v.y - u.y};
-            }
-            if (a.m - kx <= above) {
-                const C u = at(2 * a.m - kx);
-                v = C{v.x + u.x, v.y - u.y};
-            }
-        };
+        // columns outside 0 .. m fold onto their conjugates: first and last few
+        if (b <= a.w || step <= 2 * a.w) {
+            auto fold = [&](C &v, int kx) __attribute__((always_inline)) {
+                if (kx > 0 && kx <= off) {
+                    const C u = at(-kx);
+                    v = C{v.x + u.x, v.y - u.y};
+                }
+                if (a.m - kx <= above) {
+                    const C u = at(2 * a.m - kx);
+                    v = C{v.x + u.x, v.y - u.y};
+                }
+            };
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            fold(p[r], bp + r * step);
-            fold(q[r], bq + r * step);
+            for (int r = 0; r < R; ++r) {
+                fold(p[r], bp + r * step);
+                fold(q[r], bq + r * step);
+            }
         }
         auto pair = [&](C &u, C &v, int k) __attribute__((always_inline)) {  // u = H_k, v = H_(m-k)
             const Real h = Real(0.5);
@@ -534,22 +648,38 @@ __global__ __launch_bounds__(kThreads, 4) void transform_x(Args<Real> a, Real *_
     double s1 = 0.0, s2 = 0.0, pivot = 0.0;
     int cnt = 0;
     Real *rows = field + (size_t(a.z0 + z) * a.ny + y0) * a.nx;
-    fft::transform(lds, a.twx, a.m, 1, a.px, a.rx, line, a.yb, tid, kThreads,
+    const double *decy = a.decy + y0;
+    auto add = [&](double o) __attribute__((always_inline)) {
+        const double d = o - pivot;
+        s1 += d;
+        s2 = fma(d, d, s2);
+    };
+    fft::transform(lds, a.twx, 1, a.px, line, lines, tid, kThreads,
                    [&](int yy, int q, C v) __attribute__((always_inline)) {
-                       if (yy >= lines) return;
                        const int i = 2 * (2 * q < a.m ? q : q - a.m) + a.nx / 2;
-                       const Real c[2] = {v.x, v.y};
-#pragma unroll
-                       for (int h = 0; h < 2; ++h) {
-                           if (i + h < 0 || i + h >= a.nx) continue;
-                           const Real o = static_cast<Real>(static_cast<double>(c[h]) * a.decx[i + h]);
-                           rows[size_t(yy) * a.nx + i + h] = o;
-                           if (cnt == 0) pivot = static_cast<double>(o);
-                           const double d = static_cast<double>(o) - pivot;
-                           s1 += d;
-                           s2 = fma(d, d, s2);
-                           ++cnt;
+                       if (i < -1 || i >= a.nx) return;
+                       const double dy = decy[yy];
+                       Real *o = &fft::element(rows, unsigned(yy * a.nx + max(i, 0)));
+                       const bool first = i >= 0, second = i + 1 < a.nx;
+                       const C c{static_cast<Real>(static_cast<double>(v.x) * (dy * a.decx[max(i, 0)])),
+                                 static_cast<Real>(static_cast<double>(v.y) * (dy * a.decx[min(i + 1, a.nx - 1)]))};
+                       if (cnt == 0) pivot = static_cast<double>(first ? c.x : c.y);
+                       if (a.pairs) {
+                           *reinterpret_cast<C *>(o) = c;
+                           add(c.x);
+                           add(c.y);
+                           cnt += 2;
+                           return;
                        }
+                       if (first) {
+                           o[0] = c.x;
+                           add(c.x);
+                       }
+                       if (second) {
+                           o[int(first)] = c.y;
+                           add(c.y);
+                       }
+                       cnt += int(first) + int(second);
                    });
     Moments mo{double(cnt), 0.0, 0.0};
     if (cnt > 0) {
@@ -581,14 +711,6 @@ int good_length(double n)
     return best;
 }
 
-FftPlan fft_plan(int n, int first)
-{
-    FftPlan p;
-    p.n = n;
-    p.passes = fft::plan(n, first, p.kind);
-    return p;
-}
-
 }  // namespace
 
 bool transform_plan(const Geometry &g, int np_, bool f64, TransformPlan &plan)
@@ -607,13 +729,20 @@ bool transform_plan(const Geometry &g, int np_, bool f64, TransformPlan &plan)
     p.l = good_length(kMinOversampling * g.ny);
     if (p.l * csize > kLineBytes || p.m * csize > kLineBytes) return false;
     p.columns = p.m + p.w;
-    p.fx = fft_plan(p.m, f64 ? kFirstX<double> : kFirstX<float>);
-    p.fy = fft_plan(p.l, 8);
+    p.fx = fft::plan(p.m, f64 ? kFirstX<double> : kFirstX<float>, f64);
+    p.fy = fft::plan(p.l, 8, f64);
     // Kaiser-Bessel shape for the axis' oversampling s (pi w (1 - 1/(2 s)), just inside)
     p.beta_x = 0.995 * kPiD * p.w * (1.0 - 0.5 * g.nx / fx);
     p.beta_y = 0.995 * kPiD * p.w * (1.0 - 0.5 * g.ny / p.l);
     p.zb = 8;
     while (p.zb > 1 && size_t(p.zb) * p.l * csize > kLineBytes) p.zb /= 2;
+    // lines of which half a CU's LDS takes fewer planes than a matrix tile has:
+    // a block of twice the threads with the CU to itself (1024^2 x 512 x 50k,
+    // field: 12.1 -> 8.5 ms, and 6.6 -> 5.1 at longer correlation lengths)
+    if (p.zb < 8 && g.nz > p.zb && (f64 ? lds_y_bytes<double>(2 * p.zb, p.l) : lds_y_bytes<float>(2 * p.zb, p.l)) <= kMaxLds) {
+        p.zb *= 2;
+        p.wide = true;
+    }
     while (p.zb > 1 && p.zb / 2 >= g.nz) p.zb /= 2;
     p.yb = 16;
     while (p.yb > 1 && size_t(p.yb) * p.m * csize > kLineBytes) p.yb /= 2;
@@ -640,34 +769,34 @@ bool transform_plan(const Geometry &g, int np_, bool f64, TransformPlan &plan)
     const size_t np = np_;
     const int cls = f64 ? kClass<double> : kClass<float>;
     p.o_key = take(np * sizeof(unsigned));
-    p.o_first = take(np * sizeof(int));
     p.o_order = take(np * sizeof(int));
     p.o_start = take(size_t(p.l / cls) * (p.m + 2) * sizeof(int));
-    p.o_count = take(size_t(p.columns) * sizeof(int));
-    p.o_taps = take(np * (2 * cls + p.w) * sizeof(double));
+    p.o_last = take(sizeof(int));
+    p.o_taps = take(np * (2 * cls + 16) * sizeof(double));
     p.o_tw = take((size_t(p.l) + 2 * size_t(p.m)) * csize);
     p.o_rev = take((size_t(p.l) + p.m) * sizeof(unsigned short));
     p.o_dec = take((size_t(p.ny) + p.nx) * sizeof(double));
     p.o_wave = take(np * p.slab * csize);
     p.o_t = take(plane * p.slab);
     p.bytes = at;
-    return true;
+    // the y pass counts bytes from a class' first harmonic on in 32 bits
+    return np * size_t(2 * cls) * sizeof(double) < (size_t(1) << 32);
 }
 
-// Linear fits to measured times. Transform: the chain of small launches, the
-// harmonics' tables and ordering, the cells of both passes (float 512^3: 2.7
-// of 2.9 ms), their blocks, and the spread. The line between the two lies at
-// a few hundred harmonics for FP32 grids (float, direct_f32: 64^3 x 256 0.065
-// against 0.103 ms, x 64 0.058 against 0.045; bf16x3: 256^3 x 1024 0.36 against
-// 0.36, x 4096 0.43 against 1.27) and below 64 for FP64 ones (64^3 x 64 0.069
-// against 0.131 ms).
+// Linear fits to measured times, from above. Transform: the chain of small
+// launches, the harmonics' tables and ordering, the cells of both passes, their
+// blocks, and the spread. The line between the two lies at a few hundred
+// harmonics for FP32 grids (float, direct_f32: 64^3 x 256 0.060 against 0.103
+// ms, x 64 0.058 against 0.045; bf16x3: 128^3 x 1024 0.10 against 0.12, 256^3 x
+// 4096 0.33 against 1.27) and below 64 for FP64 ones (64^3 x 64 0.062 against
+// 0.131 ms).
 double transform_ms(const TransformPlan &p, bool f64)
 {
     const double cells = double(p.columns) * p.l * p.nz;
     const double blocks = double(p.columns) * ((p.nz + p.zb - 1) / p.zb) + p.nparts;
     const double waves = double(p.np_) * p.nz;
-    return f64 ? 0.05 + 1.2e-5 * p.np_ + 1.6e-8 * cells + 1.5e-5 * blocks + 8e-8 * waves
-               : 0.05 + 8.5e-6 * p.np_ + 7.5e-9 * cells + 1.2e-5 * blocks + 3e-8 * waves;
+    return f64 ? 0.055 + 1.05e-5 * p.np_ + 8e-9 * cells + 1e-5 * blocks + 4e-8 * waves
+               : 0.053 + 7e-6 * p.np_ + 5e-9 * cells + 1.1e-5 * blocks + 2e-8 * waves;
 }
 
 // The direct kernels' points and harmonics per millisecond, and for those with
@@ -706,20 +835,15 @@ bool transform_field(const TransformPlan &p, const Geometry &g, const double *d_
     a.beta_x = p.beta_x;
     a.beta_y = p.beta_y;
     a.scaling = scaling;
-    a.px = p.fx.passes;
-    a.py = p.fy.passes;
-    for (int q = 0; q < 6; ++q) {
-        a.rx[q] = p.fx.kind[q];
-        a.ry[q] = p.fy.kind[q];
-    }
+    a.px = p.fx;
+    a.py = p.fy;
     a.zb = p.zb;
     a.yb = p.yb;
     a.slab = p.slab;
     a.key = reinterpret_cast<unsigned *>(base + p.o_key);
-    a.first = reinterpret_cast<int *>(base + p.o_first);
     a.order = reinterpret_cast<int *>(base + p.o_order);
     a.start = reinterpret_cast<int *>(base + p.o_start);
-    a.count = reinterpret_cast<int *>(base + p.o_count);
+    a.last = reinterpret_cast<int *>(base + p.o_last);
     a.tapy = reinterpret_cast<double *>(base + p.o_taps);
     a.tapx = a.tapy + size_t(p.np_) * 2 * kClass<Real>;
     a.twy = reinterpret_cast<Cplx<Real> *>(base + p.o_tw);
@@ -728,18 +852,20 @@ bool transform_field(const TransformPlan &p, const Geometry &g, const double *d_
     a.revy = reinterpret_cast<unsigned short *>(base + p.o_rev);
     a.revx = a.revy + p.l;
     a.decx = reinterpret_cast<double *>(base + p.o_dec);
-    a.decy = reinterpret_cast<Real *>(a.decx + p.nx);
+    a.decy = a.decx + p.nx;
+    // a row's outputs 2 q + nx / 2 and the next one are then an aligned pair
+    a.pairs = p.nx % 4 == 0 && reinterpret_cast<uintptr_t>(d_field) % (2 * sizeof(Real)) == 0;
     a.wave = reinterpret_cast<Cplx<Real> *>(base + p.o_wave);
     a.t = reinterpret_cast<Cplx<Real> *>(base + p.o_t);
 
-    transform_keys<Real><<<(std::max(p.np_, p.columns) + 255) / 256, 256, 0, stream>>>(a, d_harm);
+    transform_keys<Real><<<(p.np_ + 255) / 256, 256, 0, stream>>>(a, d_harm);
     if (!ok(hipGetLastError(), "transform_keys")) return false;
     int sort_waves = 16;  // as many as their histograms fit in LDS
     while (size_t(sort_waves) * (p.m + 1) * sizeof(int) > (size_t(80) << 10)) sort_waves /= 2;
     transform_order<Real><<<p.l / kClass<Real>, 64 * sort_waves, size_t(sort_waves) * (p.m + 1) * sizeof(int), stream>>>(a);
     if (!ok(hipGetLastError(), "transform_order")) return false;
     a.zn = std::min(p.slab, p.nz);
-    const long items = long(p.np_) * (p.slab + 2 * kClass<Real> + p.w + 1) + p.l + 2 * long(p.m) + p.ny + p.nx;
+    const long items = long(p.np_) * (p.slab + 2 * kClass<Real> + 16) + p.l + 2 * long(p.m) + p.ny + p.nx;
     transform_tables<Real><<<int(std::min<long>((items + 255) / 256, 65536)), 256, 0, stream>>>(a, d_harm);
     if (!ok(hipGetLastError(), "transform_tables")) return false;
     if (!ok(hipEventRecord(tables_done, stream), "hipEventRecord")) return false;
@@ -755,7 +881,8 @@ bool transform_field(const TransformPlan &p, const Geometry &g, const double *d_
             transform_waves<Real><<<int(std::min<long>((waves + 255) / 256, 65536)), 256, 0, stream>>>(a, d_harm);
             if (!ok(hipGetLastError(), "transform_waves")) return false;
         }
-        transform_y<Real><<<a.nzb * p.columns, kThreads, lds_y, stream>>>(a);
+        if (p.wide) transform_y<Real, 1024><<<a.nzb * p.columns, 1024, lds_y, stream>>>(a);
+        else transform_y<Real, 512><<<a.nzb * p.columns, 512, lds_y, stream>>>(a);
         if (!ok(hipGetLastError(), "transform_y")) return false;
         transform_x<Real><<<a.zn * yblks, kThreads, lds_x, stream>>>(a, d_field, d_part);
         if (!ok(hipGetLastError(), "transform_x")) return false;

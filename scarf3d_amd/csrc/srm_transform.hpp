@@ -12,8 +12,8 @@
 // GEMM take one operation or more per point and harmonic. z stays a direct
 // sum: planes are independent, and a plane's values depend on its own z only.
 //
-// Measured, tables + field + statistics: float 512^3 x 20k 2.9 ms (mfma_bf16x3
-// 47.6, direct_f32 270), 128^3 x 5k 0.15 ms (0.44, 1.7); double 128^3 x 5k
+// Measured, tables + field + statistics: float 512^3 x 20k 2.0 ms (mfma_bf16x3
+// 47.6, direct_f32 270), 128^3 x 5k 0.13 ms (0.44, 1.7); double 128^3 x 5k
 // 0.20 ms (direct_f64 13.9). 2-norm error against the FP64 sum 1.4e-7 (4e-7,
 // 2.5e-7) in float and 8e-15 in double.
 #pragma once
@@ -21,16 +21,10 @@
 
 #include <string>
 
+#include "fft_lds.hpp"
 #include "srm_device.hpp"
 
 namespace scarf {
-
-// Passes of an in-place transform of length n (fft_lds.hpp).
-struct FftPlan {
-    int n = 0;
-    int passes = 0;
-    int kind[6] = {};
-};
 
 struct TransformPlan {
     int w = 0;             // kernel taps per axis
@@ -38,16 +32,17 @@ struct TransformPlan {
     int m = 0;             // x: half the oversampled length
     int l = 0;             // y: oversampled length, a multiple of 16
     int columns = 0;       // kept kx columns, -w/2 .. m + w - 1 - w/2
-    FftPlan fx, fy;        // lengths m (complex, for 2m reals) and l
+    fft::Passes fx, fy;    // lengths m (complex, for 2m reals) and l
     double beta_x = 0, beta_y = 0;
     int zb = 0, yb = 0;    // z planes per block of the y pass, y lines per block of the x pass
+    bool wide = false;     // y pass: one block of 1024 threads per CU
     int slab = 0;          // z planes per round of both passes
     int np_ = 0;           // padded harmonic count
     int nparts = 0;        // statistics partials, one per block of the x pass
     int groups = 0;        // their merged groups
     size_t bytes = 0;      // workspace
     // workspace offsets
-    size_t o_key = 0, o_first = 0, o_order = 0, o_start = 0, o_count = 0, o_taps = 0, o_tw = 0, o_rev = 0, o_dec = 0,
+    size_t o_key = 0, o_order = 0, o_start = 0, o_last = 0, o_taps = 0, o_tw = 0, o_rev = 0, o_dec = 0,
            o_wave = 0, o_t = 0;
 };
 

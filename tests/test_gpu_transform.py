@@ -221,3 +221,37 @@ def test_ensemble_of_few_harmonics_is_grouped(lib_f):
     b_ = lib_f.ensemble_execute(members, [b.ptr for b in bufs], "mfma_bf16x3")
     assert np.array_equal(a[:, :4], b_[:, :4])
     assert all(np.array_equal(f, b.numpy()) for f, b in zip(fields, bufs))
+
+
+WIDE = [(dict(n=(60, 1000, 13), cl=(120.0, 900.0, 40.0)), "fd"), (dict(n=(35, 2100, 9), cl=(100.0, 1500.0, 30.0)), "f"),
+        (dict(n=(41, 500, 9), cl=(100.0, 500.0, 30.0)), "d"), (dict(n=(33, 1100, 5), cl=(100.0, 900.0, 20.0)), "d"),
+        (dict(n=(60, 1000, 13), cl=(190.0, 3000.0, 40.0), acf=1, nharm=20000), "f"),
+        (dict(n=(60, 500, 13), cl=(190.0, 1500.0, 40.0), acf=1, nharm=20000), "d")]
+
+
+@pytest.mark.parametrize("kw,flavour", [(kw, f) for kw, fs in WIDE for f in fs])
+def test_long_lines_with_the_unit_to_themselves(request, kw, flavour):
+    """Lines of which eight planes fill more than half of a compute unit's LDS:
+    one block of 1024 threads each; also with most harmonics in few classes."""
+    lib = request.getfixturevalue("lib_" + flavour)
+    _check(lib, structured_cfg(ds=10.0, real=lib.dtype, **{"hurst": 0.25, "nharm": 3001, **kw}), 7)
+
+
+@pytest.mark.parametrize("nx", [64, 66, 67])
+@pytest.mark.parametrize("flavour", ["f", "d"])
+def test_fields_at_any_alignment(request, flavour, nx):
+    """Values are stored in pairs where rows and field allow it: the same bits
+    one value off, where they do not."""
+    lib = request.getfixturevalue("lib_" + flavour)
+    hip = Hip()
+    init_library(lib, structured_cfg(n=(nx, 50, 20), ds=10.0, cl=(100.0, 90.0, 50.0), hurst=0.25, nharm=2000,
+                                     real=lib.dtype))
+    lib.set_kernel("auto")
+    lib.srm_draw(3)
+    n = nx * 50 * 20
+    d = hip.empty(n + 1, lib.dtype)
+    a = lib.srm_run(d.ptr)
+    at = d.numpy()[:n].copy()
+    b = lib.srm_run(d.ptr + np.dtype(lib.dtype).itemsize)
+    assert np.array_equal(at, d.numpy()[1:]) and np.array_equal(a[:4], b[:4])
+    lib.finalize()
