@@ -1,6 +1,6 @@
 // Screening of the draw's trials on the GPU (see srm_host.hpp, TrialScreen):
-// the seed's stream is generated there and only the pairs that may pass the
-// rejection test come back.
+// the seed's stream is generated and tested there and only the pairs that may
+// pass come back.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -24,16 +24,17 @@ public:
     size_t reserved_bytes() const { return reserved_; }
     void set_elsewhere(size_t bytes) { elsewhere_ = bytes; }
 
-    bool screen(int seed, long first, long count, const uint32_t *limit, int bins, TrialBlock &out) override;
+    bool screen(int seed, long first, long count, const TrialTest &test, const uint32_t *limit, int bins,
+                TrialBlock &out) override;
 
 private:
     bool reserve(size_t pairs_chunks, size_t records);
     bool room(size_t bytes) const;
     hipStream_t stream_ = nullptr;
     void *d_gen_ = nullptr;      // generator tables
-    uint32_t *d_limit_ = nullptr;
-    uint32_t *d_out_ = nullptr;  // header: spans, total; then the records
-    uint32_t *h_out_ = nullptr;  // pinned
+    uint32_t *d_limit_ = nullptr;  // and the count of records after it
+    uint32_t *d_out_ = nullptr;    // spans of the chunks, records
+    uint32_t *h_out_ = nullptr;    // pinned, written by the device: total, pairs, raw outputs
     uint32_t *h_limit_ = nullptr;
     size_t chunks_ = 0, records_ = 0;
     size_t reserved_ = 0, elsewhere_ = 0;

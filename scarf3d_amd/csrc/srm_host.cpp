@@ -294,10 +294,11 @@ void record(const SrmSetup &s, double v1, double v2, double v3, double a, double
 // only looks up the next accepted pair. The pairs consumed, and so every
 // harmonic, are those of the one-pair-at-a-time loop.
 //
-// With a TrialScreen the stream is generated and screened elsewhere and only
-// the pairs that may pass arrive (TrialBlock); the workers give them the exact
-// test, the walk picks the trials, and the workers compute the harmonics. A
-// screen that fails leaves the rest of the draw to the blocks above.
+// With a TrialScreen the stream is generated and tested elsewhere and only the
+// pairs that may pass arrive, with verdicts (TrialBlock); the walk picks the
+// trials, with the exact test of the few that the screen left open, and the
+// workers compute the harmonics. A screen that fails leaves the rest of the
+// draw to the blocks above.
 template <class Real>
 class Sampler final : public HarmonicSampler {
 public:
@@ -392,7 +393,7 @@ public:
             }
             if (q + 3 >= blk_.end) fill(q);  // the trial and the (up to) three pairs after it
             const int64_t *raw = blk_.raw.data() + 2 * static_cast<size_t>(q - blk_.start);
-            if (take_trial(q, raw[0])) {
+            if (take_trial(q, kept_trial(raw[0]))) {
                 uint32_t v[8];
                 for (int k = 0; k < 8; ++k) v[k] = static_cast<uint32_t>(raw[k]);
                 harmonic(l, d_.n_used - 1, v);
@@ -409,17 +410,18 @@ private:
 
     // the accepted pair q: false when its harmonic is dropped (above kc, still
     // counted by the scaling)
-    bool take_trial(long q, int64_t first)
+    bool kept_trial(int64_t first) const { return !(ctx_.radial(DrawContext<Real>::uniform(first)) > ctx_.kc); }
+    bool take_trial(long q, bool keep)
     {
-        const bool keep = !(ctx_.radial(DrawContext<Real>::uniform(first)) > ctx_.kc);
         pos_ = q + (keep ? 4 : 2);
         d_.n_used += keep;
         d_.uniforms = 2 * pos_;
         return keep;
     }
 
-    // harmonic l, the kept-th kept one, from the outputs of its trial and the
-    // three pairs after it
+    // harmonic l (of the table; the records need its place among the kept ones
+    // only), the kept-th kept one, from the outputs of its trial and the three
+    // pairs after it
     void harmonic(int l, int kept, const uint32_t *raw)
     {
         const Real pi = kPi<Real>;
@@ -477,21 +479,16 @@ private:
         const double want = left * (trials_ + 3.0) * 1.01 + 8.0 * std::sqrt(left) * trials_ + 256.0;
         long count = static_cast<long>(std::min(want, double(1L << 25)));
         if (capped_) count = std::min(count, max_block_);
-        if (!screen_->screen(seed_, first, std::max(count, 4L), limit_.data(), ctx_.bins, tb_)) {
-            screen_ = nullptr;
-            return;
-        }
-        cand_.resize(tb_.total);
-        size_t at = 0;
-        for (size_t c = 0; c < tb_.chunks; ++c)
-            for (uint32_t k = 0; k < tb_.spans[2 * c + 1]; ++k) cand_[at++] = tb_.spans[2 * c] + k;
-        passed_.resize(tb_.total);
-        share(tb_.total, [&](size_t lo, size_t hi) {
-            for (size_t i = lo; i < hi; ++i) {
-                const uint32_t *r = tb_.records + size_t(TrialBlock::kWords) * cand_[i];
-                passed_[i] = ctx_.accepts(DrawContext<Real>::uniform(r[1]), DrawContext<Real>::uniform(r[2])) ? 1 : 0;
-            }
-        });
+        TrialTest t;
+        t.f64 = sizeof(Real) == 8;
+        t.acf = ctx_.spec.acf;
+        t.ndim = ndim_;
+        t.nu = static_cast<double>(ctx_.spec.nu);
+        t.range = static_cast<double>(ctx_.kmax - ctx_.kmin);
+        t.kmin = static_cast<double>(ctx_.kmin);
+        t.kc = static_cast<double>(ctx_.kc);
+        t.cnst = static_cast<double>(ctx_.cnst);
+        if (!screen_->screen(seed_, first, std::max(count, 4L), t, limit_.data(), ctx_.bins, tb_)) screen_ = nullptr;
         next_ = 0;
     }
 
@@ -501,25 +498,35 @@ private:
             screen_block(pos_);
             if (!screen_) return;
         }
-        picked_.clear();
         const int before = d_.n_used;
+        size_t picked = 0;  // their records' numbers take the place of pairs already passed
         while (l_ < n_ && d_.n_used < kept) {
-            while (next_ < cand_.size() && (!passed_[next_] || pair_of(next_) < pos_)) ++next_;
-            if (next_ == cand_.size()) {
+            long q = -1;
+            bool keep = false;
+            for (; next_ < tb_.total && q < 0; ++next_) {
+                const uint32_t w = tb_.pairs[next_], verdict = w >> 30;
+                const long at = tb_.start + static_cast<long>(w & 0x3fffffffu);
+                if (verdict == TrialBlock::kReject || at < pos_) continue;
+                keep = verdict == TrialBlock::kKeep;
+                if (verdict == TrialBlock::kUnsure) {
+                    const uint32_t *r = raw_of(next_);
+                    if (!ctx_.accepts(DrawContext<Real>::uniform(r[0]), DrawContext<Real>::uniform(r[1]))) continue;
+                    keep = kept_trial(r[0]);
+                }
+                q = at;
+            }
+            if (q < 0) {
                 pos_ = std::max(pos_, tb_.end);
                 break;
             }
-            const uint32_t *r = tb_.records + size_t(TrialBlock::kWords) * cand_[next_];
-            if (take_trial(pair_of(next_), r[1])) picked_.push_back(Picked{l_, cand_[next_]});
+            if (take_trial(q, keep)) tb_.pairs[picked++] = static_cast<uint32_t>(next_ - 1);
             ++l_;
         }
-        share(picked_.size(), [&](size_t lo, size_t hi) {
-            for (size_t i = lo; i < hi; ++i)
-                harmonic(picked_[i].l, before + static_cast<int>(i),
-                         tb_.records + size_t(TrialBlock::kWords) * picked_[i].record + 1);
+        share(picked, [&](size_t lo, size_t hi) {
+            for (size_t i = lo; i < hi; ++i) harmonic(0, before + static_cast<int>(i), raw_of(tb_.pairs[i]));
         });
     }
-    long pair_of(size_t i) const { return tb_.start + tb_.records[size_t(TrialBlock::kWords) * cand_[i]]; }
+    const uint32_t *raw_of(size_t i) const { return tb_.raw + TrialBlock::kRaw * i; }
 
     // make pairs [first, first + >= 4) resident
     void fill(long first)
@@ -543,10 +550,6 @@ private:
         pool_->run(job);
     }
 
-    struct Picked {
-        int l;
-        uint32_t record;
-    };
     const int n_, ndim_, seed_;
     const bool rows_only_;
     const SrmSetup setup_;
@@ -563,10 +566,7 @@ private:
     double trials_ = 1;
     std::vector<uint32_t> limit_;
     TrialBlock tb_;
-    std::vector<uint32_t> cand_;   // records in stream order
-    std::vector<uint8_t> passed_;  // their exact tests
-    std::vector<Picked> picked_;
-    size_t next_ = 0;              // first of cand_ not yet passed by the walk
+    size_t next_ = 0;  // first of tb_ not yet passed by the walk
     std::unique_lock<std::mutex> lock_;
     std::unique_ptr<WorkerPool> own_;
     WorkerPool *pool_ = nullptr;

@@ -75,25 +75,37 @@ template <class Real>
 int srm_setup(const SrmConfig &cfg, SrmSetup &out, std::string &err);
 
 // Pairs of a seed's stream screened for the rejection test: every pair in
-// [start, end) that may pass it, in records of kWords words {pair - start,
-// the 8 generator outputs of the pair and the three after it}. Chunk c of the
-// block holds spans[2 c + 1] records from spans[2 c] on; chunks and their
-// records are in stream order.
+// [start, end) that may pass it, in stream order, as pair - start with a
+// verdict in the top two bits, and the 8 generator outputs of each and of the
+// three pairs after it.
 struct TrialBlock {
-    static constexpr int kWords = 9;
+    static constexpr int kRaw = 8;
+    enum : uint32_t { kReject = 0, kKeep = 1, kDrop = 2, kUnsure = 3 };
     long start = 0, end = 0;
-    const uint32_t *spans = nullptr, *records = nullptr;
-    size_t chunks = 0, total = 0;
+    uint32_t *pairs = nullptr;  // the walk's to overwrite
+    const uint32_t *raw = nullptr;
+    size_t total = 0;
+};
+
+// The rejection test of a pair of outputs (see DrawContext::accepts): values
+// that the roundings of the pair's type make are held in doubles.
+struct TrialTest {
+    bool f64 = false;
+    int acf = 0, ndim = 3;
+    double nu = 0, range = 0, kmin = 0, kc = 0, cnst = 0;  // range: kmax - kmin
 };
 
 // Where the stream is generated and screened, other than by the draw's own
-// threads. A pair is kept when its second output is below limit[b], b the
-// first output's bin of 2^31 / bins values. The block stays valid until the
-// next call. False: not possible now (the draw then screens for itself).
+// threads. A pair is held when its second output is below limit[b], b the
+// first output's bin of 2^31 / bins values, and gets kReject, kKeep or kDrop
+// (above kc) where the test's roundings cannot decide it, kUnsure otherwise.
+// The block stays valid until the next call. False: not possible now (the draw
+// then screens for itself).
 class TrialScreen {
 public:
     virtual ~TrialScreen() = default;
-    virtual bool screen(int seed, long first, long count, const uint32_t *limit, int bins, TrialBlock &out) = 0;
+    virtual bool screen(int seed, long first, long count, const TrialTest &test, const uint32_t *limit, int bins,
+                        TrialBlock &out) = 0;
 };
 
 // The harmonic draw of one seed as a resumable walk: draw_until(m) runs the

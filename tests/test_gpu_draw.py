@@ -56,3 +56,15 @@ def test_screened_draw_is_the_oracles(request, oracle, flavour, name, kw, block)
         err = np.abs(d.numpy() - np.asarray(ref).reshape(-1, order="F")).max() / cfg["sigma"]
         print(f"  kept {n} of {cfg['nharm']}, max {err:.2e} sigma", flush=True)
         assert err <= 1e-10
+
+
+# a wave's share of the stream: one round of 64 pairs, a few, all 32; one group
+# of chunks put in order, with a remainder, and many
+SIZES = [dict(nharm=130, dh=50.0), dict(nharm=1501, dh=20.0), dict(nharm=9001, dh=4.0), dict(nharm=12000, dh=2.0)]
+
+
+@pytest.mark.parametrize("kw", SIZES, ids=[str(k["nharm"]) for k in SIZES])
+@pytest.mark.parametrize("flavour", ["f", "d"])
+def test_short_and_long_screened_draws(request, oracle, flavour, kw):
+    test_screened_draw_is_the_oracles(request, oracle, flavour, "sizes",
+                                      dict(n=(9, 8, 3), cl=(300.0, 200.0, 250.0), hurst=0.4, box=1000.0, **kw), 0)
