@@ -42,6 +42,7 @@ UNITS = [
     ("srm_host.cpp", DEVICE + HOST_EXACT, "srm_host.o"),
     ("quadpack.cpp", DEVICE + HOST_EXACT, "quadpack.o"),
     ("fim.hip", DEVICE, "fim.o"),
+    ("fim_dft.hip", DEVICE, "fim_dft.o"),
     ("fim_host.cpp", DEVICE + HOST_EXACT, "fim_host.o"),
     ("scarf_capi.cpp", DEVICE + HOST_EXACT, "scarf_capi_f.o"),
     ("scarf_capi.cpp", DEVICE + HOST_EXACT + ["-DDOUBLE_PREC"], "scarf_capi_d.o"),
@@ -160,7 +161,8 @@ def build(jobs: int = 4, verbose: bool = False) -> list[Path]:
         futs = [ex.submit(_compile, s, f, o, verbose) for s, f, o in UNITS]
         for fut in futs:
             fut.result()
-    shared = ["srm_kernels.o", "srm_mfma.o", "srm_transform.o", "srm_points.o", "srm_draw.o", "srm_host.o", "quadpack.o", "fim.o", "fim_host.o"]
+    shared = ["srm_kernels.o", "srm_mfma.o", "srm_transform.o", "srm_points.o", "srm_draw.o", "srm_host.o", "quadpack.o", "fim.o",
+              "fim_dft.o", "fim_host.o"]
     outs = []
     for obj, name in (("scarf_capi_f.o", "libscarf3df.so"), ("scarf_capi_d.o", "libscarf3d.so")):
         out = LIB / name

@@ -23,6 +23,7 @@
 #include <string>
 
 #include "fim.hpp"
+#include "fim_dft.hpp"
 #include "srm_stats.hpp"
 #include "fim_stream.hpp"
 
@@ -399,6 +400,10 @@ struct FimDevice::Impl {
     size_t pt_cap = 0;
     int *d_tab = nullptr;  // per-axis nearest indices of a structured block
     size_t tab_cap = 0;
+    void *d_dft = nullptr;  // tables of the dense transform, then its moment triples
+    size_t dft_cap = 0;
+    int dft_n[3] = {0, 0, 0};  // internal grid and sizeof(Real) of the tables
+    int dft_real = 0;
     hipfftHandle plan = 0;  // c2r over the whole internal grid
     bool plans = false;
     int plan_n[3] = {0, 0, 0};
@@ -437,6 +442,25 @@ struct FimDevice::Impl {
         }
         cap = bytes;
         reserved += bytes;
+        return true;
+    }
+    // Room for the dense transform's tables, in the place of an FFT plan and,
+    // as a plan's workspace, not counted in `reserved`
+    bool room_for_dft(size_t bytes, hipStream_t stream)
+    {
+        if (bytes <= dft_cap) return true;
+        if (d_dft) {
+            (void)hipStreamSynchronize(stream);
+            (void)hipFree(d_dft);
+        }
+        dft_real = 0;
+        dft_cap = 0;
+        if (hipMalloc(&d_dft, bytes) != hipSuccess) {
+            (void)hipGetLastError();  // the FFT library's transform runs instead
+            d_dft = nullptr;
+            return false;
+        }
+        dft_cap = bytes;
         return true;
     }
     void drop_plans()
@@ -524,20 +548,37 @@ bool FimDevice::run(const FimSetup<Real> &s, int rescale, double mute, double ta
                 "hipMemcpyAsync"))
             return false;
     }
-    // transform: one c2r over the internal grid (backward, unnormalized; the
-    // kx = 0 and Nyquist planes are Hermitian after fim_symmetry)
-    if (!m.plans || m.plan_n[0] != n1 || m.plan_n[1] != n2 || m.plan_n[2] != n3 || m.plan_real != int(sizeof(Real))) {
-        m.drop_plans();
-        const hipfftResult r = n3 > 1 ? hipfftPlan3d(&m.plan, n3, n2, n1, FftTypes<Real>::c2r)
-                                      : hipfftPlan2d(&m.plan, n2, n1, FftTypes<Real>::c2r);
-        if (!fft_ok(r, "hipfftPlan (c2r)")) return false;
-        m.plans = true;
-        m.plan_n[0] = n1;
-        m.plan_n[1] = n2;
-        m.plan_n[2] = n3;
-        m.plan_real = int(sizeof(Real));
+    // transform: dense, or one c2r over the internal grid (backward,
+    // unnormalized; the kx = 0 and Nyquist planes are Hermitian after
+    // fim_symmetry) where that is faster or the dense tables find no room
+    const size_t table_bytes = fim_dft::table_bytes<Real>(n1, n2, n3);
+    const long dft_parts = fim_dft::parts<Real>(n1, n2, n3);
+    bool dense = fim_dft::chosen<Real>(n1, n2, n3);
+    if (dense && !m.room_for_dft(table_bytes + 3 * sizeof(double) * size_t(dft_parts), stream)) dense = false;
+    if (dense) {
+        if (m.dft_n[0] != n1 || m.dft_n[1] != n2 || m.dft_n[2] != n3 || m.dft_real != int(sizeof(Real))) {
+            m.dft_real = 0;
+            if (!ok(fim_dft::make_tables<Real>(m.d_dft, n1, n2, n3, stream), "transform tables")) return false;
+            m.dft_n[0] = n1;
+            m.dft_n[1] = n2;
+            m.dft_n[2] = n3;
+            m.dft_real = int(sizeof(Real));
+        }
+    } else {
+        if (!m.plans || m.plan_n[0] != n1 || m.plan_n[1] != n2 || m.plan_n[2] != n3 ||
+            m.plan_real != int(sizeof(Real))) {
+            m.drop_plans();
+            const hipfftResult r = n3 > 1 ? hipfftPlan3d(&m.plan, n3, n2, n1, FftTypes<Real>::c2r)
+                                          : hipfftPlan2d(&m.plan, n2, n1, FftTypes<Real>::c2r);
+            if (!fft_ok(r, "hipfftPlan (c2r)")) return false;
+            m.plans = true;
+            m.plan_n[0] = n1;
+            m.plan_n[1] = n2;
+            m.plan_n[2] = n3;
+            m.plan_real = int(sizeof(Real));
+        }
+        if (!fft_ok(hipfftSetStream(m.plan, stream), "hipfftSetStream")) return false;
     }
-    if (!fft_ok(hipfftSetStream(m.plan, stream), "hipfftSetStream")) return false;
 
     Cplx<Real> *S = static_cast<Cplx<Real> *>(m.d_spec);
     Real *R = static_cast<Real *>(m.d_real);
@@ -571,13 +612,24 @@ bool FimDevice::run(const FimSetup<Real> &s, int rescale, double mute, double ta
     fim_symmetry<Real><<<static_cast<int>((sym + 255) / 256), 256, 0, stream>>>(S, n1, n2, n3, h);
     if (!ok(hipGetLastError(), "fim_symmetry launch")) return false;
     if (!ok(hipEventRecord(m.ev[2], stream), "hipEventRecord")) return false;
-    if (!fft_ok(FftTypes<Real>::exec_c2r(m.plan, S, R), "hipfftExecC2R")) return false;
-    if (!ok(hipEventRecord(m.ev[3], stream), "hipEventRecord")) return false;
-    // statistics of the scaled internal field; scaling, rescale and taper
-    fim_moments<Real><<<kScaleBlocks, 256, 0, stream>>>(R, total, s.scaling, m.d_part);
-    if (!ok(hipGetLastError(), "fim_moments launch")) return false;
-    fim_finalize<Real><<<1, 256, 0, stream>>>(m.d_part, kScaleBlocks, static_cast<double>(s.sigma), m.d_stat);
+    // and the statistics of the scaled internal field, which the dense
+    // transform takes as it writes it
+    if (dense) {
+        double *part = reinterpret_cast<double *>(static_cast<char *>(m.d_dft) + table_bytes);
+        if (!ok(fim_dft::run<Real>(S, R, m.d_dft, n1, n2, n3, s.scaling, part, stream), "transform launch"))
+            return false;
+        if (!ok(hipEventRecord(m.ev[3], stream), "hipEventRecord")) return false;
+        fim_finalize<Real><<<1, 256, 0, stream>>>(part, static_cast<int>(dft_parts), static_cast<double>(s.sigma),
+                                                  m.d_stat);
+    } else {
+        if (!fft_ok(FftTypes<Real>::exec_c2r(m.plan, S, R), "hipfftExecC2R")) return false;
+        if (!ok(hipEventRecord(m.ev[3], stream), "hipEventRecord")) return false;
+        fim_moments<Real><<<kScaleBlocks, 256, 0, stream>>>(R, total, s.scaling, m.d_part);
+        if (!ok(hipGetLastError(), "fim_moments launch")) return false;
+        fim_finalize<Real><<<1, 256, 0, stream>>>(m.d_part, kScaleBlocks, static_cast<double>(s.sigma), m.d_stat);
+    }
     if (!ok(hipGetLastError(), "fim_finalize launch")) return false;
+    // scaling, rescale and taper
     Real scale = s.scaling;  // still to apply to R when the mapping reads it
     if (rescale == 1 || npoi > 0) {
         const int blocks = static_cast<int>(std::min<long>(lines, kRowBlocks));
