@@ -215,18 +215,20 @@ __global__ __launch_bounds__(256) void fim_moments(const Real *__restrict__ R, l
 // mean, variance, info(3) = sqrt(real(var)), info(4) = real(mean) and the
 // rescale factor sigma / info(3) (src/scarflib_fim.f90:1001-1031; one
 // process: parallel_variance returns its single set unchanged)
+// one block: its threads each merge every kFinalize-th triple (7876 of 502^3: 20 us with 256)
+constexpr int kFinalize = 1024;
 template <class Real>
-__global__ __launch_bounds__(256) void fim_finalize(const double *__restrict__ part, int nparts, double sigma,
+__global__ __launch_bounds__(kFinalize) void fim_finalize(const double *__restrict__ part, int nparts, double sigma,
                                                     double *__restrict__ stat)
 {
-    __shared__ double sm[3][256];
+    __shared__ double sm[3][kFinalize];
     Moments m{0.0, 0.0, 0.0};
-    for (int b = threadIdx.x; b < nparts; b += 256) merge_moments(m, Moments{part[3 * b], part[3 * b + 1], part[3 * b + 2]});
+    for (int b = threadIdx.x; b < nparts; b += kFinalize) merge_moments(m, Moments{part[3 * b], part[3 * b + 1], part[3 * b + 2]});
     sm[0][threadIdx.x] = m.n;
     sm[1][threadIdx.x] = m.mean;
     sm[2][threadIdx.x] = m.m2;
     __syncthreads();
-    for (int stride = 128; stride >= 1; stride >>= 1) {
+    for (int stride = kFinalize / 2; stride >= 1; stride >>= 1) {
         if (threadIdx.x < stride) {
             Moments x{sm[0][threadIdx.x], sm[1][threadIdx.x], sm[2][threadIdx.x]};
             merge_moments(x, Moments{sm[0][threadIdx.x + stride], sm[1][threadIdx.x + stride], sm[2][threadIdx.x + stride]});
@@ -283,7 +285,7 @@ __global__ __launch_bounds__(256) void fim_epilogue(Real *__restrict__ R, int n1
 // 1-based internal index along one axis for coordinate x, 0 for the halo,
 // -1 outside
 template <class Real>
-__device__ inline int axis_index(Real x, Real dh, int np)
+__host__ __device__ inline int axis_index(Real x, Real dh, int np)
 {
 #pragma clang fp contract(off)
     const Real c = (x / dh + Real(3)) - Real(1);
@@ -307,21 +309,43 @@ __device__ inline Real gather(const Real *__restrict__ R, int n1, int n2, int n3
 // the block's nx + ny + nz indices are computed once; tab holds x, then y,
 // then z.
 template <class Real>
-__global__ __launch_bounds__(256) void fim_axis_tables(int *__restrict__ tab, int nx, int ny, int nz, int fx, int fy,
-                                                       int fz, Real ds, Real dh, Real ox, Real oy, Real oz, int n1,
-                                                       int n2, int n3)
-{
+struct Axis {
+    int count, first, n;  // outputs, first one's 1-based number, internal points
+    Real ds, dh, off;
+    // index of output e; rises with e, until it is -1
+    __host__ __device__ int index(int e) const
+    {
 #pragma clang fp contract(off)
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e < nx) {
-        tab[e] = axis_index(static_cast<Real>(fx - 1 + e) * ds - ox, dh, n1);
-    } else if (e < nx + ny) {
-        const int j = e - nx;
-        tab[e] = axis_index(static_cast<Real>(fy - 1 + j) * ds - oy, dh, n2);
-    } else if (e < nx + ny + nz) {
-        const int k = e - nx - ny;
-        tab[e] = axis_index(static_cast<Real>(fz - 1 + k) * ds - oz, dh, n3);
+        return axis_index(static_cast<Real>(first - 1 + e) * ds - off, dh, n);
     }
+};
+// first (if not null), for y and then z: the first output whose index is v or
+// more, v = 0 .. n + 1, where every output has an index
+template <class Real>
+__global__ __launch_bounds__(256) void fim_axis_tables(int *__restrict__ tab, Axis<Real> x, Axis<Real> y, Axis<Real> z,
+                                                       int *__restrict__ first)
+{
+    int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e < x.count) {
+        tab[e] = x.index(e);
+        return;
+    }
+    tab += x.count;
+    e -= x.count;
+    const bool along_y = e < y.count;
+    const Axis<Real> a = along_y ? y : z;
+    if (!along_y) {
+        tab += y.count;
+        e -= y.count;
+        if (first) first += y.n + 2;
+    }
+    if (e >= a.count) return;
+    const int index = a.index(e);
+    tab[e] = index;
+    if (!first) return;
+    for (int v = e > 0 ? a.index(e - 1) + 1 : 0; v <= index; ++v) first[v] = e;
+    if (e == a.count - 1)
+        for (int v = index + 1; v <= a.n + 1; ++v) first[v] = a.count;
 }
 
 // The block's values: each block walks groups of 4 output x-lines
@@ -385,6 +409,7 @@ struct FftTypes<double> {
 };
 
 constexpr int kScaleBlocks = 2048;  // 8 blocks of 256 per compute unit
+constexpr long kDirectPoints = 1L << 25;  // internal points from which the transform writes a block itself
 constexpr long kRowBlocks = 8192;   // row-walking passes: 32 blocks per compute unit
 
 }  // namespace
@@ -400,7 +425,7 @@ struct FimDevice::Impl {
     size_t pt_cap = 0;
     int *d_tab = nullptr;  // per-axis nearest indices of a structured block
     size_t tab_cap = 0;
-    void *d_dft = nullptr;  // tables of the dense transform, then its moment triples
+    void *d_dft = nullptr;  // tables of the dense transform, its moment triples, the nodes' first outputs
     size_t dft_cap = 0;
     int dft_n[3] = {0, 0, 0};  // internal grid and sizeof(Real) of the tables
     int dft_real = 0;
@@ -553,8 +578,10 @@ bool FimDevice::run(const FimSetup<Real> &s, int rescale, double mute, double ta
     // fim_symmetry) where that is faster or the dense tables find no room
     const size_t table_bytes = fim_dft::table_bytes<Real>(n1, n2, n3);
     const long dft_parts = fim_dft::parts<Real>(n1, n2, n3);
+    const size_t part_bytes = 3 * sizeof(double) * size_t(dft_parts);
     bool dense = fim_dft::chosen<Real>(n1, n2, n3);
-    if (dense && !m.room_for_dft(table_bytes + 3 * sizeof(double) * size_t(dft_parts), stream)) dense = false;
+    if (dense && !m.room_for_dft(table_bytes + part_bytes + sizeof(int) * (size_t(n2) + n3 + 4), stream))
+        dense = false;
     if (dense) {
         if (m.dft_n[0] != n1 || m.dft_n[1] != n2 || m.dft_n[2] != n3 || m.dft_real != int(sizeof(Real))) {
             m.dft_real = 0;
@@ -604,7 +631,41 @@ bool FimDevice::run(const FimSetup<Real> &s, int rescale, double mute, double ta
     a.acf = s.acf;
     const long items = (lines + a.lines_per_item - 1) / a.lines_per_item;
     const int sblocks = static_cast<int>(std::min<long>((items + 3) / 4, 2048));
+    // a structured block's nearest indices; direct: the transform's last pass
+    // writes the block, every point of which has a node, and R is not needed
+    const Axis<Real> ax{fe[0] - fs[0] + 1, fs[0], n1, s.ds, s.dh, s.off_axis[0]};
+    const Axis<Real> ay{fe[1] - fs[1] + 1, fs[1], n2, s.ds, s.dh, s.off_axis[1]};
+    const Axis<Real> az{fe[2] - fs[2] + 1, fs[2], n3, s.ds, s.dh, s.off_axis[2]};
+    const long rows = long(ay.count) * az.count;
+    fim_dft::Nearest<Real> nearest;
+    if (structured) {
+        if (rows >= (long(1) << 31)) {
+            err = "FIM: output grid too large for the mapping launch";
+            return false;
+        }
+        const size_t outputs = size_t(ax.count) + ay.count + az.count;
+        if (!m.grow(reinterpret_cast<void **>(&m.d_tab), m.tab_cap, sizeof(int) * outputs, stream,
+                    reserved_elsewhere, err))
+            return false;
+        // calls, direct against R and fim_map_grid, in ms: 502^3 1.73 : 1.83, 610 x 366 x 364 1.32 : 1.42, 640 x 640
+        // x 102 0.74 : 0.81, double 502 x 502 x 202 1.49 : 1.62; 258^3 0.355 : 0.348, 302 x 258 0.095 : 0.090
+        if (dense && total >= kDirectPoints && rescale != 1 && npoi == 0 && ax.index(0) > 0 && ax.index(ax.count - 1) > 0 && ay.index(0) > 0 &&
+            ay.index(ay.count - 1) > 0 && az.index(0) >= 0 && az.index(az.count - 1) >= 0) {
+            nearest.field = d_field;
+            nearest.nx = ax.count;
+            nearest.ny = ay.count;
+            nearest.x = m.d_tab;
+            nearest.first_y = reinterpret_cast<const int *>(static_cast<char *>(m.d_dft) + table_bytes + part_bytes);
+            nearest.first_z = nearest.first_y + n2 + 2;
+        }
+    }
+    const bool direct = nearest.field != nullptr;
     if (!ok(hipEventRecord(m.ev[0], stream), "hipEventRecord")) return false;
+    if (structured) {
+        fim_axis_tables<Real><<<static_cast<unsigned>((long(ax.count) + ay.count + az.count + 255) / 256), 256, 0,
+                                stream>>>(m.d_tab, ax, ay, az, direct ? const_cast<int *>(nearest.first_y) : nullptr);
+        if (!ok(hipGetLastError(), "fim_axis_tables launch")) return false;
+    }
     fim_spectrum<Real><<<sblocks, 256, 0, stream>>>(S, a, m.d_gen, items);
     if (!ok(hipGetLastError(), "fim_spectrum launch")) return false;
     if (!ok(hipEventRecord(m.ev[1], stream), "hipEventRecord")) return false;
@@ -616,17 +677,17 @@ bool FimDevice::run(const FimSetup<Real> &s, int rescale, double mute, double ta
     // transform takes as it writes it
     if (dense) {
         double *part = reinterpret_cast<double *>(static_cast<char *>(m.d_dft) + table_bytes);
-        if (!ok(fim_dft::run<Real>(S, R, m.d_dft, n1, n2, n3, s.scaling, part, stream), "transform launch"))
+        if (!ok(fim_dft::run<Real>(S, R, nearest, m.d_dft, n1, n2, n3, s.scaling, part, stream), "transform launch"))
             return false;
         if (!ok(hipEventRecord(m.ev[3], stream), "hipEventRecord")) return false;
-        fim_finalize<Real><<<1, 256, 0, stream>>>(part, static_cast<int>(dft_parts), static_cast<double>(s.sigma),
+        fim_finalize<Real><<<1, kFinalize, 0, stream>>>(part, static_cast<int>(dft_parts), static_cast<double>(s.sigma),
                                                   m.d_stat);
     } else {
         if (!fft_ok(FftTypes<Real>::exec_c2r(m.plan, S, R), "hipfftExecC2R")) return false;
         if (!ok(hipEventRecord(m.ev[3], stream), "hipEventRecord")) return false;
         fim_moments<Real><<<kScaleBlocks, 256, 0, stream>>>(R, total, s.scaling, m.d_part);
         if (!ok(hipGetLastError(), "fim_moments launch")) return false;
-        fim_finalize<Real><<<1, 256, 0, stream>>>(m.d_part, kScaleBlocks, static_cast<double>(s.sigma), m.d_stat);
+        fim_finalize<Real><<<1, kFinalize, 0, stream>>>(m.d_part, kScaleBlocks, static_cast<double>(s.sigma), m.d_stat);
     }
     if (!ok(hipGetLastError(), "fim_finalize launch")) return false;
     // scaling, rescale and taper
@@ -642,22 +703,9 @@ bool FimDevice::run(const FimSetup<Real> &s, int rescale, double mute, double ta
     if (!ok(hipEventRecord(m.ev[4], stream), "hipEventRecord")) return false;
     // nearest-neighbour values at the caller's points
     if (structured) {
-        const int nx = fe[0] - fs[0] + 1, ny = fe[1] - fs[1] + 1, nz = fe[2] - fs[2] + 1;
-        const long rows = long(ny) * nz;
-        if (rows >= (long(1) << 31)) {
-            err = "FIM: output grid too large for the mapping launch";
-            return false;
-        }
-        const int blocks = static_cast<int>(std::min<long>(rows, kRowBlocks));
-        if (!m.grow(reinterpret_cast<void **>(&m.d_tab), m.tab_cap, sizeof(int) * size_t(nx + ny + nz), stream,
-                    reserved_elsewhere, err))
-            return false;
-        fim_axis_tables<Real><<<(nx + ny + nz + 255) / 256, 256, 0, stream>>>(
-            m.d_tab, nx, ny, nz, fs[0], fs[1], fs[2], s.ds, s.dh, s.off_axis[0], s.off_axis[1], s.off_axis[2], n1, n2,
-            n3);
-        if (!ok(hipGetLastError(), "fim_axis_tables launch")) return false;
-        fim_map_grid<Real><<<blocks, 256, 0, stream>>>(R, n1, n2, n3, scale, d_field, m.d_tab, nx, ny,
-                                                       static_cast<int>(rows));
+        if (!direct)
+            fim_map_grid<Real><<<static_cast<int>(std::min<long>(rows, kRowBlocks)), 256, 0, stream>>>(
+                R, n1, n2, n3, scale, d_field, m.d_tab, ax.count, ay.count, static_cast<int>(rows));
     } else {
         const int mblocks = static_cast<int>(std::max<long>(1, std::min<long>((npoints + 255) / 256, 8192)));
         fim_map_points<Real><<<mblocks, 256, 0, stream>>>(R, n1, n2, n3, s.dh, scale, d_field, d_points,

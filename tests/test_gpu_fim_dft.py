@@ -13,7 +13,7 @@ from __future__ import annotations
 
 import numpy as np
 import pytest
-from test_gpu_fim import _check, _fim, _say
+from test_gpu_fim import _check, _fim, _run, _say
 
 from scarf3d_amd.workloads import structured_cfg
 
@@ -61,3 +61,35 @@ def test_tables_follow_the_grid(lib_f, lib_d):
         _say(n, flav)
         _check(lib, _grid(n, np.float32 if flav == "f" else np.float64), 413, flav)
         lib.finalize()
+
+
+# From 2^25 internal points on the transform's last pass writes a block itself. A point of interest
+# that reaches no point keeps the field by way of the internal grid: equal bit for bit.
+MODEL = (801, 213, 205)  # internal 802 x 214 x 206
+BLOCKS = [
+    (dict(n=MODEL, ds=25.0), "the whole model"),
+    (dict(n=(400, 106, 102), ds=50.0), "nodes without an output"),
+    (dict(n=(81, 63, 49), ds=20.0), "nodes with two outputs"),
+    (dict(n=(20, 16, 29), fs=(11, 5, 1), ds=25.0), "an inner block"),
+    (dict(n=(1, 1, 1), fs=MODEL, ds=25.0), "the model's last point"),
+]
+
+
+@pytest.mark.parametrize("flav", ["f", "d"])
+@pytest.mark.parametrize("kw,why", BLOCKS, ids=[b[1].replace(" ", "_") for b in BLOCKS])
+def test_blocks_of_the_last_pass(lib_f, lib_d, kw, why, flav):
+    lib = lib_f if flav == "f" else lib_d
+    got = []
+    for poi in (None, np.full((3, 1), -1e6)):
+        extra = {} if poi is None else dict(poi=poi, mute=1.0, taper=1.0)
+        cfg = structured_cfg(cl=(400.0, 300.0, 200.0), hurst=0.3, sigma=0.05, dh=25.0,
+                             real=np.float32 if flav == "f" else np.float64, **kw, **extra)
+        cfg["nc"] = (0.0, 0.0, 0.0)
+        cfg["fc"] = tuple((n - 1) * 25.0 for n in MODEL)
+        _say(why, flav, "through the internal grid" if extra else "")
+        field, stats = _run(lib, _fim(cfg), 414)
+        lib.finalize()
+        got.append((np.array(field), np.array(stats[:4])))
+    assert np.any(got[0][0])
+    assert np.array_equal(got[0][0], got[1][0])
+    assert np.array_equal(got[0][1], got[1][1])
