@@ -74,7 +74,11 @@ __host__ __device__ inline void jump(const uint32_t (*jt)[4], uint64_t n, uint32
 // The walk of one work item of the spectrum kernel: x-lines [l0, l1) of n1
 // positions each (line L starts at stream position n1 L), lane `lane` of a
 // 64-wide wave visiting points i = lane, lane + 64, ... < h of every line.
-// f(line, i, value) receives the stream value of position i + n1 line.
+// f(line, i, value) receives the stream value of position i + n1 line, the
+// lines in ascending order for each i. Values n1 apart follow the two-term
+// recursion of the characteristic polynomial of A^n1,
+//   x[L + 1] = trace x[L] - det x[L - 1],
+// half the products of a step of the state.
 // pw: the power table (a copy in LDS on the device); line_step = A^n1;
 // s0: state of stream position 0.
 template <class F>
@@ -85,13 +89,34 @@ __host__ __device__ inline void walk_item(const uint32_t *pw, const Tables *t, c
     uint32_t r0 = s0[0], r1 = s0[1];
     jump(t->jump, uint64_t(n1) * uint64_t(l0), r0, r1);  // position n1 l0
     matvec(t->lane[lane], r0, r1);                       // + lane
-    for (long line = l0; line < l1; ++line) {
-        uint32_t q0 = r0, q1 = r1;
-        for (int i = lane; i < h; i += 64) {
-            f(line, i, value(pw, q0));
-            matvec(t->step64, q0, q1);
+    const uint32_t trace = mod_m(uint64_t(line_step[0]) + line_step[3]);
+    const uint32_t minus_det = mod_m(uint64_t(mod_m(uint64_t(line_step[1]) * line_step[2])) + kM -
+                                     mod_m(uint64_t(line_step[0]) * line_step[3]));
+    struct Point {
+        uint32_t x, next;
+    };
+    // four points of a line at a time: what they write is near in time too
+    // (spectrum of 502^3 in float: one at a time 177 us, two 146, four 137;
+    // 256 x 256 x 102 in double: two 105 us, four 92)
+    constexpr int C = 4;
+    for (int i = lane; i < h; i += 64 * C) {
+        Point p[C];
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            if (i + 64 * c >= h) break;
+            p[c] = Point{r0, mod_m(uint64_t(line_step[0]) * r0 + uint64_t(line_step[1]) * r1)};
+            matvec(t->step64, r0, r1);
         }
-        matvec(line_step, r0, r1);
+        for (long line = l0; line < l1; ++line) {
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                if (i + 64 * c >= h) break;
+                f(line, i + 64 * c, value(pw, p[c].x));
+                const uint32_t after = mod_m(uint64_t(trace) * p[c].next + uint64_t(minus_det) * p[c].x);
+                p[c].x = p[c].next;
+                p[c].next = after;
+            }
+        }
     }
 }
 
