@@ -17,7 +17,8 @@ extern "C" {
 enum scarf_kernel {
     SCARF_KERNEL_AUTO = 0,        /* grids: a fast nonuniform transform of the library's precision where that is faster
                                      than the direct sum (from a few hundred harmonics on), else mfma_bf16x3 or
-                                     direct_f32 (float lib), direct_f64 (double lib); point lists: direct_f32,
+                                     direct_f32 (float lib), direct_f64 (double lib); point lists: interpolated
+                                     from a grid by that transform where that is faster, else direct_f32,
                                      direct_f64 */
     SCARF_KERNEL_DIRECT_F32 = 1,  /* FP32 cos on FP64-reduced phases, FP64-promoted sums */
     SCARF_KERNEL_DIRECT_F64 = 2,  /* FP64 throughout */
