@@ -8,10 +8,12 @@
 //   partials (3 doubles per block), statistics (6 doubles), points of
 //   interest; the generator tables (fim_stream.hpp: 18 KB of powers of the
 //   primitive root, the companion-matrix powers), uploaded once per process.
-// Work per internal point (bytes of HBM): spectrum 8 (written), symmetry
-// reads/writes 2 planes, the c2r transform ~3 passes over S plus R, statistics 4
-// (R read), epilogue 8 if active, mapping 4 per output point plus the
-// gathered R values.
+// Work per internal point (bytes of HBM, float): spectrum 4 (written), symmetry
+// reads/writes 2 planes, the dense transform 8 each along y and z, 4 read and
+// 4 written along x with the statistics (fim_dft.hpp); with the FFT library's
+// transform, or a block that a rescale or a point of interest changes, also
+// statistics 4 (R read), epilogue 8 if active, mapping 4 per output point plus
+// the gathered R values.
 #include <hip/hip_runtime.h>
 #include <hipfft/hipfft.h>
 
