@@ -134,13 +134,14 @@ __global__ __launch_bounds__(256) void points_order(GridArgs a, const double *__
 // took 0.31 and, with 14 taps, two thirds of the products, 3.8 ms. Visited by
 // bins, points share lines and the grid is read from HBM about once.
 template <class Real>
-__global__ __launch_bounds__(256) void points_interpolate(GridArgs a, const Real *__restrict__ grid,
-                                                          const double *__restrict__ pts, long npts,
-                                                          const int *__restrict__ perm, Real *__restrict__ field)
+__global__ __launch_bounds__(kPointsThreads) void points_interpolate(GridArgs a, const Real *__restrict__ grid,
+                                                                     const double *__restrict__ pts, long first,
+                                                                     long npts, const int *__restrict__ perm,
+                                                                     Real *__restrict__ field)
 {
     constexpr int W = kTaps<Real>;
     const int tap = threadIdx.x % W;
-    const long s = blockIdx.x * long(256 / W) + threadIdx.x / W;
+    const long s = first + blockIdx.x * long(kPointsThreads / W) + threadIdx.x / W;
     const long i = s < npts ? (perm ? perm[s] : s) : 0;  // spare lanes repeat a point
     const double e_beta = exp(-a.beta);
     double t[3] = {1.0, 1.0, 1.0};
@@ -195,6 +196,15 @@ __global__ __launch_bounds__(256) void points_moments(const Real *__restrict__ v
 }
 
 }  // namespace
+
+std::vector<PointsLaunch> points_launches(long npts, bool f64)
+{
+    const long per_block = kPointsThreads / (f64 ? kTaps<double> : kTaps<float>);
+    std::vector<PointsLaunch> out;
+    for (long first = 0; first < npts; first += kPointsBlocks * per_block)
+        out.push_back({first, static_cast<unsigned>(std::min(kPointsBlocks, (npts - first + per_block - 1) / per_block))});
+    return out;
+}
 
 bool points_plan(const double lo[3], const double hi[3], const double wmax[3], bool flat, long npts, int np_, bool f64,
                  PointsPlan &p)
@@ -311,8 +321,10 @@ bool points_field(const PointsPlan &p, const double *d_pts, const double *d_harm
         points_order<Real><<<blocks, 256, 0, stream>>>(a, d_pts, p.npts, count, perm);
         if (!ok(hipGetLastError(), "points_order")) return false;
     }
-    points_interpolate<Real><<<unsigned((p.npts * kTaps<Real> + 255) / 256), 256, 0, stream>>>(a, grid, d_pts, p.npts, perm, d_field);
-    if (!ok(hipGetLastError(), "points_interpolate")) return false;
+    for (const PointsLaunch &l : points_launches(p.npts, sizeof(Real) == sizeof(double))) {
+        points_interpolate<Real><<<l.blocks, kPointsThreads, 0, stream>>>(a, grid, d_pts, l.first, p.npts, perm, d_field);
+        if (!ok(hipGetLastError(), "points_interpolate")) return false;
+    }
     points_moments<Real><<<p.nparts, 256, 0, stream>>>(d_field, p.npts, d_part);
     return ok(hipGetLastError(), "points_moments");
 }

@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include <string>
+#include <vector>
 
 #include "srm_transform.hpp"
 
@@ -30,6 +31,17 @@ struct PointsPlan {
     size_t bytes = 0;
     size_t o_grid = 0, o_record = 0, o_work = 0, o_part = 0, o_count = 0, o_perm = 0;
 };
+
+// The interpolation's launches: a thread per point and tap would pass the 2^32
+// threads that one launch can have (from 2^29 points in float, 2^28 in double),
+// so each takes the points of 2^18 blocks, 8M in float and 4M in double.
+struct PointsLaunch {
+    long first = 0;  // point
+    unsigned blocks = 0;
+};
+constexpr int kPointsThreads = 256;
+constexpr long kPointsBlocks = 1L << 18;
+std::vector<PointsLaunch> points_launches(long npts, bool f64);
 
 // lo, hi: the points' extent; wmax: the largest |w| per axis of the record.
 // False where the grid would be too large or the extent is not finite.

@@ -1,0 +1,7 @@
+"""Host-side rules of the device paths, at sizes no test could run: checked on
+the CPU through the built library's internal headers."""
+from native_lib import build_check, run_check
+
+
+def test_point_lists_of_any_size_launch_within_the_limit(tmp_path):
+    assert "0 bad" in run_check(build_check("points_launches", tmp_path))
