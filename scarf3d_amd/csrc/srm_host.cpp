@@ -402,8 +402,6 @@ public:
         return d_.n_used;
     }
 
-    HarmonicDraw take() { return std::move(d_); }
-
 private:
     // fewer pairs cost less here (17 ns each) than the round trip to the GPU (about 50 us)
     static constexpr double kScreenPairs = 2000.0;
@@ -588,14 +586,6 @@ std::unique_ptr<HarmonicSampler> HarmonicSampler::create_rows(const SrmConfig &c
     return std::unique_ptr<HarmonicSampler>(new Sampler<Real>(cfg, setup, seed, threads, block_pairs, true, screen));
 }
 
-template <class Real>
-HarmonicDraw srm_draw(const SrmConfig &cfg, const SrmSetup &s, int seed, int threads, long block_pairs)
-{
-    Sampler<Real> w(cfg, s, seed, threads, block_pairs);
-    w.draw_until(cfg.nharm);
-    return w.take();
-}
-
 HarmonicTable build_table(const SrmSetup &s, const HarmonicDraw &d)
 {
     HarmonicTable t;
@@ -620,8 +610,6 @@ HarmonicTable build_table(const SrmSetup &s, const HarmonicDraw &d)
 
 template int srm_setup<float>(const SrmConfig &, SrmSetup &, std::string &);
 template int srm_setup<double>(const SrmConfig &, SrmSetup &, std::string &);
-template HarmonicDraw srm_draw<float>(const SrmConfig &, const SrmSetup &, int, int, long);
-template HarmonicDraw srm_draw<double>(const SrmConfig &, const SrmSetup &, int, int, long);
 template std::unique_ptr<HarmonicSampler> HarmonicSampler::create<float>(const SrmConfig &, const SrmSetup &, int,
                                                                          int, long);
 template std::unique_ptr<HarmonicSampler> HarmonicSampler::create<double>(const SrmConfig &, const SrmSetup &, int,

@@ -112,7 +112,7 @@ public:
 // reference's draw loop until m harmonics have been kept (or every harmonic
 // has been drawn), so that a caller can hand the first harmonics to the
 // device while the rest are still drawn. Where the walk is cut never
-// changes the harmonics: srm_draw is one draw_until to the end.
+// changes the harmonics.
 // threads <= 0: default_draw_threads(); block_pairs <= 0: 2^18 pairs per
 // block at most (smaller blocks only change how the work is cut, never the
 // harmonics).
@@ -138,12 +138,10 @@ public:
     virtual HarmonicRows rows(int k0, int k1) const = 0;
 };
 
-template <class Real>
-HarmonicDraw srm_draw(const SrmConfig &cfg, const SrmSetup &setup, int seed, int threads = 0, long block_pairs = 0);
-
 // SCARF_DRAW_THREADS if set, else min(16, hardware threads)
 int default_draw_threads();
 
+// device records of a whole draw by create(): what create_rows() is checked against
 HarmonicTable build_table(const SrmSetup &setup, const HarmonicDraw &draw);
 
 }  // namespace scarf
