@@ -24,6 +24,7 @@
 #include <cstring>
 #include <string>
 
+#include "device_budget.hpp"
 #include "fim.hpp"
 #include "fim_dft.hpp"
 #include "srm_stats.hpp"
@@ -451,26 +452,24 @@ struct FimDevice::Impl {
     int plan_real = 0;  // sizeof(Real) of the plans
     hipEvent_t ev[6] = {};
     bool ready = false;  // the fixed buffers and events exist
-    size_t reserved = 0;
 
-    // grows *p to `bytes` (kept when large enough); the stream is drained
-    // before a buffer it may still use is freed
-    bool grow(void **p, size_t &cap, size_t bytes, hipStream_t stream, size_t elsewhere, std::string &err)
+    // grows *p to `bytes` (kept when large enough), the library's spares
+    // making room if they must; the stream is drained before a buffer it may
+    // still use is freed
+    bool grow(void **p, size_t &cap, size_t bytes, hipStream_t stream, std::string &err)
     {
         if (bytes <= cap && *p) return true;
-        if (const char *e = std::getenv("SCARF_DEVICE_MEMORY_LIMIT")) {
-            const double limit = std::atof(e);
-            const size_t after = elsewhere + reserved + bytes - std::min(bytes, cap);
-            if (limit > 0 && double(after) > limit) {
-                err = "device memory limit SCARF_DEVICE_MEMORY_LIMIT=" + std::string(e) + " bytes: the library holds " +
-                      std::to_string(elsewhere + reserved) + " and would need " + std::to_string(after);
-                return false;
-            }
-        }
+        if (grow_if_room(p, cap, bytes, stream, err)) return true;
+        device_budget().drop_spares();
+        return grow_if_room(p, cap, bytes, stream, err);
+    }
+    bool grow_if_room(void **p, size_t &cap, size_t bytes, hipStream_t stream, std::string &err)
+    {
+        if (!device_budget().fits(bytes - std::min(bytes, cap), &err)) return false;
         if (*p) {
             (void)hipStreamSynchronize(stream);
             (void)hipFree(*p);
-            reserved -= cap;
+            device_budget().give(cap);
             *p = nullptr;
             cap = 0;
         }
@@ -482,27 +481,34 @@ struct FimDevice::Impl {
             return false;
         }
         cap = bytes;
-        reserved += bytes;
+        device_budget().take(bytes);
         return true;
     }
-    // Room for the dense transform's tables, in the place of an FFT plan and,
-    // as a plan's workspace, not counted in `reserved`
-    bool room_for_dft(size_t bytes, hipStream_t stream)
+    // Room for the dense transform's tables, which are a spare: without it the
+    // FFT library's transform runs instead
+    bool room_for_dft(size_t bytes)
     {
         if (bytes <= dft_cap) return true;
-        if (d_dft) {
-            (void)hipStreamSynchronize(stream);
-            (void)hipFree(d_dft);
-        }
-        dft_real = 0;
-        dft_cap = 0;
+        drop_dft();
+        if (!device_budget().fits(bytes)) return false;
         if (hipMalloc(&d_dft, bytes) != hipSuccess) {
-            (void)hipGetLastError();  // the FFT library's transform runs instead
+            (void)hipGetLastError();
             d_dft = nullptr;
             return false;
         }
         dft_cap = bytes;
+        device_budget().take(bytes);
         return true;
+    }
+    void drop_dft()
+    {
+        if (!d_dft) return;
+        (void)hipDeviceSynchronize();
+        (void)hipFree(d_dft);
+        d_dft = nullptr;
+        device_budget().give(dft_cap);
+        dft_cap = 0;
+        dft_real = 0;
     }
     void drop_plans()
     {
@@ -512,7 +518,11 @@ struct FimDevice::Impl {
     }
 };
 
-FimDevice::FimDevice() : impl_(new Impl) {}
+FimDevice::FimDevice() : impl_(new Impl)
+{
+    Impl *m = impl_.get();
+    device_budget().add_spare(m, [m] { m->drop_dft(); });
+}
 
 FimDevice::~FimDevice()
 {
@@ -521,12 +531,10 @@ FimDevice::~FimDevice()
     impl_.release();
 }
 
-size_t FimDevice::reserved_bytes() const { return impl_ ? impl_->reserved : 0; }
-
 template <class Real>
 bool FimDevice::run(const FimSetup<Real> &s, int rescale, double mute, double taper, int seed, int fs[3], int fe[3],
                     bool structured, const double *d_points, long npoints, Real *d_field, double stats[4],
-                    hipStream_t stream, size_t reserved_elsewhere, std::string &err)
+                    hipStream_t stream, std::string &err)
 {
     Impl &m = *impl_;
     auto ok = [&](hipError_t e, const char *what) {
@@ -560,15 +568,15 @@ bool FimDevice::run(const FimSetup<Real> &s, int rescale, double mute, double ta
                 return false;
             }
             m.d_gen = static_cast<GenTables *>(g);
-            m.reserved += sizeof(GenTables);
+            device_budget().take(sizeof(GenTables));
         }
         if (!m.d_part) {
             if (!ok(hipMalloc(&m.d_part, sizeof(double) * 3 * kScaleBlocks), "hipMalloc")) return false;
-            m.reserved += sizeof(double) * 3 * kScaleBlocks;
+            device_budget().take(sizeof(double) * 3 * kScaleBlocks);
         }
         if (!m.d_stat) {
             if (!ok(hipMalloc(&m.d_stat, sizeof(double) * 8), "hipMalloc")) return false;
-            m.reserved += sizeof(double) * 8;
+            device_budget().take(sizeof(double) * 8);
         }
         if (!m.h_stat && !ok(hipHostMalloc(reinterpret_cast<void **>(&m.h_stat), sizeof(double) * 8,
                                            hipHostMallocDefault),
@@ -578,15 +586,28 @@ bool FimDevice::run(const FimSetup<Real> &s, int rescale, double mute, double ta
             if (!e && !ok(hipEventCreate(&e), "hipEventCreate")) return false;
         m.ready = true;
     }
-    if (!m.grow(&m.d_spec, m.spec_cap, sizeof(Cplx<Real>) * size_t(h) * size_t(lines), stream, reserved_elsewhere,
-                err))
+    if (!m.grow(&m.d_spec, m.spec_cap, sizeof(Cplx<Real>) * size_t(h) * size_t(lines), stream, err))
         return false;
-    if (!m.grow(&m.d_real, m.real_cap, sizeof(Real) * size_t(total), stream, reserved_elsewhere, err)) return false;
+    if (!m.grow(&m.d_real, m.real_cap, sizeof(Real) * size_t(total), stream, err)) return false;
     const int npoi = static_cast<int>(s.pt.size() / 3);
     if (npoi > 0) {
-        if (!m.grow(&m.d_pt, m.pt_cap, sizeof(Real) * s.pt.size(), stream, reserved_elsewhere, err)) return false;
+        if (!m.grow(&m.d_pt, m.pt_cap, sizeof(Real) * s.pt.size(), stream, err)) return false;
         if (!ok(hipMemcpyAsync(m.d_pt, s.pt.data(), sizeof(Real) * s.pt.size(), hipMemcpyHostToDevice, stream),
                 "hipMemcpyAsync"))
+            return false;
+    }
+    // a structured block's nearest indices
+    const Axis<Real> ax{fe[0] - fs[0] + 1, fs[0], n1, s.ds, s.dh, s.off_axis[0]};
+    const Axis<Real> ay{fe[1] - fs[1] + 1, fs[1], n2, s.ds, s.dh, s.off_axis[1]};
+    const Axis<Real> az{fe[2] - fs[2] + 1, fs[2], n3, s.ds, s.dh, s.off_axis[2]};
+    const long rows = long(ay.count) * az.count;
+    if (structured) {
+        if (rows >= (long(1) << 31)) {
+            err = "FIM: output grid too large for the mapping launch";
+            return false;
+        }
+        const size_t outputs = size_t(ax.count) + ay.count + az.count;
+        if (!m.grow(reinterpret_cast<void **>(&m.d_tab), m.tab_cap, sizeof(int) * outputs, stream, err))
             return false;
     }
     // transform: dense, or one c2r over the internal grid (backward,
@@ -596,8 +617,7 @@ bool FimDevice::run(const FimSetup<Real> &s, int rescale, double mute, double ta
     const long dft_parts = fim_dft::parts<Real>(n1, n2, n3);
     const size_t part_bytes = 3 * sizeof(double) * size_t(dft_parts);
     bool dense = fim_dft::chosen<Real>(n1, n2, n3);
-    if (dense && !m.room_for_dft(table_bytes + part_bytes + sizeof(int) * (size_t(n2) + n3 + 4), stream))
-        dense = false;
+    if (dense && !m.room_for_dft(table_bytes + part_bytes + sizeof(int) * (size_t(n2) + n3 + 4))) dense = false;
     if (dense) {
         if (m.dft_n[0] != n1 || m.dft_n[1] != n2 || m.dft_n[2] != n3 || m.dft_real != int(sizeof(Real))) {
             m.dft_real = 0;
@@ -650,22 +670,10 @@ bool FimDevice::run(const FimSetup<Real> &s, int rescale, double mute, double ta
     a.acf = s.acf;
     const long items = (lines + a.lines_per_item - 1) / a.lines_per_item;
     const int sblocks = static_cast<int>(std::min<long>((items + 3) / 4, 2048));
-    // a structured block's nearest indices; direct: the transform's last pass
-    // writes the block, every point of which has a node, and R is not needed
-    const Axis<Real> ax{fe[0] - fs[0] + 1, fs[0], n1, s.ds, s.dh, s.off_axis[0]};
-    const Axis<Real> ay{fe[1] - fs[1] + 1, fs[1], n2, s.ds, s.dh, s.off_axis[1]};
-    const Axis<Real> az{fe[2] - fs[2] + 1, fs[2], n3, s.ds, s.dh, s.off_axis[2]};
-    const long rows = long(ay.count) * az.count;
+    // direct: the transform's last pass writes the block, every point of which
+    // has a node, and R is not needed
     fim_dft::Nearest<Real> nearest;
     if (structured) {
-        if (rows >= (long(1) << 31)) {
-            err = "FIM: output grid too large for the mapping launch";
-            return false;
-        }
-        const size_t outputs = size_t(ax.count) + ay.count + az.count;
-        if (!m.grow(reinterpret_cast<void **>(&m.d_tab), m.tab_cap, sizeof(int) * outputs, stream,
-                    reserved_elsewhere, err))
-            return false;
         // calls, direct against R and fim_map_grid, in ms: 502^3 1.73 : 1.83, 610 x 366 x 364 1.32 : 1.42, 640 x 640
         // x 102 0.74 : 0.81, double 502 x 502 x 202 1.49 : 1.62; 258^3 0.355 : 0.348, 302 x 258 0.095 : 0.090
         if (dense && total >= kDirectPoints && rescale != 1 && npoi == 0 && ax.index(0) > 0 && ax.index(ax.count - 1) > 0 && ay.index(0) > 0 &&
@@ -758,8 +766,8 @@ bool FimDevice::run(const FimSetup<Real> &s, int rescale, double mute, double ta
 }
 
 template bool FimDevice::run<float>(const FimSetup<float> &, int, double, double, int, int[3], int[3], bool,
-                                    const double *, long, float *, double[4], hipStream_t, size_t, std::string &);
+                                    const double *, long, float *, double[4], hipStream_t, std::string &);
 template bool FimDevice::run<double>(const FimSetup<double> &, int, double, double, int, int[3], int[3], bool,
-                                     const double *, long, double *, double[4], hipStream_t, size_t, std::string &);
+                                     const double *, long, double *, double[4], hipStream_t, std::string &);
 
 }  // namespace scarf

@@ -255,9 +255,6 @@ bool ensure_device()
         return false;
     }
     if (!s.trials) s.trials = std::make_unique<scarf::TrialDevice>();
-    const size_t fim = s.fim ? s.fim->reserved_bytes() : 0;
-    s.trials->set_elsewhere(s.device->reserved_bytes() + fim);
-    s.device->set_external_reserved(s.trials->reserved_bytes() + fim);
     return true;
 }
 
@@ -366,7 +363,7 @@ int execute_fim(int seed, real *d_field, real stats[], const scarf::Device::Slab
     }
     double st[4] = {};
     if (!s.fim->run<real>(fs, s.cfg.rescale, s.cfg.mute, s.cfg.taper, seed, fsi, fei, s.cfg.structured, pts,
-                          s.cfg.npts, d_field, st, s.device->stream(), s.device->reserved_bytes(), err))
+                          s.cfg.npts, d_field, st, s.device->stream(), err))
         return fail(err);
     if (stats) {
         clear_stats(stats);

@@ -9,6 +9,7 @@
 #include <string>
 #include <vector>
 
+#include "device_budget.hpp"
 #include "srm_host.hpp"
 
 namespace scarf {
@@ -55,7 +56,7 @@ class TileTuner;
 
 class Device {
 public:
-    Device() = default;
+    Device();
     ~Device();
     Device(const Device &) = delete;
     Device &operator=(const Device &) = delete;
@@ -162,30 +163,35 @@ public:
     int last_nbx() const { return last_nbx_; }
     int last_tk() const { return last_tk_; }
 
-    // device bytes held by the library's grow-only buffers
-    size_t reserved_bytes() const { return reserved_; }
-    // device bytes the library holds in other buffers (FIM's), counted with
-    // these against SCARF_DEVICE_MEMORY_LIMIT
-    void set_external_reserved(size_t bytes) { external_ = bytes; }
-
 private:
     // Grows *ptr to `bytes` (keeps it when large enough). With
     // SCARF_DEVICE_MEMORY_LIMIT=<bytes> set, a call that would leave the
     // buffers holding more than that fails with an error instead, as a
     // failed hipMalloc does: the allocation-failure paths can be exercised.
-    bool reserve(void **ptr, size_t &cap, size_t bytes, std::string &err);
+    bool grow(void **ptr, size_t &cap, size_t bytes, std::string &err);
     // the same on a typed member: the pointer is written back whatever the
     // outcome (after a failed hipMalloc it is null, its capacity 0)
     template <class T>
-    bool reserve(T *&ptr, size_t &cap, size_t bytes, std::string &err)
+    bool reserve_if_room(T *&ptr, size_t &cap, size_t bytes, std::string &err)
     {
         void *p = ptr;
-        const bool ok = reserve(&p, cap, bytes, err);
+        const bool ok = grow(&p, cap, bytes, err);
         ptr = static_cast<T *>(p);
         return ok;
     }
-    size_t reserved_ = 0;
-    size_t external_ = 0;
+    // the same for a buffer that the call cannot do without: the library's
+    // spares make room for it
+    template <class T>
+    bool reserve(T *&ptr, size_t &cap, size_t bytes, std::string &err)
+    {
+        if (reserve_if_room(ptr, cap, bytes, err)) return true;
+        device_budget().drop_spares();
+        return reserve_if_room(ptr, cap, bytes, err);
+    }
+    // tables and statistics partials of a field pass, together
+    bool workspace(size_t table_bytes, size_t part_bytes, std::string &err);
+    // frees the buffers that hold nothing between two passes
+    void drop_scratch();
     // statistics, epilogue, field hand-over and timings after the field
     // kernels; slab_first/slab_points name the parts whose events are
     // slab_ev_. part/stat/poi: device room for the partials, the statistics

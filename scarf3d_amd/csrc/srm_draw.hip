@@ -20,6 +20,7 @@
 #include <cmath>
 #include <cstdlib>
 
+#include "device_budget.hpp"
 #include "fim_stream.hpp"
 
 namespace scarf {
@@ -176,22 +177,18 @@ __global__ __launch_bounds__(kThreads) void draw_order(int chunks, uint32_t reco
 
 }  // namespace
 
+TrialDevice::TrialDevice()
+{
+    device_budget().add_spare(this, [this] { drop(); });
+}
+
 TrialDevice::~TrialDevice()
 {
-    if (stream_) (void)hipStreamSynchronize(stream_);
-    void *dev[] = {d_gen_, d_limit_, d_out_};
-    for (void *p : dev)
-        if (p) (void)hipFree(p);
+    device_budget().remove_spare(this);
+    drop();
     if (h_out_) (void)hipHostFree(h_out_);
     if (h_limit_) (void)hipHostFree(h_limit_);
     if (stream_) (void)hipStreamDestroy(stream_);
-}
-
-bool TrialDevice::room(size_t bytes) const
-{
-    const char *e = std::getenv("SCARF_DEVICE_MEMORY_LIMIT");
-    const double limit = e ? std::atof(e) : 0.0;
-    return !(limit > 0 && double(elsewhere_ + reserved_ + bytes) > limit);
 }
 
 // words of the device's block: a span per chunk, the records; of the host's:
@@ -199,8 +196,27 @@ bool TrialDevice::room(size_t bytes) const
 static size_t device_words(size_t chunks, size_t records) { return (2 * chunks + 3) / 4 * 4 + kWords * records; }
 static size_t host_words(size_t records) { return 4 + (records + 3) / 4 * 4 + kRaw * records; }
 
+constexpr size_t kLimitBytes = (kBinsMax + 1) * sizeof(uint32_t);
+
+void TrialDevice::drop()
+{
+    if (stream_) (void)hipStreamSynchronize(stream_);
+    auto free = [](void *p, size_t bytes) {
+        if (!p) return;
+        (void)hipFree(p);
+        device_budget().give(bytes);
+    };
+    free(d_gen_, sizeof(GenTables));
+    free(d_limit_, kLimitBytes);
+    free(d_out_, device_words(chunks_, records_) * sizeof(uint32_t));
+    d_gen_ = nullptr;
+    d_limit_ = d_out_ = nullptr;
+    chunks_ = records_ = 0;
+}
+
 bool TrialDevice::reserve(size_t chunks, size_t records)
 {
+    DeviceBudget &budget = device_budget();
     auto ok = [](hipError_t e) {
         if (e == hipSuccess) return true;
         (void)hipGetLastError();  // leaves no error for the launch checks of other calls
@@ -208,7 +224,7 @@ bool TrialDevice::reserve(size_t chunks, size_t records)
     };
     if (!stream_ && !ok(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking))) return false;
     if (!d_gen_) {
-        if (!room(sizeof(GenTables))) return false;
+        if (!budget.fits(sizeof(GenTables))) return false;
         GenTables t;
         fim_stream::make_tables(t);
         void *g = nullptr;
@@ -218,15 +234,19 @@ bool TrialDevice::reserve(size_t chunks, size_t records)
             return false;
         }
         d_gen_ = g;
-        reserved_ += sizeof t;
+        budget.take(sizeof t);
     }
     if (!d_limit_) {
-        if (!room((kBinsMax + 1) * sizeof(uint32_t)) || !ok(hipMalloc(reinterpret_cast<void **>(&d_limit_), (kBinsMax + 1) * sizeof(uint32_t))))
-            return false;
-        reserved_ += (kBinsMax + 1) * sizeof(uint32_t);
+        void *p = nullptr;
+        if (!budget.fits(kLimitBytes) || !ok(hipMalloc(&p, kLimitBytes))) return false;
+        d_limit_ = static_cast<uint32_t *>(p);
+        budget.take(kLimitBytes);
     }
-    if (!h_limit_ && !ok(hipHostMalloc(reinterpret_cast<void **>(&h_limit_), (kBinsMax + 1) * sizeof(uint32_t), hipHostMallocDefault)))
-        return false;
+    if (!h_limit_) {
+        void *p = nullptr;
+        if (!ok(hipHostMalloc(&p, kLimitBytes, hipHostMallocDefault))) return false;
+        h_limit_ = static_cast<uint32_t *>(p);
+    }
     if (chunks <= chunks_ && records <= records_ && d_out_ && h_out_) return true;
     const size_t old = device_words(chunks_, records_) * sizeof(uint32_t);
     const size_t c = std::max(chunks, chunks_), r = std::max(records, records_);
@@ -235,22 +255,24 @@ bool TrialDevice::reserve(size_t chunks, size_t records)
         (void)hipStreamSynchronize(stream_);
         (void)hipFree(d_out_);
         d_out_ = nullptr;
-        reserved_ -= old;
+        budget.give(old);
     }
     if (h_out_) {
         (void)hipHostFree(h_out_);
         h_out_ = nullptr;
     }
     chunks_ = records_ = 0;
-    if (!room(bytes) || !ok(hipMalloc(reinterpret_cast<void **>(&d_out_), bytes))) return false;
-    if (!ok(hipHostMalloc(reinterpret_cast<void **>(&h_out_), host_words(r) * sizeof(uint32_t), hipHostMallocDefault))) {
-        (void)hipFree(d_out_);
-        d_out_ = nullptr;
+    void *d = nullptr, *h = nullptr;
+    if (!budget.fits(bytes) || !ok(hipMalloc(&d, bytes))) return false;
+    if (!ok(hipHostMalloc(&h, host_words(r) * sizeof(uint32_t), hipHostMallocDefault))) {
+        (void)hipFree(d);
         return false;
     }
+    d_out_ = static_cast<uint32_t *>(d);
+    h_out_ = static_cast<uint32_t *>(h);
     chunks_ = c;
     records_ = r;
-    reserved_ += bytes;
+    budget.take(bytes);
     return true;
 }
 

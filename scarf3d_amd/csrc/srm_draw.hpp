@@ -14,22 +14,17 @@ namespace scarf {
 
 class TrialDevice : public TrialScreen {
 public:
-    TrialDevice() = default;
+    TrialDevice();
     ~TrialDevice() override;
     TrialDevice(const TrialDevice &) = delete;
     TrialDevice &operator=(const TrialDevice &) = delete;
-
-    // device bytes held; `elsewhere`: those of the library's other buffers,
-    // counted with these against SCARF_DEVICE_MEMORY_LIMIT
-    size_t reserved_bytes() const { return reserved_; }
-    void set_elsewhere(size_t bytes) { elsewhere_ = bytes; }
 
     bool screen(int seed, long first, long count, const TrialTest &test, const uint32_t *limit, int bins,
                 TrialBlock &out) override;
 
 private:
     bool reserve(size_t pairs_chunks, size_t records);
-    bool room(size_t bytes) const;
+    void drop();  // the device's buffers; the last block of records stays in the host's memory
     hipStream_t stream_ = nullptr;
     void *d_gen_ = nullptr;      // generator tables
     uint32_t *d_limit_ = nullptr;  // and the count of records after it
@@ -37,7 +32,6 @@ private:
     uint32_t *h_out_ = nullptr;    // pinned, written by the device: total, pairs, raw outputs
     uint32_t *h_limit_ = nullptr;
     size_t chunks_ = 0, records_ = 0;
-    size_t reserved_ = 0, elsewhere_ = 0;
 };
 
 }  // namespace scarf

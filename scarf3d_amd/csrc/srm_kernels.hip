@@ -20,6 +20,7 @@
 #include <cstdlib>
 #include <string>
 
+#include "device_budget.hpp"
 #include "extent.hpp"
 #include "srm_device.hpp"
 #include "srm_mfma.hpp"
@@ -493,8 +494,42 @@ TileTuner &Device::tuner()
     return *tuner_;
 }
 
+DeviceBudget &device_budget()
+{
+    static DeviceBudget *b = new DeviceBudget;  // outlives every owner of a buffer
+    return *b;
+}
+
+bool DeviceBudget::fits(size_t more, std::string *err) const
+{
+    const char *e = std::getenv("SCARF_DEVICE_MEMORY_LIMIT");
+    const double limit = e ? std::atof(e) : 0.0;
+    if (!(limit > 0) || double(held_ + more) <= limit) return true;
+    if (err)
+        *err = "device memory limit SCARF_DEVICE_MEMORY_LIMIT=" + std::string(e) + " bytes: the library holds " +
+               std::to_string(held_) + " and would need " + std::to_string(held_ + more);
+    return false;
+}
+
+void DeviceBudget::remove_spare(const void *owner)
+{
+    spares_.erase(std::remove_if(spares_.begin(), spares_.end(), [&](const auto &s) { return s.first == owner; }),
+                  spares_.end());
+}
+
+void DeviceBudget::drop_spares()
+{
+    for (const auto &s : spares_) s.second();
+}
+
+Device::Device()
+{
+    device_budget().add_spare(this, [this] { drop_scratch(); });
+}
+
 Device::~Device()
 {
+    device_budget().remove_spare(this);
     if (device_ < 0) return;
     hipSetDevice(device_);
     if (stream_) hipStreamSynchronize(stream_);
@@ -536,30 +571,53 @@ bool Device::ensure(std::string &err)
     return true;
 }
 
-bool Device::reserve(void **ptr, size_t &cap, size_t bytes, std::string &err)
+bool Device::grow(void **ptr, size_t &cap, size_t bytes, std::string &err)
 {
-    const bool grow = !(bytes <= cap && *ptr);
-    if (const char *e = std::getenv("SCARF_DEVICE_MEMORY_LIMIT")) {
-        const double limit = std::atof(e);
-        const size_t after = reserved_ + external_ + (grow ? bytes - std::min(bytes, cap) : 0);
-        if (limit > 0 && double(after) > limit) {
-            err = "device memory limit SCARF_DEVICE_MEMORY_LIMIT=" + std::string(e) + " bytes: the library holds " +
-                  std::to_string(reserved_ + external_) + " and would need " + std::to_string(after);
-            return false;
-        }
-    }
-    if (!grow) return true;
+    const bool larger = !(bytes <= cap && *ptr);
+    if (!device_budget().fits(larger ? bytes - std::min(bytes, cap) : 0, &err)) return false;
+    if (!larger) return true;
     if (*ptr) {
         HIP_TRY(hipStreamSynchronize(stream_));
         HIP_TRY(hipFree(*ptr));
         *ptr = nullptr;
-        reserved_ -= cap;
+        device_budget().give(cap);
         cap = 0;
     }
-    HIP_TRY(hipMalloc(ptr, std::max<size_t>(bytes, 256)));
+    const hipError_t e = hipMalloc(ptr, std::max<size_t>(bytes, 256));
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // leaves no error for the launch checks of other calls
+        *ptr = nullptr;
+        err = "hipMalloc of " + std::to_string(bytes) + " bytes: " + hipGetErrorString(e);
+        return false;
+    }
     cap = bytes;
-    reserved_ += cap;
+    device_budget().take(cap);
     return true;
+}
+
+void Device::drop_scratch()
+{
+    auto drop = [&](auto &ptr, size_t &cap) {
+        if (!ptr) return;
+        (void)hipStreamSynchronize(stream_);
+        (void)hipFree(ptr);
+        ptr = nullptr;
+        device_budget().give(cap);
+        cap = 0;
+    };
+    drop(d_tab_, tab_cap_);
+    drop(d_part_, part_cap_);
+    drop(d_member_, member_cap_);
+}
+
+bool Device::workspace(size_t table_bytes, size_t part_bytes, std::string &err)
+{
+    auto both = [&] {
+        return reserve_if_room(d_tab_, tab_cap_, table_bytes, err) && reserve_if_room(d_part_, part_cap_, part_bytes, err);
+    };
+    if (both()) return true;
+    device_budget().drop_spares();
+    return both();
 }
 
 void *Device::field_buffer(size_t bytes, std::string &err)
@@ -625,8 +683,9 @@ bool Device::reserve_members(const std::vector<Member> &members)
         work = std::max(work, plan.bytes);
         parts = std::max(parts, size_t(3) * (plan.nparts + plan.groups));
     }
-    ok = stage_record(staged, err) && reserve(d_member_, member_cap_, rec, err) && reserve(d_tab_, tab_cap_, work, err) &&
-         reserve(d_part_, part_cap_, (parts + 6 * members.size()) * sizeof(double), err);
+    ok = stage_record(staged, err) && reserve_if_room(d_member_, member_cap_, rec, err) &&
+         reserve_if_room(d_tab_, tab_cap_, work, err) &&
+         reserve_if_room(d_part_, part_cap_, (parts + 6 * members.size()) * sizeof(double), err);
     if (!ok) (void)hipGetLastError();
     return ok;
 }
@@ -764,17 +823,15 @@ bool Device::run(const Geometry &g, int kernel, double scaling, const Epilogue &
         const bool f64 = sizeof(Real) == sizeof(double);
         if (npts_ != npts || !points_plan(pts_lo_, pts_hi_, wmax_, g.flat, npts, np_, f64, points) ||
             !(points_ms(points, f64) < points_direct_ms(npts, np_, otherwise == kKernelDirectF64)) ||
-            !reserve(d_tab_, tab_cap_, points.bytes, err) ||
-            !reserve(d_part_, part_cap_, size_t(3) * points.nparts * sizeof(double), err)) {
-            (void)hipGetLastError();  // a refused allocation
+            !reserve_if_room(d_tab_, tab_cap_, points.bytes, err) ||
+            !reserve_if_room(d_part_, part_cap_, size_t(3) * points.nparts * sizeof(double), err)) {
             err.clear();
             kernel = otherwise;
         }
     } else if (kernel == kKernelTransform) {
         if (!transform_plan(g, np_, sizeof(Real) == sizeof(double), transform) ||
-            !reserve(d_tab_, tab_cap_, transform.bytes, err) ||
-            !reserve(d_part_, part_cap_, size_t(3) * (transform.nparts + transform.groups) * sizeof(double), err)) {
-            (void)hipGetLastError();  // a refused allocation
+            !reserve_if_room(d_tab_, tab_cap_, transform.bytes, err) ||
+            !reserve_if_room(d_part_, part_cap_, size_t(3) * (transform.nparts + transform.groups) * sizeof(double), err)) {
             err.clear();
             kernel = otherwise;
         }
@@ -801,9 +858,8 @@ bool Device::run(const Geometry &g, int kernel, double scaling, const Epilogue &
             last_nbx_ = plan.nbx;
             last_tk_ = plan.tk;
             plan.zscale = mfma_zscale(kernel, amp_max_);
-            if (!reserve(d_tab_, tab_cap_, plan.table_bytes, err)) return false;
             nparts = plan.nparts;
-            if (!reserve(d_part_, part_cap_, size_t(3) * nparts * sizeof(double), err)) return false;
+            if (!workspace(plan.table_bytes, size_t(3) * nparts * sizeof(double), err)) return false;
             if (!mfma_tables(plan, g, d_harm_, np_, d_tab_, stream_, err)) return false;
             HIP_TRY(hipEventRecord(ev_[1], stream_));
             if (on_slab && !ep.active() && plan.tiles_k > 1) {
@@ -835,11 +891,10 @@ bool Device::run(const Geometry &g, int kernel, double scaling, const Epilogue &
             const bool f64 = kernel == kKernelDirectF64;
             const size_t elt = f64 ? sizeof(double) : sizeof(float);
             const size_t tab_bytes = size_t(np_) * (size_t(g.nx) + g.ny + g.nz) * elt + size_t(np_) * sizeof(float);
-            if (!reserve(d_tab_, tab_cap_, tab_bytes, err)) return false;
             const int tiles_i = int((g.nx + kDirB - 1) / kDirB);
             const long tiles_c = (long(g.ny) * g.nz + kDirB - 1) / kDirB;
             nparts = int(tiles_i * tiles_c);
-            if (!reserve(d_part_, part_cap_, size_t(3) * nparts * sizeof(double), err)) return false;
+            if (!workspace(tab_bytes, size_t(3) * nparts * sizeof(double), err)) return false;
             const long tab_elems = long(np_) * (g.nx + g.ny + g.nz);
             const int tblocks = int(std::min<long>((tab_elems + 255) / 256, 65536));
             if (f64) {
@@ -1087,9 +1142,8 @@ bool Device::run_streamed(const Geometry &g, int kernel, int nharm, double scali
     if (!reserve(d_harm_, harm_cap_, rec_bytes, err)) return false;
     nharm_ = 0;  // the streamed record is not a resident table for run()
     if (!stage_record(rec_bytes, err)) return false;
-    if (!reserve(d_tab_, tab_cap_, plan.table_bytes, err)) return false;
     const int nparts = plan.nparts;
-    if (!reserve(d_part_, part_cap_, size_t(3) * nparts * sizeof(double), err)) return false;
+    if (!workspace(plan.table_bytes, size_t(3) * nparts * sizeof(double), err)) return false;
 
     timings_ = Timings{};
     HIP_TRY(hipEventRecord(ev_[0], stream_));
