@@ -188,6 +188,8 @@ private:
         device_budget().drop_spares();
         return reserve_if_room(ptr, cap, bytes, err);
     }
+    template <class Real>
+    bool upload_widened(const Real *const (&axes)[3], long n, std::string &err);
     // tables and statistics partials of a field pass, together
     bool workspace(size_t table_bytes, size_t part_bytes, std::string &err);
     // frees the buffers that hold nothing between two passes

@@ -756,20 +756,22 @@ __global__ __launch_bounds__(256) void clear(double *__restrict__ dst, long n)
 // The caller's thread reads them: with a pool's threads a call is as fast
 // (3.2 against 3.3 ms), and the caller's next writes to its arrays are slower
 // (their lines sit in other cores' caches: +5 to 10 ms for new coordinates).
+// Without device room for the raw coordinates they are widened on the host.
 template <class Real>
 bool Device::upload_points(const Real *x, const Real *y, const Real *z, long n, std::string &err)
 {
     npts_ = 0;
     const size_t total = size_t(z ? 3 : 2) * n;
     if (!reserve(d_pts_, pts_cap_, size_t(3) * n * sizeof(double), err)) return false;
-    if (!reserve(d_tab_, tab_cap_, total * sizeof(Real), err)) return false;
+    const Real *axes[3] = {x, y, z};
+    std::string no_room;
+    if (!reserve_if_room(d_tab_, tab_cap_, total * sizeof(Real), no_room)) return upload_widened(axes, n, err);
     if (!h_pts_) {
         for (auto &e : pts_ev_)
             if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&h_pts_), kPointStages * kPointStage, hipHostMallocDefault));
     }
     HIP_TRY(hipStreamSynchronize(stream_));  // the ring is free
-    const Real *axes[3] = {x, y, z};
     const size_t chunk = kPointStage / sizeof(Real);
     long piece = 0;
     for (int d = 0; d < 3; ++d) {
@@ -798,6 +800,25 @@ bool Device::upload_points(const Real *x, const Real *y, const Real *z, long n, 
         clear<<<blocks, 256, 0, stream_>>>(d_pts_ + 2 * size_t(n), n);
         HIP_TRY(hipGetLastError());
     }
+    npts_ = n;
+    return true;
+}
+
+template <class Real>
+bool Device::upload_widened(const Real *const (&axes)[3], long n, std::string &err)
+{
+    std::vector<double> pts(size_t(3) * n);
+    for (int d = 0; d < 3; ++d) {
+        pts_lo_[d] = pts_hi_[d] = 0.0;
+        if (!axes[d]) continue;
+        std::copy(axes[d], axes[d] + n, pts.begin() + size_t(d) * n);
+        Real lo = axes[d][0], hi = axes[d][0];
+        add_extent(axes[d], size_t(n), lo, hi);
+        pts_lo_[d] = lo;
+        pts_hi_[d] = hi;
+    }
+    HIP_TRY(hipMemcpyAsync(d_pts_, pts.data(), pts.size() * sizeof(double), hipMemcpyHostToDevice, stream_));
+    HIP_TRY(hipStreamSynchronize(stream_));
     npts_ = n;
     return true;
 }
