@@ -223,8 +223,10 @@ private:
     bool queue_record(const HarmonicRows &t, int np_, double *staged, double *record, std::string &err);
     double *d_member_ = nullptr;  // record of run_members (the resident one stays)
     size_t member_cap_ = 0;
-    double *h_rec_ = nullptr;  // pinned staging of the record
+    double *h_rec_ = nullptr;  // staging of the record
     size_t h_rec_cap_ = 0;
+    std::unique_ptr<double[]> pageable_rec_;  // holds it where pinned memory is refused
+    void drop_record_stage();
     // per-axis tables (FP32 or FP64 revolutions, operand tables of the GEMM)
     void *d_tab_ = nullptr;
     size_t tab_cap_ = 0;

@@ -537,7 +537,7 @@ Device::~Device()
     for (void *b : bufs)
         if (b) hipFree(b);
     if (h_stat_) hipHostFree(h_stat_);
-    if (h_rec_) hipHostFree(h_rec_);
+    drop_record_stage();
     if (h_pts_) hipHostFree(h_pts_);
     for (auto &e : pts_ev_)
         if (e) hipEventDestroy(e);
@@ -626,18 +626,31 @@ void *Device::field_buffer(size_t bytes, std::string &err)
     return d_field_;
 }
 
-// Pinned room for a record, free to be written: the copies queued from it
-// have run.
+// Host room for a record, free to be written: the copies queued from it have
+// run. Pinned, or pageable where pinned memory is refused.
 bool Device::stage_record(size_t bytes, std::string &err)
 {
     HIP_TRY(hipStreamSynchronize(stream_));
     if (h_rec_cap_ >= bytes) return true;
-    if (h_rec_) HIP_TRY(hipHostFree(h_rec_));
-    h_rec_ = nullptr;
-    h_rec_cap_ = 0;
-    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&h_rec_), bytes, hipHostMallocDefault));
+    drop_record_stage();
+    void *p = nullptr;
+    if (hipHostMalloc(&p, bytes, hipHostMallocDefault) == hipSuccess) {
+        h_rec_ = static_cast<double *>(p);
+    } else {
+        (void)hipGetLastError();  // leaves no error for the launch checks of other calls
+        pageable_rec_.reset(new double[(bytes + sizeof(double) - 1) / sizeof(double)]);
+        h_rec_ = pageable_rec_.get();
+    }
     h_rec_cap_ = bytes;
     return true;
+}
+
+void Device::drop_record_stage()
+{
+    if (h_rec_ && !pageable_rec_) (void)hipHostFree(h_rec_);
+    pageable_rec_.reset();
+    h_rec_ = nullptr;
+    h_rec_cap_ = 0;
 }
 
 bool Device::queue_record(const HarmonicRows &t, int np_, double *staged, double *record, std::string &err)
@@ -756,7 +769,8 @@ __global__ __launch_bounds__(256) void clear(double *__restrict__ dst, long n)
 // The caller's thread reads them: with a pool's threads a call is as fast
 // (3.2 against 3.3 ms), and the caller's next writes to its arrays are slower
 // (their lines sit in other cores' caches: +5 to 10 ms for new coordinates).
-// Without device room for the raw coordinates they are widened on the host.
+// Without device room for the raw coordinates, or pinned memory, they are
+// widened on the host.
 template <class Real>
 bool Device::upload_points(const Real *x, const Real *y, const Real *z, long n, std::string &err)
 {
@@ -764,13 +778,18 @@ bool Device::upload_points(const Real *x, const Real *y, const Real *z, long n, 
     const size_t total = size_t(z ? 3 : 2) * n;
     if (!reserve(d_pts_, pts_cap_, size_t(3) * n * sizeof(double), err)) return false;
     const Real *axes[3] = {x, y, z};
-    std::string no_room;
-    if (!reserve_if_room(d_tab_, tab_cap_, total * sizeof(Real), no_room)) return upload_widened(axes, n, err);
     if (!h_pts_) {
         for (auto &e : pts_ev_)
             if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&h_pts_), kPointStages * kPointStage, hipHostMallocDefault));
+        void *p = nullptr;
+        if (hipHostMalloc(&p, kPointStages * kPointStage, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            return upload_widened(axes, n, err);
+        }
+        h_pts_ = static_cast<char *>(p);
     }
+    std::string no_room;
+    if (!reserve_if_room(d_tab_, tab_cap_, total * sizeof(Real), no_room)) return upload_widened(axes, n, err);
     HIP_TRY(hipStreamSynchronize(stream_));  // the ring is free
     const size_t chunk = kPointStage / sizeof(Real);
     long piece = 0;
