@@ -710,14 +710,17 @@ bool Device::run_members(const std::vector<Member> &members, const MemberDraw &d
     const size_t n = members.size();
     double *staged = h_rec_, *stat = d_part_ + part_cap_ / sizeof(double) - 6 * n;
     HIP_TRY(hipSetDevice(device_));
+    // whichever way the call ends, an error or a draw's exception among them,
+    // nothing is left in flight: the fields are the caller's
+    struct Drain {
+        hipStream_t stream;
+        ~Drain() { (void)hipStreamSynchronize(stream); }
+    } drain{stream_};
     HIP_TRY(hipEventRecord(ev_[0], stream_));
     for (size_t q = 0; q < n; ++q) {
         const Member &m = members[q];
         HarmonicRows t;
-        if (!draw(static_cast<int>(q), t, err)) {
-            (void)hipStreamSynchronize(stream_);
-            return false;
-        }
+        if (!draw(static_cast<int>(q), t, err)) return false;
         const int np_ = static_cast<int>(round_up(std::max(t.n, 1), kHarmPad));
         TransformPlan plan;
         if (t.n > m.nharm || !transform_plan(m.g, np_, sizeof(Real) == sizeof(double), plan)) {
