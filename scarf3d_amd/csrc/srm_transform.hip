@@ -747,11 +747,13 @@ bool transform_plan(const Geometry &g, int np_, bool f64, TransformPlan &plan)
     p.yb = 16;
     while (p.yb > 1 && size_t(p.yb) * p.m * csize > kLineBytes) p.yb /= 2;
     while (p.yb > 1 && p.yb / 2 >= g.ny) p.yb /= 2;
-    // planes per round: eight blocks' worth, more while the intermediate stays small
-    const size_t plane = size_t(p.columns) * p.ny * csize;
+    // planes per round: eight blocks' worth, more while the intermediate and
+    // the harmonics' values (which outgrow it on thin blocks) stay small
+    const size_t plane = size_t(p.columns) * p.ny * csize, values = size_t(np_) * csize;
     const int zmax = (g.nz + p.zb - 1) / p.zb * p.zb;
     p.slab = 8 * p.zb;
-    while (p.slab < zmax && plane * p.slab * 2 <= (size_t(192) << 20)) p.slab *= 2;
+    while (p.slab < zmax && plane * p.slab * 2 <= (size_t(192) << 20) && values * p.slab * 2 <= (size_t(256) << 20))
+        p.slab *= 2;
     p.slab = std::min(p.slab, zmax);
     // short lines: more of them per block, as long as the blocks still fill the device
     while (p.yb >= 16 && p.yb < 256 && 2 * p.yb * p.m <= 4096 && long(g.nz) * g.ny / (2 * p.yb) >= 1024) p.yb *= 2;
