@@ -34,6 +34,7 @@ constexpr int kThreads = 512;
 constexpr int kWaves = kThreads / 64;
 constexpr int kBinsMax = 4096;
 constexpr int kRaw = TrialBlock::kRaw, kWords = kRaw + 1;
+constexpr double kMostRecords = 1 << 20;  // expected ones, of a block
 constexpr int kGroup = 64;  // chunks that a block puts in order
 
 struct ScreenArgs {
@@ -287,6 +288,9 @@ bool TrialDevice::screen(int seed, long first, long count, const TrialTest &test
         return false;
     double share = 0.0;
     for (int b = 0; b < bins; ++b) share += std::min(1.0, double(limit[b]) / Yarn2::kModulus) / bins;
+    // the records of a block take 36 bytes each here and in pinned memory: a
+    // long draw takes several blocks
+    if (share * double(count) > kMostRecords) count = std::max(4L, static_cast<long>(kMostRecords / share));
     const double mean = share * double(count);
     const int rounds = static_cast<int>(std::clamp(count / (64L * 1024), 1L, long(kRounds)));
     const size_t chunks = size_t((count + 64L * rounds - 1) / (64L * rounds));

@@ -99,8 +99,8 @@ struct TrialTest {
 // threads. A pair is held when its second output is below limit[b], b the
 // first output's bin of 2^31 / bins values, and gets kReject, kKeep or kDrop
 // (above kc) where the test's roundings cannot decide it, kUnsure otherwise.
-// The block stays valid until the next call. False: not possible now (the draw
-// then screens for itself).
+// A block may end before first + count; it stays valid until the next call.
+// False: not possible now (the draw then screens for itself).
 class TrialScreen {
 public:
     virtual ~TrialScreen() = default;
