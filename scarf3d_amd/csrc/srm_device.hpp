@@ -221,6 +221,7 @@ private:
     // rows, zero-padded to np_ per field, to a device record by way of their
     // place in the staging memory
     bool queue_record(const HarmonicRows &t, int np_, double *staged, double *record, std::string &err);
+    static constexpr size_t kMemberStage = size_t(64) << 20;  // of an ensemble's records at a time
     double *d_member_ = nullptr;  // record of run_members (the resident one stays)
     size_t member_cap_ = 0;
     double *h_rec_ = nullptr;  // staging of the record

@@ -684,7 +684,7 @@ bool Device::upload_table(const HarmonicRows &t, std::string &err)
 template <class Real>
 bool Device::reserve_members(const std::vector<Member> &members)
 {
-    size_t rec = 0, staged = 0, work = 0, parts = 0;
+    size_t rec = 0, all = 0, work = 0, parts = 0;
     std::string err;
     bool ok = hipSetDevice(device_) == hipSuccess;
     for (const Member &m : members) {
@@ -692,11 +692,11 @@ bool Device::reserve_members(const std::vector<Member> &members)
         const int np_ = static_cast<int>(round_up(std::max(m.nharm, 1), kHarmPad));
         if (!ok || !transform_plan(m.g, np_, sizeof(Real) == sizeof(double), plan)) return false;
         rec = std::max(rec, size_t(5) * np_ * sizeof(double));
-        staged += size_t(5) * np_ * sizeof(double);
+        all += size_t(5) * np_ * sizeof(double);
         work = std::max(work, plan.bytes);
         parts = std::max(parts, size_t(3) * (plan.nparts + plan.groups));
     }
-    ok = stage_record(staged, err) && reserve_if_room(d_member_, member_cap_, rec, err) &&
+    ok = stage_record(std::min(all, std::max(rec, kMemberStage)), err) && reserve_if_room(d_member_, member_cap_, rec, err) &&
          reserve_if_room(d_tab_, tab_cap_, work, err) &&
          reserve_if_room(d_part_, part_cap_, (parts + 6 * members.size()) * sizeof(double), err);
     if (!ok) (void)hipGetLastError();
@@ -728,6 +728,10 @@ bool Device::run_members(const std::vector<Member> &members, const MemberDraw &d
             return false;
         }
         Real *field = static_cast<Real *>(m.d_field);
+        if (staged + size_t(5) * np_ > h_rec_ + h_rec_cap_ / sizeof(double)) {  // full: once the copies have run
+            HIP_TRY(hipStreamSynchronize(stream_));
+            staged = h_rec_;
+        }
         if (!queue_record(t, np_, staged, d_member_, err) ||
             !transform_field<Real>(plan, m.g, d_member_, d_tab_, m.scaling, field, d_part_, stream_, ev_[1], err))
             return false;
