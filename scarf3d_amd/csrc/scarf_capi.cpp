@@ -688,6 +688,7 @@ void scarf_finalize(void)
     s.cfg = SrmConfig{};
     s.x = s.y = s.z = nullptr;
     s.error.clear();
+    if (s.device) s.device->give_back();
 }
 
 // Single-writer versions of write_one / write_slice (src/scarflib_common.f90:245-418,

@@ -610,8 +610,14 @@ void Device::drop_scratch()
     drop(d_member_, member_cap_);
 }
 
+void Device::give_back()
+{
+    if (tab_cap_ > std::max(tab_grids_, kKeepWorkspace)) drop_scratch();
+}
+
 bool Device::workspace(size_t table_bytes, size_t part_bytes, std::string &err)
 {
+    tab_grids_ = std::max(tab_grids_, table_bytes);
     auto both = [&] {
         return reserve_if_room(d_tab_, tab_cap_, table_bytes, err) && reserve_if_room(d_part_, part_cap_, part_bytes, err);
     };
@@ -881,6 +887,8 @@ bool Device::run(const Geometry &g, int kernel, double scaling, const Epilogue &
             !reserve_if_room(d_part_, part_cap_, size_t(3) * (transform.nparts + transform.groups) * sizeof(double), err)) {
             err.clear();
             kernel = otherwise;
+        } else {
+            tab_grids_ = std::max(tab_grids_, transform.bytes);
         }
     }
     const bool mfma = g.structured && (kernel == kKernelMfmaBf16x3 || kernel == kKernelMfmaF16x2 ||

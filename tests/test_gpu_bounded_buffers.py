@@ -1,5 +1,6 @@
 """Buffers that outlive a call are bounded: records of long draws come in
-blocks, an ensemble's records go up 64 MiB at a time.
+blocks, an ensemble's records go up 64 MiB at a time, a point list's large
+workspace is given back.
 
 Tolerance of the draw, before any run: FP64 sums of 1.2e6 harmonics at phases
 below 1e4 rad, 1e-10 sigma."""
@@ -8,6 +9,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
+from native_lib import build_check, run_check
 from scarf3d_amd.hip import Hip
 from srm_cases import init_product, oracle_field, structured_cfg
 
@@ -51,3 +53,9 @@ def test_an_ensemble_of_more_records_than_are_staged_at_a_time(lib_f):
         lib_f.finalize()
         assert np.array_equal(bufs[q].numpy(), single.reshape(-1, order="F")), q
         assert np.array_equal(stats[q, :4], one[:4]), q
+
+
+def test_a_lists_large_workspace_is_given_back(tmp_path):
+    out = run_check(build_check("give_back", tmp_path))
+    print(out, flush=True)
+    assert out.rstrip().endswith("0 bad")
