@@ -105,7 +105,7 @@ scarf::WorkerPool &drain_pool()
     return *p;
 }
 
-// ensemble members' host draws: one member per thread at a time
+// ensemble members' setups and short draws: one member per thread at a time
 scarf::WorkerPool &member_pool()
 {
     static scarf::WorkerPool *p = new scarf::WorkerPool(
@@ -910,14 +910,53 @@ static int scarf_ensemble_execute_body(int n, const struct scarf_member *members
     for (int m = 0; m < n; ++m)
         if (!errs[m].empty()) return fail("member " + std::to_string(m) + ": " + errs[m]);
     if (!ensure_device()) return -1;
-    // A member's draw: trials screened on the GPU, exact tests and harmonics
-    // on every worker, so members follow one another.
-    auto draw_member = [&](int m) {
+    // Draws: short ones side by side on one thread each, the others one after
+    // the other, trials screened on the GPU and the rest on every worker.
+    const int threads = member_pool().size();
+    std::vector<scarf::DrawCost> cost(n);
+    for (int m = 0; m < n; ++m) cost[m] = scarf::draw_cost(cfgs[m].nharm, setups[m]);
+    const std::vector<char> side = scarf::draws_side_by_side(cost, threads);
+    std::vector<char> done(n, 0);
+    std::unique_ptr<scarf::HarmonicSampler> held;  // of a member whose rows are read from it
+    std::vector<int> kept(n, 0);
+    auto draw_one = [&](int m, bool alone, bool hold) {
         const auto t0 = std::chrono::steady_clock::now();
-        std::unique_ptr<scarf::HarmonicSampler> w = sampler(cfgs[m], setups[m], members[m].seed);
-        w->draw_until(INT_MAX);
+        std::unique_ptr<scarf::HarmonicSampler> w =
+            alone ? scarf::HarmonicSampler::create_rows<real>(cfgs[m], setups[m], members[m].seed, nullptr, 1)
+                  : sampler(cfgs[m], setups[m], members[m].seed);
+        kept[m] = w->draw_until(INT_MAX);
+        if (hold) {
+            held = std::move(w);
+        } else {
+            const scarf::HarmonicRows t = w->rows(0, kept[m]);
+            const size_t np_ = nps[m] = std::max(64, (kept[m] + 63) / 64 * 64);
+            records[m].assign(5 * np_, 0.0);
+            for (int f = 0; f < 5; ++f) std::copy(t.field[f], t.field[f] + t.n, records[m].begin() + f * np_);
+        }
+        done[m] = 1;
         host_s[m] += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-        return w;
+    };
+    // draws member m, and with it the next short draws, up to `most` of them
+    auto draw_member = [&](int m, int most, bool hold, std::string &e) {
+        if (done[m]) return true;
+        if (!side[m]) {
+            draw_one(m, false, hold);
+            return true;
+        }
+        std::vector<int> batch;
+        for (int q = m; q < n && static_cast<int>(batch.size()) < most; ++q)
+            if (side[q] && !done[q]) batch.push_back(q);
+        std::atomic<size_t> at{0};
+        const std::function<void(int)> job = [&](int) {
+            for (size_t q = at++; q < batch.size(); q = at++) guard(batch[q], [&] { draw_one(batch[q], true, false); });
+        };
+        member_pool().run(job);
+        for (int q : batch)
+            if (!errs[q].empty()) {
+                e = "member " + std::to_string(q) + ": " + errs[q];
+                return false;
+            }
+        return true;
     };
     std::vector<double> st;
     double ms = 0;
@@ -926,9 +965,15 @@ static int scarf_ensemble_execute_body(int n, const struct scarf_member *members
     // each drawn while the device computes the one before, where that is
     // faster than all draws followed by the grouped launch (5e10 points and
     // harmonics per ms, at least 8e-5 ms per harmonic of the longest member).
-    // Draws: measured 0.15 ms and 2.5e-5 ms per harmonic.
     bool transform = choose;
-    double by_transform = 0, draws = 0, work = 0, longest = 0;
+    double by_transform = 0, draws = 0, work = 0, longest = 0, alone = 0;
+    int sides = 0;
+    for (int m = 0; m < n; ++m) {
+        if (!side[m]) draws += cost[m].screened;
+        else alone += cost[m].alone;
+        sides += side[m];
+    }
+    if (sides > 0) draws += alone / std::min(sides, threads);
     std::vector<scarf::Device::Member> tm(transform ? n : 0);
     for (int m = 0; transform && m < n; ++m) {
         tm[m].g = geometry(cfgs[m]);
@@ -940,28 +985,27 @@ static int scarf_ensemble_execute_body(int n, const struct scarf_member *members
         scarf::TransformPlan plan;
         transform = scarf::transform_plan(tm[m].g, (cfgs[m].nharm + 63) / 64 * 64, kDouble, plan);
         by_transform += scarf::transform_ms(plan, kDouble);
-        draws += 0.15 + 2.5e-5 * cfgs[m].nharm;
         work += double(tm[m].g.points()) * cfgs[m].nharm;
         longest = std::max(longest, double(cfgs[m].nharm));
     }
     const double grouped = draws + 0.1 + std::max(work / 5e10, 8e-5 * longest);
     if (transform && std::max(by_transform, draws) < grouped && s.device->reserve_members<real>(tm)) {
-        std::unique_ptr<scarf::HarmonicSampler> w;
-        const scarf::Device::MemberDraw draw = [&](int m, scarf::HarmonicRows &rows, std::string &) {
-            w.reset();  // its lease of the workers ends before the next draw
-            w = draw_member(m);
-            rows = w->rows(0, w->draw_until(INT_MAX));
+        const scarf::Device::MemberDraw draw = [&](int m, scarf::HarmonicRows &rows, std::string &e) {
+            held.reset();  // its lease of the workers ends before the next draw
+            if (m > 0) std::vector<double>().swap(records[m - 1]);
+            if (!draw_member(m, 2 * threads, true, e)) return false;
+            if (held) {
+                rows = held->rows(0, kept[m]);
+            } else {
+                for (int f = 0; f < 5; ++f) rows.field[f] = records[m].data() + size_t(f) * nps[m];
+                rows.n = kept[m];
+            }
             return true;
         };
         if (!s.device->run_members<real>(tm, draw, st, ms, err)) return fail(err);
     } else {
-        for (int m = 0; m < n; ++m) {
-            const std::unique_ptr<scarf::HarmonicSampler> w = draw_member(m);
-            const scarf::HarmonicRows t = w->rows(0, w->draw_until(INT_MAX));
-            nps[m] = std::max(64, (t.n + 63) / 64 * 64);
-            records[m].assign(size_t(5) * nps[m], 0.0);
-            for (int f = 0; f < 5; ++f) std::copy(t.field[f], t.field[f] + t.n, records[m].begin() + size_t(f) * nps[m]);
-        }
+        for (int m = 0; m < n; ++m)
+            if (!draw_member(m, n, false, err)) return fail(err);
         if (ensemble_grouped(cfgs, setups, records, nps, d_fields, kernel, st, ms) != 0) return -1;
     }
     s.ensemble_ms = ms;

@@ -141,6 +141,21 @@ public:
 // SCARF_DRAW_THREADS if set, else min(16, hardware threads)
 int default_draw_threads();
 
+// Pairs of the stream that a draw is expected to consume: nharm over the mean
+// acceptance of the rejection test, and the three after each trial that passes.
+double expected_trials(const SrmSetup &setup);  // per harmonic
+double expected_pairs(int nharm, const SrmSetup &setup);
+
+// Estimated milliseconds of a draw on one thread, and of one on all threads
+// with its trials screened on the GPU where that pays.
+struct DrawCost {
+    double alone = 0, screened = 0;
+};
+DrawCost draw_cost(int nharm, const SrmSetup &setup);
+// Which of several draws run side by side on one thread each: the others follow
+// one another, screened.
+std::vector<char> draws_side_by_side(const std::vector<DrawCost> &cost, int threads);
+
 // device records of a whole draw by create(): what create_rows() is checked against
 HarmonicTable build_table(const SrmSetup &setup, const HarmonicDraw &draw);
 
