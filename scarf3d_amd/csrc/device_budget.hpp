@@ -4,6 +4,8 @@
 // spares: they are given back when another buffer finds no room, so that a
 // call needs no more room than what it computes from.
 #pragma once
+#include <hip/hip_runtime.h>
+
 #include <cstddef>
 #include <functional>
 #include <string>
@@ -33,5 +35,9 @@ private:
 };
 
 DeviceBudget &device_budget();
+
+// hipMalloc of a buffer outside the account, the spares making room where the
+// device has none left; leaves no error for the launch checks of other calls
+hipError_t malloc_with_spares(void **ptr, size_t bytes);
 
 }  // namespace scarf

@@ -631,8 +631,16 @@ bool FimDevice::run(const FimSetup<Real> &s, int rescale, double mute, double ta
         if (!m.plans || m.plan_n[0] != n1 || m.plan_n[1] != n2 || m.plan_n[2] != n3 ||
             m.plan_real != int(sizeof(Real))) {
             m.drop_plans();
-            const hipfftResult r = n3 > 1 ? hipfftPlan3d(&m.plan, n3, n2, n1, FftTypes<Real>::c2r)
-                                          : hipfftPlan2d(&m.plan, n2, n1, FftTypes<Real>::c2r);
+            auto make = [&] {
+                return n3 > 1 ? hipfftPlan3d(&m.plan, n3, n2, n1, FftTypes<Real>::c2r)
+                              : hipfftPlan2d(&m.plan, n2, n1, FftTypes<Real>::c2r);
+            };
+            hipfftResult r = make();
+            if (r != HIPFFT_SUCCESS) {  // no room for its work buffer: the library's spares make some
+                (void)hipGetLastError();
+                device_budget().drop_spares();
+                r = make();
+            }
             if (!fft_ok(r, "hipfftPlan (c2r)")) return false;
             m.plans = true;
             m.plan_n[0] = n1;

@@ -522,6 +522,19 @@ void DeviceBudget::drop_spares()
     for (const auto &s : spares_) s.second();
 }
 
+hipError_t malloc_with_spares(void **ptr, size_t bytes)
+{
+    hipError_t e = hipMalloc(ptr, bytes);
+    if (e == hipSuccess) return e;
+    (void)hipGetLastError();
+    device_budget().drop_spares();
+    e = hipMalloc(ptr, bytes);
+    if (e == hipSuccess) return e;
+    (void)hipGetLastError();
+    *ptr = nullptr;
+    return e;
+}
+
 Device::Device()
 {
     device_budget().add_spare(this, [this] { drop_scratch(); });

@@ -30,6 +30,7 @@
 #include <utility>
 #include <vector>
 
+#include "device_budget.hpp"
 #include "srm_mfma.hpp"
 #include "srm_stats.hpp"
 
@@ -1119,12 +1120,12 @@ bool Ensemble::run(hipStream_t stream, int kernel, const std::vector<EnsembleMem
         release();
         ENS_TRY(hipEventCreate(&ev_[0]));
         ENS_TRY(hipEventCreate(&ev_[1]));
-        ENS_TRY(hipMalloc(&d_rec_, rec_total * sizeof(double)));
-        ENS_TRY(hipMalloc(&d_tab_, std::max<size_t>(tab_total, 256)));
-        ENS_TRY(hipMalloc(&d_part_, size_t(3) * parts_total * sizeof(double)));
-        ENS_TRY(hipMalloc(&d_desc_, size_t(n) * sizeof(MemberDesc)));
-        ENS_TRY(hipMalloc(&d_items_, costed.size() * sizeof(int2)));
-        ENS_TRY(hipMalloc(&d_stat_, size_t(6) * n * sizeof(double)));
+        ENS_TRY(malloc_with_spares(&d_rec_, rec_total * sizeof(double)));
+        ENS_TRY(malloc_with_spares(&d_tab_, std::max<size_t>(tab_total, 256)));
+        ENS_TRY(malloc_with_spares(&d_part_, size_t(3) * parts_total * sizeof(double)));
+        ENS_TRY(malloc_with_spares(&d_desc_, size_t(n) * sizeof(MemberDesc)));
+        ENS_TRY(malloc_with_spares(&d_items_, costed.size() * sizeof(int2)));
+        ENS_TRY(malloc_with_spares(&d_stat_, size_t(6) * n * sizeof(double)));
         rec_bytes_ = rec_total * sizeof(double);
         nitems_ = static_cast<int>(costed.size());
         nmembers_ = n;
@@ -1186,7 +1187,7 @@ bool Ensemble::run(hipStream_t stream, int kernel, const std::vector<EnsembleMem
             items.insert(items.end(), lists[b].begin(), lists[b].end());
             first[b + 1] = static_cast<int>(items.size());
         }
-        ENS_TRY(hipMalloc(&d_first_, first.size() * sizeof(int)));
+        ENS_TRY(malloc_with_spares(&d_first_, first.size() * sizeof(int)));
         ENS_TRY(hipMemcpy(d_items_, items.data(), items.size() * sizeof(int2), hipMemcpyHostToDevice));
         ENS_TRY(hipMemcpy(d_first_, first.data(), first.size() * sizeof(int), hipMemcpyHostToDevice));
 
@@ -1196,7 +1197,7 @@ bool Ensemble::run(hipStream_t stream, int kernel, const std::vector<EnsembleMem
         for (int m = 0; m < n; ++m)
             targs[m] = table_args(plans[m], members[m].g, static_cast<const double *>(d_rec_) + rec_off[m],
                                   members[m].np_, static_cast<char *>(d_tab_) + tab_off[m]);
-        ENS_TRY(hipMalloc(&d_targs_, size_t(n) * sizeof(TableArgs)));
+        ENS_TRY(malloc_with_spares(&d_targs_, size_t(n) * sizeof(TableArgs)));
         ENS_TRY(hipMemcpy(d_targs_, targs.data(), size_t(n) * sizeof(TableArgs), hipMemcpyHostToDevice));
 
         ENS_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
@@ -1290,7 +1291,7 @@ bool tune_reserve(void **p, size_t &cap, size_t bytes, std::string &err)
     if (*p) (void)hipFree(*p);
     *p = nullptr;
     cap = 0;
-    const hipError_t e = hipMalloc(p, bytes);
+    const hipError_t e = malloc_with_spares(p, bytes);
     if (e != hipSuccess) {
         err = std::string("tile tuner: hipMalloc: ") + hipGetErrorString(e);
         return false;
@@ -1319,7 +1320,9 @@ bool TileTuner::prepare(double **rec, int np_, hipStream_t stream, std::string &
         ENS_TRY(hipEventCreate(&ev_[1]));
     }
     if (!*rec) {
-        ENS_TRY(hipMalloc(rec, size_t(5) * np_ * sizeof(double)));
+        void *p = nullptr;
+        ENS_TRY(malloc_with_spares(&p, size_t(5) * np_ * sizeof(double)));
+        *rec = static_cast<double *>(p);
         tune_record<<<(np_ + 255) / 256, 256, 0, stream>>>(*rec, np_);
         ENS_TRY(hipGetLastError());
     }
