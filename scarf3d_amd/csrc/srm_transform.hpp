@@ -15,7 +15,8 @@
 // Measured, tables + field + statistics: float 512^3 x 20k 2.0 ms (mfma_bf16x3
 // 47.6, direct_f32 270), 128^3 x 5k 0.13 ms (0.44, 1.7); double 128^3 x 5k
 // 0.20 ms (direct_f64 13.9). 2-norm error against the FP64 sum 1.4e-7 (4e-7,
-// 2.5e-7) in float and 8e-15 in double.
+// 2.5e-7) in float; against extended precision 2.8e-15 (3.8e-15) in double, 128
+// x 100 x 60 x 4000.
 #pragma once
 #include <hip/hip_runtime.h>
 
