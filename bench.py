@@ -221,20 +221,19 @@ FIM_CASE = dict(n=(500, 500, 500), ds=50.0, acf=0, hurst=0.25, cl=(2000.0,) * 3,
 
 def fim_bytes(npts, nout):
     """Least HBM bytes of one FIM realization (float library): the half
-    spectrum written once (8 B per complex value) and read once by the
-    transform, which writes the internal field once (4 B per point); the
-    statistics read it once (4 B); the mapping reads one internal value and
-    writes one output value per output point (8 B). The transform itself
-    takes several passes (a 3D FFT of non-power-of-two lengths), so the
-    fraction of HBM bandwidth this gives is a floor."""
+    spectrum written once and read once (8 B per complex value), the output
+    written once (4 B per point). The transform's passes along y and z move
+    the half spectrum between them, the last one takes the statistics and
+    writes the caller's block, so the fraction of HBM bandwidth this gives is
+    a floor."""
     n1, n2, n3 = npts
     half = (n1 // 2 + 1) * n2 * n3
-    return 8 * half + 8 * half + 4 * n1 * n2 * n3 + 4 * n1 * n2 * n3 + 8 * nout
+    return 8 * half + 8 * half + 4 * nout
 
 
 def measure_fim(steps, warmup, cpu=True):
     """FIM (method 0) at FIM_CASE: the first call of the process (runtime,
-    transform plans, buffers), then warm scarf_execute_device (field in HBM)
+    transform tables, buffers), then warm scarf_execute_device (field in HBM)
     and scarf_execute (field into a host array) calls, wall clock, with the
     device pass times the library reports in stats(5:8)."""
     import scarf3d_amd
@@ -286,9 +285,9 @@ def measure_fim(steps, warmup, cpu=True):
            "internal_mpts_per_s": _sig(nint_ / (dev * 1e-3) / 1e6),
            "hbm": {"algorithmic_bytes": B, "achieved_gbs": _sig(B / (dev * 1e-3) / 1e9), "peak_gbs": PEAK_HBM_GBS,
                    "frac": _sig(B / (dev * 1e-3) / 1e9 / PEAK_HBM_GBS)},
-           "note": "scarf_execute_device wall clock per call (spectrum, symmetry, one hipFFT 3D c2r, statistics, "
-                   "mapping); stage ms from the library's stats(5:8), HIP events; hbm.frac counts the least "
-                   "bytes of each stage (fim_bytes)"}
+           "note": "scarf_execute_device wall clock per call (spectrum, symmetry, dense transform with the "
+                   "statistics and the caller's block); stage ms from the library's stats(5:8), HIP events; "
+                   "hbm.frac counts the spectrum written and read once and the output written once (fim_bytes)"}
     log(f"[bench] FIM {c['n']} (internal {npts}): first call {first_ms:.1f} ms, {dev:.2f} ms per call "
         f"(spectrum {part[0]:.2f}, symmetry {part[1]:.3f}, transforms {part[2]:.2f}, mapping {part[3]:.2f} ms), "
         f"host-array call {float(np.mean(hms)):.1f} ms")
