@@ -95,14 +95,18 @@ struct scarf_member {
 };
 
 /* Runs n realizations in one persistent grouped-GEMM launch (MFMA kernel
- * `kernel`, SCARF_KERNEL_AUTO = mfma_bf16x3) replayed from a hipGraph
- * captured per ensemble shape. d_fields[m]: device output of member m.
- * stats: n x 8 values laid out like scarf_execute's. Harmonics are drawn on
- * the host in parallel, one independent stream per seed. */
+ * `kernel`) replayed from a hipGraph captured per ensemble shape, or, with
+ * SCARF_KERNEL_AUTO, one after the other by the fast transform where that is
+ * faster (else the grouped launch of mfma_bf16x3). d_fields[m]: device output
+ * of member m. stats: n x 8 values laid out like scarf_execute's. Every member
+ * has an independent stream by its seed; short draws run side by side, the
+ * others one after the other with their trials on the GPU. After an error no
+ * work is left in flight on the members' fields. */
 int scarf_ensemble_execute(int n, const struct scarf_member *members, real *const *d_fields, real *stats,
                            int kernel);
 
-/* Device milliseconds of the last ensemble (graph launch to completion). */
+/* Device milliseconds of the last ensemble (graph launch to completion; by the
+ * transform, from the first member to the last, their draws' waits included). */
 double scarf_ensemble_last_ms(void);
 
 /* Block tile of the last MFMA run: out = {x points, j values, k values}

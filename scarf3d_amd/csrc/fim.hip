@@ -63,8 +63,8 @@ struct SpecArgs {
 // its first line's start (companion-matrix powers A^(2^b)), lane l steps to
 // position l and walks the item's lines, one value after the other, for each of
 // its points i = l + 64 t: stores are coalesced. Bound by the integer products
-// of the walk and of the powers: 137 us at 502^3 in float for 0.5 GB written
-// (0.1 ms); 203 us with a step of the state per point, line by line, and a
+// of the walk and of the powers: 137 to 162 us by box at 502^3 in float for 0.5
+// GB written (0.1 ms); 203 us with a step of the state per point, line by line, and a
 // jump every 8 lines.
 template <class Real>
 __global__ __launch_bounds__(256) void fim_spectrum(Cplx<Real> *__restrict__ S, SpecArgs<Real> a,

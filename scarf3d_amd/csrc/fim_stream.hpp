@@ -96,7 +96,7 @@ __host__ __device__ inline void walk_item(const uint32_t *pw, const Tables *t, c
         uint32_t x, next;
     };
     // four points of a line at a time: what they write is near in time too
-    // (spectrum of 502^3 in float: one at a time 177 us, two 146, four 137;
+    // (spectrum of 502^3 in float, one box: one at a time 177 us, two 146, four 137;
     // 256 x 256 x 102 in double: two 105 us, four 92)
     constexpr int C = 4;
     for (int i = lane; i < h; i += 64 * C) {
