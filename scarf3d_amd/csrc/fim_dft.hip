@@ -23,6 +23,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 #include "srm_stats.hpp"
 
@@ -84,12 +85,24 @@ __device__ __forceinline__ void together(T &...v)
 }
 
 // step(s, table value) for s = 0 .. steps - 1, with the table values of the
-// next group of steps in flight from L2 while one is multiplied. The sums of
-// a group start from zero and are added to the totals by flush(): a chain of
-// 16 terms and one of steps / 4 sums round less than one over all terms (502^3
-// in float 3.0e-7 off FP64, with one chain 5.3e-7, the FFT library 4.1e-7;
-// 214 x 186 x 138 in double 5.4e-16, the library 1.05e-15).
-template <class V, class Step, class Flush>
+// next group of steps in flight from L2 while one is multiplied. The sums of F
+// steps, of a group at most, start from zero and are added to the totals by
+// flush(): a chain of 16 terms and one of steps / 4 sums round less than one
+// over all terms (502^3 in float 3.0e-7 off FP64, with one chain 5.3e-7, the FFT
+// library 4.1e-7; 214 x 186 x 138 in double 4.7e-16 off extended precision, the
+// library 9.9e-16).
+//
+// The library's FP32 transform rounds less where its lengths are short (2.3e-7 of
+// a field's 3.1e-7 are the spectrum's), so float lines up to 128 take chains of 8
+// terms, up to 64 of 4, with totals and last combinations in FP64. Against
+// extended precision, float fields, so / with chains of 16 / the library: 62 x
+// 58 x 46 3.11e-7 / 3.45e-7 / 3.23e-7, 96 x 120 x 64 2.73e-7 / 3.07e-7 / 2.87e-7,
+// 128^3 3.10e-7 / 3.39e-7 / 3.06e-7 (calls 115, 111 and 112 us). Longer lines
+// would pay 11 to 30% of a call for 2 to 9% (258^3 338 -> 438 us) and stay as
+// they are: up to 9% above the library where only one of the axes has a large
+// prime factor (142 x 162 x 182 3.16e-7 / 2.90e-7), below it where two have
+// (214 x 186 x 138 3.20e-7 / 3.38e-7).
+template <int F, class V, class Step, class Flush>
 __device__ __forceinline__ void for_steps(const V *__restrict__ t, int steps, const Step &step, const Flush &flush)
 {
     constexpr int U = sizeof(V) > 16 ? 2 : 4;
@@ -103,17 +116,22 @@ __device__ __forceinline__ void for_steps(const V *__restrict__ t, int steps, co
         for (int u = 0; u < U; ++u) next[u] = t[min(s + U + u, steps - 1) * 64];
         __builtin_amdgcn_sched_barrier(0);  // not moved down to their use
 #pragma unroll
-        for (int u = 0; u < U; ++u) step(s + u, w[u], u == 0);
-        flush();
+        for (int u = 0; u < U; ++u) {
+            step(s + u, w[u], u % F == 0);
+            if (u % F == F - 1 || u == U - 1) flush();
+        }
 #pragma unroll
         for (int u = 0; u < U; ++u) w[u] = next[u];
     }
     if (s == steps) return;
 #pragma unroll
     for (int u = 0; u < U - 1; ++u)
-        if (s + u < steps) step(s + u, w[u], u == 0);
-    flush();
+        if (s + u < steps) {
+            step(s + u, w[u], u % F == 0);
+            if (u % F == F - 1 || s + u == steps - 1) flush();
+        }
 }
+
 
 // sine and cosine of r/n turns, 0 <= r < n, from the distance to the nearest
 // quarter: a quotient near 1 would lose up to 7e-16 to its own rounding
@@ -181,14 +199,17 @@ __device__ inline long place_of(long block, long total)
 }
 
 // Lines of n elements `stride` apart, 16 neighbouring ones per block, in place:
-// a block reads its lines before it writes any.
-template <class Real>
-__global__ __launch_bounds__(64 * kColumnWaves<Real>) void dft_columns(Vec<Real, 2> *__restrict__ S, const Vec<Real, 2> *__restrict__ table,
+// a block reads its lines before it writes any. Sum: the type of the totals; FP64
+// ones of FP32 fields take more registers, and their blocks have 8 waves at most.
+template <class Real, class Sum, int Chain>
+__global__ __launch_bounds__(sizeof(Sum) > sizeof(Real) ? 512 : 64 * kColumnWaves<Real>) void dft_columns(Vec<Real, 2> *__restrict__ S, const Vec<Real, 2> *__restrict__ table,
                                                     int n, long stride, int columns, long plane, int per_plane,
                                                     long blocks)
 {
     using V2 = Vec<Real, 2>;
     using V4 = Vec<Real, 4>;
+    using S2 = Vec<Sum, 2>;
+    using S4 = Vec<Sum, 4>;
     extern __shared__ __align__(16) char shared[];
     const long place = place_of(blockIdx.x, blocks);
     if (place >= blocks) return;
@@ -232,13 +253,14 @@ __global__ __launch_bounds__(64 * kColumnWaves<Real>) void dft_columns(Vec<Real,
     __syncthreads();
     const V2 *turn = table + tiles(n) * steps * 64;
     for (int tile = wave; tile < tiles(n); tile += waves) {
-        V4 ca[4], sd[4], part[8];
+        V4 part[8];
+        S4 ca[4], sd[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) ca[r] = sd[r] = V4{Real(0), Real(0), Real(0), Real(0)};
+        for (int r = 0; r < 4; ++r) ca[r] = sd[r] = S4{Sum(0), Sum(0), Sum(0), Sum(0)};
         V2 wk[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) wk[r] = turn[min(tile * 16 + row_of<Real>(lane, r), half)];
-        for_steps(table + tile * steps * 64 + lane, steps, [&](int s, V2 w, bool fresh) __attribute__((always_inline)) {
+        for_steps<Chain>(table + tile * steps * 64 + lane, steps, [&](int s, V2 w, bool fresh) __attribute__((always_inline)) {
             const V4 a = sum[s * 64 + lane], d = diff[s * 64 + lane], zero{Real(0), Real(0), Real(0), Real(0)};
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -248,8 +270,8 @@ __global__ __launch_bounds__(64 * kColumnWaves<Real>) void dft_columns(Vec<Real,
         }, [&]() __attribute__((always_inline)) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                ca[r] += part[r];
-                sd[r] += part[4 + r];
+                ca[r] += __builtin_convertvector(part[r], S4);
+                sd[r] += __builtin_convertvector(part[4 + r], S4);
             }
         });
         if (first + (lane & 15) >= columns) continue;
@@ -258,17 +280,18 @@ __global__ __launch_bounds__(64 * kColumnWaves<Real>) void dft_columns(Vec<Real,
         for (int r = 0; r < 4; ++r) {
             const int k = tile * 16 + row_of<Real>(lane, r);
             if (k > half) continue;
-            const V2 w = wk[r];
-            const V2 y0{ca[0][r] - sd[1][r], ca[1][r] + sd[0][r]}, y1{ca[2][r] - sd[3][r], ca[3][r] + sd[2][r]};
-            const V2 wy{w.x * y1.x - w.y * y1.y, w.x * y1.y + w.y * y1.x};
-            out[k * stride] = y0 + wy;
-            out[(k + m) * stride] = y0 - wy;
+            const S2 w = __builtin_convertvector(wk[r], S2);
+            auto put = [&](int at, S2 v) __attribute__((always_inline)) { out[at * stride] = __builtin_convertvector(v, V2); };
+            const S2 y0{ca[0][r] - sd[1][r], ca[1][r] + sd[0][r]}, y1{ca[2][r] - sd[3][r], ca[3][r] + sd[2][r]};
+            const S2 wy{w.x * y1.x - w.y * y1.y, w.x * y1.y + w.y * y1.x};
+            put(k, y0 + wy);
+            put(k + m, y0 - wy);
             if (k == 0 || 2 * k == m) continue;
             // Y[M - k] and w^(M - k) = -conj(w^k)
-            const V2 z0{ca[0][r] + sd[1][r], ca[1][r] - sd[0][r]}, z1{ca[2][r] + sd[3][r], ca[3][r] - sd[2][r]};
-            const V2 wz{w.x * z1.x + w.y * z1.y, w.x * z1.y - w.y * z1.x};
-            out[(m - k) * stride] = z0 - wz;
-            out[(n - k) * stride] = z0 + wz;
+            const S2 z0{ca[0][r] + sd[1][r], ca[1][r] - sd[0][r]}, z1{ca[2][r] + sd[3][r], ca[3][r] - sd[2][r]};
+            const S2 wz{w.x * z1.x + w.y * z1.y, w.x * z1.y - w.y * z1.x};
+            put(m - k, z0 - wz);
+            put(n - k, z0 + wz);
         }
     }
 }
@@ -280,8 +303,8 @@ __global__ __launch_bounds__(64 * kColumnWaves<Real>) void dft_columns(Vec<Real,
 // of LDS, since a wave's product holds 16 positions of 16 lines; from there
 // they go to the caller's grid where nothing else follows (500^3: 1 GB and
 // 0.27 ms less than by way of R and a pass that gathers).
-template <class Real>
-__global__ __launch_bounds__(1024) void dft_rows(const Vec<Real, 2> *__restrict__ S, Real *__restrict__ R,
+template <class Real, class Sum, int Chain>
+__global__ __launch_bounds__(sizeof(Sum) > sizeof(Real) ? 512 : 1024) void dft_rows(const Vec<Real, 2> *__restrict__ S, Real *__restrict__ R,
                                                  Nearest<Real> to, const Vec<Real, 4> *__restrict__ table, int n,
                                                  int n2, int lines, Real scaling, double *__restrict__ part)
 {
@@ -325,13 +348,15 @@ __global__ __launch_bounds__(1024) void dft_rows(const Vec<Real, 2> *__restrict_
         }
     }
     __syncthreads();
-    V4 ce[T], se[T], co[T], so[T], sums[T][4];
+    using S4 = Vec<Sum, 4>;
+    V4 sums[T][4];
+    S4 ce[T], se[T], co[T], so[T];
 #pragma unroll
-    for (int t = 0; t < T; ++t) ce[t] = se[t] = co[t] = so[t] = V4{Real(0), Real(0), Real(0), Real(0)};
+    for (int t = 0; t < T; ++t) ce[t] = se[t] = co[t] = so[t] = S4{Sum(0), Sum(0), Sum(0), Sum(0)};
     const bool busy = wave < tiles(n);
     if (busy) {
         const V4 *b = x + (lane >> 4) * (L + 1) + (lane & 15);
-        for_steps(table + wave * steps * 64 + lane, steps, [&](int s, V4 c, bool fresh) __attribute__((always_inline)) {
+        for_steps<Chain>(table + wave * steps * 64 + lane, steps, [&](int s, V4 c, bool fresh) __attribute__((always_inline)) {
             const V4 zero{Real(0), Real(0), Real(0), Real(0)};
 #pragma unroll
             for (int t = 0; t < T; ++t) {
@@ -342,10 +367,10 @@ __global__ __launch_bounds__(1024) void dft_rows(const Vec<Real, 2> *__restrict_
         }, [&]() __attribute__((always_inline)) {
 #pragma unroll
             for (int t = 0; t < T; ++t) {
-                ce[t] += sums[t][0];
-                se[t] += sums[t][1];
-                co[t] += sums[t][2];
-                so[t] += sums[t][3];
+                ce[t] += __builtin_convertvector(sums[t][0], S4);
+                se[t] += __builtin_convertvector(sums[t][1], S4);
+                co[t] += __builtin_convertvector(sums[t][2], S4);
+                so[t] += __builtin_convertvector(sums[t][3], S4);
             }
         });
     }
@@ -359,13 +384,13 @@ __global__ __launch_bounds__(1024) void dft_rows(const Vec<Real, 2> *__restrict_
             for (int r = 0; r < 4; ++r) {
                 const int i = wave * 16 + row_of<Real>(lane, r);
                 if (i > half) continue;
-                const Real c = ce[t][r] + co[t][r], d = ce[t][r] - co[t][r];
-                const Real s = se[t][r] + so[t][r], u = se[t][r] - so[t][r];
-                line[i] = c - s;
-                line[m + i] = d - u;
+                const Sum c = ce[t][r] + co[t][r], d = ce[t][r] - co[t][r];
+                const Sum s = se[t][r] + so[t][r], u = se[t][r] - so[t][r];
+                line[i] = Real(c - s);
+                line[m + i] = Real(d - u);
                 if (i == 0) continue;
-                line[n - i] = c + s;
-                if (2 * i < m) line[m - i] = d + u;
+                line[n - i] = Real(c + s);
+                if (2 * i < m) line[m - i] = Real(d + u);
             }
         }
     }
@@ -462,10 +487,15 @@ hipError_t columns_pass(Vec<Real, 2> *S, const Vec<Real, 2> *table, int n, long 
     const size_t lds = columns_lds<Real>(n);
     const int per_plane = (columns + 15) / 16;
     const long blocks = long(per_plane) * planes;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&dft_columns<Real>),
+    auto kernel = &dft_columns<Real, Real, 4>;
+    if constexpr (sizeof(Real) == 4) {
+        if (n <= 128) kernel = &dft_columns<Real, double, 2>;
+        if (n <= 64) kernel = &dft_columns<Real, double, 1>;
+    }
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (e != hipSuccess) return e;
-    dft_columns<Real><<<unsigned((blocks + kXcds - 1) / kXcds * kXcds), column_threads<Real>(n, lds), lds, stream>>>(
+    kernel<<<unsigned((blocks + kXcds - 1) / kXcds * kXcds), column_threads<Real>(n, lds), lds, stream>>>(
         S, table, n, stride, columns, plane, per_plane, blocks);
     return hipGetLastError();
 }
@@ -479,7 +509,8 @@ hipError_t columns_pass(Vec<Real, 2> *S, const Vec<Real, 2> *table, int n, long 
 //   a large prime factor   502^3 1.90 : 3.41, 258^3 0.35 : 0.75, 802 x 802 x 257 3.41 : 5.61,
 //                          double 214 x 186 x 138 0.23 : 0.42, 2D 302 x 258 0.090 : 0.101,
 //                          502 x 502 0.102 : 0.107, 614 x 402 0.113 : 0.113, 802 x 802 0.149 : 0.135
-//   none                   32^3 0.075 : 0.073, 64^3 0.078 : 0.082, 128^3 0.111 : 0.123, 256^3 0.33 : 0.31,
+//   none                   32 x 48 x 40 0.078 : 0.093, 64^3 0.081 : 0.079, 96 x 120 x 64 0.089 : 0.106,
+//                          128^3 0.115 : 0.112, 256^3 0.33 : 0.31,
 //                          800 x 800 x 256 3.13 : 2.74, 2D 64 x 64 0.080 : 0.071, double 64^3 0.085 : 0.091,
 //                          128^3 0.158 : 0.152, 256^3 0.65 : 0.52
 // So: with a large prime factor every 3D grid whose lines fit the LDS, and 2D
@@ -537,10 +568,15 @@ hipError_t run(void *S, Real *R, const Nearest<Real> &to, const void *tables, in
     if (e == hipSuccess) e = columns_pass<Real>(s, y, n2, h, h, long(h) * n2, n3, stream);
     if (e != hipSuccess) return e;
     const size_t lds = rows_lds<Real>(n1);
-    e = hipFuncSetAttribute(reinterpret_cast<const void *>(&dft_rows<Real>),
+    auto kernel = &dft_rows<Real, Real, 4>;
+    if constexpr (sizeof(Real) == 4) {
+        if (n1 <= 128) kernel = &dft_rows<Real, double, 2>;
+        if (n1 <= 64) kernel = &dft_rows<Real, double, 1>;
+    }
+    e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
                             hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (e != hipSuccess) return e;
-    dft_rows<Real><<<unsigned(parts<Real>(n1, n2, n3)), 64 * std::max(4, tiles(n1)), lds, stream>>>(
+    kernel<<<unsigned(parts<Real>(n1, n2, n3)), 64 * std::max(4, tiles(n1)), lds, stream>>>(
         s, R, to, x, n1, n2, n2 * n3, scaling, part);
     return hipGetLastError();
 }
