@@ -92,8 +92,8 @@ __device__ __forceinline__ void together(T &...v)
 // library 4.1e-7; 214 x 186 x 138 in double 4.7e-16 off extended precision, the
 // library 9.9e-16).
 //
-// The library's FP32 transform rounds less where its lengths are short (2.3e-7 of
-// a field's 3.1e-7 are the spectrum's), so float lines up to 128 take chains of 8
+// The library's FP32 transform rounds less where its lengths are short (of a
+// field's 3.1e-7 some 2.9e-7 are the spectrum's), so float lines up to 128 take chains of 8
 // terms, up to 64 of 4, with totals and last combinations in FP64. Against
 // extended precision, float fields, so / with chains of 16 / the library: 62 x
 // 58 x 46 3.11e-7 / 3.45e-7 / 3.23e-7, 96 x 120 x 64 2.73e-7 / 3.07e-7 / 2.87e-7,
