@@ -93,15 +93,17 @@ __device__ __forceinline__ void together(T &...v)
 // library 9.9e-16).
 //
 // The library's FP32 transform rounds less where its lengths are short (of a
-// field's 3.1e-7 some 2.9e-7 are the spectrum's), so float lines up to 128 take chains of 8
-// terms, up to 64 of 4, with totals and last combinations in FP64. Against
-// extended precision, float fields, so / with chains of 16 / the library: 62 x
-// 58 x 46 3.11e-7 / 3.45e-7 / 3.23e-7, 96 x 120 x 64 2.73e-7 / 3.07e-7 / 2.87e-7,
-// 128^3 3.10e-7 / 3.39e-7 / 3.06e-7 (calls 115, 111 and 112 us). Longer lines
-// would pay 11 to 30% of a call for 2 to 9% (258^3 338 -> 438 us) and stay as
-// they are: up to 9% above the library where only one of the axes has a large
-// prime factor (142 x 162 x 182 3.16e-7 / 2.90e-7), below it where two have
-// (214 x 186 x 138 3.20e-7 / 3.38e-7).
+// field's 3.1e-7 some 2.9e-7 are the spectrum's) or few have a large prime factor.
+// So float lines up to 64 take chains of 4 terms, and lines up to 128, or 288
+// where at most one axis has a large prime factor, of 8 terms, with totals and
+// last combinations in FP64. Float fields against extended precision, so / with
+// chains of 16 / the library, and their calls: 62 x 58 x 46 3.11e-7 / 3.45e-7 /
+// 3.23e-7; 96 x 120 x 64 2.73e-7 / 3.07e-7 / 2.87e-7, 89 / 87 / 106 us; 128^3
+// 3.10e-7 / 3.39e-7 / 3.06e-7, 115 / 111 / 112 us; 256 x 252 x 62 3.31e-7 / 3.64e-7
+// / 3.29e-7, 150 / 135 / 172 us; 256 x 256 x 102 3.17e-7 / 3.50e-7 / 3.13e-7, 214 /
+// 183 / 187 us. Other lines stay as they are: with two large prime factors the
+// library is further off (214 x 186 x 138 3.20e-7 / 3.38e-7), and 258^3 would pay
+// 338 -> 438 us.
 template <int F, class V, class Step, class Flush>
 __device__ __forceinline__ void for_steps(const V *__restrict__ t, int steps, const Step &step, const Flush &flush)
 {
@@ -482,14 +484,14 @@ bool large_prime(int n)
 
 template <class Real>
 hipError_t columns_pass(Vec<Real, 2> *S, const Vec<Real, 2> *table, int n, long stride, int columns, long plane,
-                        int planes, hipStream_t stream)
+                        int planes, int careful, hipStream_t stream)
 {
     const size_t lds = columns_lds<Real>(n);
     const int per_plane = (columns + 15) / 16;
     const long blocks = long(per_plane) * planes;
     auto kernel = &dft_columns<Real, Real, 4>;
     if constexpr (sizeof(Real) == 4) {
-        if (n <= 128) kernel = &dft_columns<Real, double, 2>;
+        if (n <= careful) kernel = &dft_columns<Real, double, 2>;
         if (n <= 64) kernel = &dft_columns<Real, double, 1>;
     }
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
@@ -562,15 +564,17 @@ hipError_t run(void *S, Real *R, const Nearest<Real> &to, const void *tables, in
     const auto *x = static_cast<const Vec<Real, 4> *>(tables);
     const auto *y = reinterpret_cast<const Vec<Real, 2> *>(x + rows_table<Real>(n1));
     const int h = n1 / 2 + 1;
+    // float lines up to this length have FP64 totals (for_steps)
+    const int careful = int(large_prime(n1)) + int(large_prime(n2)) + int(large_prime(n3)) <= 1 ? 288 : 128;
     hipError_t e = hipSuccess;
     if (n3 > 1)
-        e = columns_pass<Real>(s, y + columns_table<Real>(n2), n3, long(h) * n2, h * n2, 0, 1, stream);
-    if (e == hipSuccess) e = columns_pass<Real>(s, y, n2, h, h, long(h) * n2, n3, stream);
+        e = columns_pass<Real>(s, y + columns_table<Real>(n2), n3, long(h) * n2, h * n2, 0, 1, careful, stream);
+    if (e == hipSuccess) e = columns_pass<Real>(s, y, n2, h, h, long(h) * n2, n3, careful, stream);
     if (e != hipSuccess) return e;
     const size_t lds = rows_lds<Real>(n1);
     auto kernel = &dft_rows<Real, Real, 4>;
     if constexpr (sizeof(Real) == 4) {
-        if (n1 <= 128) kernel = &dft_rows<Real, double, 2>;
+        if (n1 <= careful) kernel = &dft_rows<Real, double, 2>;
         if (n1 <= 64) kernel = &dft_rows<Real, double, 1>;
     }
     e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),

@@ -2,7 +2,7 @@
 // host: 2-norm error over 2-norm of the result.
 //
 // Bounds, before any run. A rounding to FP32 is 2.4e-8 rms. A line's products sum
-// in chains of 4 terms (up to 64) or 8 (up to 128): 2.4e-8 sqrt(c / 2), 3.4e-8 or
+// in chains of 4 terms (up to 64) or 8 (up to 128 or 288): 2.4e-8 sqrt(c / 2), 3.4e-8 or
 // 4.8e-8; the folded inputs, the matrices, the twiddles and the result round once
 // each, 4.8e-8. Over three axes 1.02e-7 and 1.18e-7; a sixth more allowed. (With
 // chains of 16, totals and combinations in FP32: 1.6e-7.)
@@ -112,6 +112,9 @@ int main()
     check(66, 70, 122, eight);
     check(128, 126, 94, eight);
     check(128, 62, 40, eight);
+    check(256, 40, 38, eight);  // one axis with a large prime factor: up to 288
+    check(38, 288, 130, eight);
+    check(258, 128, 1, eight);
     std::printf("%d bad\n", bad);
     return bad != 0;
 }
